@@ -18,9 +18,10 @@
 //   k_setup_clip  triangles crossing the near/far plane or the guard band:
 //                 Sutherland-Hodgman fan, each fan triangle binned on its own
 //   k_raster_lane per (scene, bin): one binned triangle per lane, large
-//                 rectangles from an LDS queue by the whole workgroup; depth
-//                 test as a 64-bit LDS atomicMin of (window depth bits,
-//                 primitive order); visibility keys to HBM, or, in the
+//                 rectangles from an LDS queue by a wave each, in 8x8
+//                 pixel blocks; depth test as a 64-bit LDS atomicMin of
+//                 (window depth bits, primitive order); visibility keys to
+//                 HBM, or, in the
 //                 frame's last raster phase of an unlit renderer, the bin
 //                 resolved in place from its LDS keys (k_raster_pairs:
 //                 selectable pair-parallel form; k_raster_full: exact rescan
@@ -105,6 +106,16 @@ __device__ __forceinline__ int32_t imul24(int32_t a, int32_t b) {
 // truncation is exact (an integer division costs ~25 VALU operations).
 __device__ __forceinline__ int div_small(int l, float inv) {
   return (int)(((float)l + 0.5f) * inv);
+}
+
+// The thread index through an opaque move, for the helpers of the persistent
+// rasteriser: what they derive from it (pixel offsets and the like) would
+// otherwise be hoisted out of its loop over the bins, where it costs more
+// registers than the loop has and is spilled to scratch memory.
+__device__ __forceinline__ int local_tid() {
+  int t = (int)threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
 }
 
 struct Snap {
@@ -908,19 +919,34 @@ __global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams p,
 // Rasterisation helpers: LDS visibility tile with 64-bit atomicMin keys
 // --------------------------------------------------------------------------
 
-// A triangle the whole workgroup rasterises, set up once by the lane that
-// queued it: its three edge functions (fill-rule bias included) at the bin's
-// first pixel centre, exact in 64 bits, and their steps per pixel right and
-// down; narrow = every value over the bin (and a bin past it) fits in 32 bits.
-struct BigTri {
-  long long e[3];
-  int32_t dx[3], dy[3];  // edge vectors (|d| < 2^23); per pixel right -dy * 256, down dx * 256
-  float z0, dzdx, dzdy, zlo;
+// Edge functions in pixel steps.  With E0 the 64-bit edge value (fill-rule
+// bias included) at one pixel centre, the value k = dx * ny - dy * nx pixels
+// away is E0 + 256 k, and E0 + 256 k >= 0 exactly when (E0 >> 8) + k >= 0
+// (arithmetic shift).  |d| < 2^23 and a bin has at most 32 pixels a side, so
+// |k| < 2^29 inside a bin, and E0 >> 8 clamped to +-2^30 keeps the sign of
+// every sum: all triangles, also those reaching out to the guard band, step
+// in 32 bits, by the plain edge vector.
+__device__ __forceinline__ int32_t edge_steps(long long e) {
+  e >>= 8;
+  constexpr long long kLim = 1ll << 30;
+  return (int32_t)(e < -kLim ? -kLim : (e > kLim ? kLim : e));
+}
+
+// A triangle a whole wave rasterises, set up once by the lane that queued
+// it: its three edge functions at the bin's first pixel centre (edge_steps)
+// and the edge vectors, the depth plane and the covered pixel rectangle.
+struct alignas(16) BigTri {
+  int32_t e[3];
+  float z0;
+  int32_t dx[3];         // |d| < 2^23; per pixel right -dy, down dx
+  float dzdx;
+  int32_t dy[3];
+  float dzdy;
+  float zlo;             // depth_floor()
   int32_t X0, Y0;        // vertex 0, the depth plane's origin
   uint32_t prim;
   uint8_t x0, y0, x1, y1;  // covered pixel rectangle, relative to the bin
-  uint16_t npx;            // its pixel count
-  uint16_t narrow;
+  uint32_t pad[3];
 };
 
 struct RasterCtx {
@@ -941,39 +967,41 @@ __device__ __forceinline__ bool small_box(const int32_t* X, const int32_t* Y) {
   return ex < 16384 && ey < 16384;
 }
 
-__device__ __forceinline__ void depth_key_min(const RasterCtx& rc, float z0, float dzdx, float dzdy,
-                                              float zlo, const int32_t* X, const int32_t* Y,
-                                              uint32_t prim, int px, int py) {
-  const float z = depth_at(z0, dzdx, dzdy, zlo, X[0], Y[0], px * 256 + 128,
-                           py * 256 + 128);
-  if (z < 1.0f) {
-    const unsigned long long key = ((unsigned long long)__float_as_uint(z) << 32) | prim;
-    atomicMin(&rc.vis[__mul24(py - rc.bin.y0, rc.B) + (px - rc.bin.x0)], key);
-  }
+// The depth of a fragment is the plane's value raised to the nearest vertex
+// depth and to 0 (depth_at()): with a floor of the larger of the two, both
+// comparisons become one, z > floor ? z : floor, which also takes -0 to the
+// floor.  A NaN nearest depth makes every fragment's depth 0.
+__device__ __forceinline__ float depth_floor(float zlo, float& z0, float& dzdx, float& dzdy) {
+  if (zlo != zlo) z0 = dzdx = dzdy = 0.0f;
+  return zlo > 0.0f ? zlo : 0.0f;
+}
+
+// merges one covered pixel: zx = z0 + dzdx * ox, zy = dzdy * oy (the op
+// order of depth_at); a depth of 1 or more is never stored
+__device__ __forceinline__ void merge_key(unsigned long long* vis, int at, float zx, float zy,
+                                          float floor_z, uint32_t prim) {
+  const float s = zx + zy;
+  const float z = s > floor_z ? s : floor_z;
+  if (z < 1.0f) atomicMin(&vis[at], ((unsigned long long)__float_as_uint(z) << 32) | prim);
 }
 
 // queue entry of a triangle with a known depth plane and pixel rectangle r
 // (inside the bin)
 __device__ __forceinline__ void make_big(const RasterCtx& rc, const int32_t* X, const int32_t* Y,
                                          float z0, float dzdx, float dzdy, float zlo,
-                                         uint32_t prim, const PixRect& r, int npx, BigTri& b) {
+                                         uint32_t prim, const PixRect& r, BigTri& b) {
   const long long Px0 = (long long)rc.bin.x0 * 256 + 128, Py0 = (long long)rc.bin.y0 * 256 + 128;
-  bool narrow = true;
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     const int j = (i + 1) % 3;
     const int32_t dx = X[j] - X[i], dy = Y[j] - Y[i];
     const long long bias = (dy < 0 || (dy == 0 && dx > 0)) ? 0 : -1;
-    const long long e = (long long)dx * (Py0 - Y[i]) - (long long)dy * (Px0 - X[i]) + bias;
-    // window coordinates stay within the guard band (|X|, |Y| < 2^22), so
-    // |d| * 256 < 2^31
-    b.e[i] = e;
+    b.e[i] = edge_steps((long long)dx * (Py0 - Y[i]) - (long long)dy * (Px0 - X[i]) + bias);
     b.dx[i] = dx;
     b.dy[i] = dy;
-    const long long reach = (llabs((long long)dx) + llabs((long long)dy)) * 256 * 64;
-    narrow = narrow && llabs(e) + reach < (1ll << 31);
   }
-  b.z0 = z0; b.dzdx = dzdx; b.dzdy = dzdy; b.zlo = zlo;
+  b.zlo = depth_floor(zlo, z0, dzdx, dzdy);
+  b.z0 = z0; b.dzdx = dzdx; b.dzdy = dzdy;
   b.X0 = X[0];
   b.Y0 = Y[0];
   b.prim = prim;
@@ -981,127 +1009,106 @@ __device__ __forceinline__ void make_big(const RasterCtx& rc, const int32_t* X, 
   b.y0 = (uint8_t)(r.y0 - rc.bin.y0);
   b.x1 = (uint8_t)(r.x1 - rc.bin.x0);
   b.y1 = (uint8_t)(r.y1 - rc.bin.y0);
-  b.npx = (uint16_t)npx;
-  b.narrow = narrow ? 1 : 0;
 }
 
-// The queued triangles, a wave at a time each: a wave claims the next
-// triangle (LDS counter `next`) and spreads its pixel rectangle over its
-// lanes, pixel p = lane + 64 i of the rectangle in row-major order; each
-// lane evaluates the edge functions at its pixel directly (exact: 32-bit
-// when narrow) and merges a covered pixel with an LDS atomicMin, so the
-// waves need no ownership of pixels and a triangle costs
-// ceil(pixels / 64) wave steps.
-__device__ void raster_big_waves(const RasterCtx& rc, const BigTri* big, int nb, int* next) {
-  const int lane = (int)threadIdx.x & 63;
-  if (threadIdx.x == 0)
-    for (int q = 0; q < nb; ++q) *rc.pairs += big[q].npx;
-  for (;;) {
-    int q = 0;
-    if (lane == 0) q = atomicAdd(next, 1);
-    q = __builtin_amdgcn_readfirstlane(q);
-    if (q >= nb) break;
+// a value the whole wave shares, in a scalar register
+__device__ __forceinline__ int32_t uniform(int32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ float uniform(float v) {
+  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+
+// The queued triangles, a wave at a time each (every fourth one: the queue's
+// order is random, so the waves share it evenly): a wave walks the bin's 8x8
+// pixel blocks that the triangle reaches, one pixel per lane.  A block is left out when one
+// edge function is negative at the block's corner that maximises it (exact:
+// the functions are linear); lanes 0-15 test the bin's at most 16 blocks at
+// once.  A block step is then three additions (block offset, a scalar, plus
+// the lane's own offset), the depth and the LDS atomicMin.
+__device__ void raster_big_waves(const RasterCtx& rc, const BigTri* big, int nb) {
+  const int tid = local_tid();
+  const int lane = tid & 63;
+  const int lx = lane & 7, ly = lane >> 3;          // pixel in a block
+  const int cx = 8 * (lane & 3), cy = 8 * ((lane >> 2) & 3);  // lanes 0-15: a block's origin
+  const int bw = rc.bin.x1 - rc.bin.x0 + 1, bh = rc.bin.y1 - rc.bin.y0 + 1;
+  const int at0 = __mul24(ly, rc.B) + lx;
+  for (int q = uniform(tid >> 6); q < nb; q += kBlock / 64) {
     const BigTri& t = big[q];
-    const int x0 = t.x0, y0 = t.y0, w = t.x1 - t.x0 + 1, npx = t.npx;
-    const float inv_w = 1.0f / (float)w;
-    const int32_t X0 = t.X0, Y0 = t.Y0;
-    const float z0 = t.z0, dzdx = t.dzdx, dzdy = t.dzdy, zlo = t.zlo;
-    const uint32_t prim = t.prim;
-    int32_t dx[3], dy[3];
-    long long e[3];
+    int32_t dx[3], dy[3], el[3];
+    bool reach = lane < 16 && cx <= t.x1 && cx + 7 >= t.x0 && cy <= t.y1 && cy + 7 >= t.y0;
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-      dx[i] = t.dx[i];
-      dy[i] = t.dy[i];
-      e[i] = t.e[i];
+      dx[i] = uniform(t.dx[i]);
+      dy[i] = uniform(t.dy[i]);
+      const int32_t e = uniform(t.e[i]);
+      el[i] = e + imul24(dx[i], ly) - imul24(dy[i], lx);
+      reach = reach && e + imul24(dx[i], dx[i] > 0 ? cy + 7 : cy) -
+                              imul24(dy[i], dy[i] < 0 ? cx + 7 : cx) >= 0;
     }
-    // integer products below are of a pixel offset (< 64) and an edge
-    // vector component (|d| < 2^23) or a bin dimension: 24-bit multiplies
-    const bool narrow = t.narrow;
-    for (int pi = lane; pi < npx; pi += 64) {
-      const int ry = div_small(pi, inv_w);
-      const int lx = x0 + (pi - __mul24(ry, w)), ly = y0 + ry;
-      bool in;
-      if (narrow) {
-        uint32_t v[3];
+    const float z0 = uniform(t.z0), dzdx = uniform(t.dzdx), dzdy = uniform(t.dzdy),
+                floor_z = uniform(t.zlo);
+    const uint32_t prim = (uint32_t)uniform((int32_t)t.prim);
+    const int32_t ox0 = (((rc.bin.x0 + lx) << 8) | 128) - uniform(t.X0);
+    const int32_t oy0 = (((rc.bin.y0 + ly) << 8) | 128) - uniform(t.Y0);
+    for (uint32_t m = (uint32_t)__ballot(reach); m != 0u; m &= m - 1u) {
+      const int k = __ffs(m) - 1;
+      const int bx = 8 * (k & 3), by = 8 * (k >> 2);
+      int32_t v = 0;
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
-          v[i] = (uint32_t)e[i] + (uint32_t)(imul24(dx[i], ly) - imul24(dy[i], lx)) * 256u;
-        in = (int32_t)(v[0] | v[1] | v[2]) >= 0;
-      } else {
-        long long v[3];
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-          v[i] = e[i] + (long long)(imul24(dx[i], ly) - imul24(dy[i], lx)) * 256;
-        in = (v[0] | v[1] | v[2]) >= 0;
-      }
-      if (in) {
+      for (int i = 0; i < 3; ++i) v |= el[i] + (dx[i] * by - dy[i] * bx);
+      // (a bin at the viewport's edge has fewer pixels than the tile)
+      if (v >= 0 && lx < bw - bx && ly < bh - by) {
         ++*rc.frags;
-        const float z = depth_at(z0, dzdx, dzdy, zlo, X0, Y0, ((rc.bin.x0 + lx) << 8) | 128,
-                                 ((rc.bin.y0 + ly) << 8) | 128);
-        if (z < 1.0f)
-          atomicMin(&rc.vis[__mul24(ly, rc.B) + lx],
-                    ((unsigned long long)__float_as_uint(z) << 32) | prim);
+        const float zx = z0 + dzdx * (float)(ox0 + (bx << 8));
+        const float zy = dzdy * (float)(oy0 + (by << 8));
+        merge_key(rc.vis, at0 + by * rc.B + bx, zx, zy, floor_z, prim);
       }
     }
   }
 }
 
 // this lane walks the clipped rectangle r of one front-facing triangle with
-// a known depth plane row by row, edge functions stepped by additions
+// a known depth plane row by row, edge functions stepped by additions.  The
+// depth plane's pixel offsets are integers below 2^24, so stepping them by
+// 256 as floats is exact.
 __device__ void raster_walk(const RasterCtx& rc, const int32_t* X, const int32_t* Y, float z0,
                             float dzdx, float dzdy, float zlo, uint32_t prim, const PixRect& r) {
-  if (small_box(X, Y)) {
-    int32_t dx[3], dy[3], bias[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const int j = (i + 1) % 3;
-      dx[i] = X[j] - X[i];
-      dy[i] = Y[j] - Y[i];
-      bias[i] = (dy[i] < 0 || (dy[i] == 0 && dx[i] > 0)) ? 0 : -1;
-    }
-    const int32_t Px0 = r.x0 * 256 + 128;
-    for (int py = r.y0; py <= r.y1; ++py) {
-      const int32_t Py = py * 256 + 128;
-      int32_t e[3];
-#pragma unroll
-      for (int i = 0; i < 3; ++i) e[i] = dx[i] * (Py - Y[i]) - dy[i] * (Px0 - X[i]) + bias[i];
-      for (int px = r.x0; px <= r.x1; ++px) {
-        if ((e[0] | e[1] | e[2]) >= 0) {
-          ++*rc.frags;
-          depth_key_min(rc, z0, dzdx, dzdy, zlo, X, Y, prim, px, py);
-        }
-#pragma unroll
-        for (int i = 0; i < 3; ++i) e[i] -= dy[i] * 256;
-      }
-    }
-    return;
-  }
-  // large boxes: the same edge functions in 64 bits, stepped along the row
-  int32_t dx[3], dy[3];
+  int32_t dx[3], dy[3], er[3];
+  const int32_t Px0 = (r.x0 << 8) | 128, Py0 = (r.y0 << 8) | 128;
+  const bool small = small_box(X, Y);
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     const int j = (i + 1) % 3;
     dx[i] = X[j] - X[i];
     dy[i] = Y[j] - Y[i];
+    const int32_t bias = (dy[i] < 0 || (dy[i] == 0 && dx[i] > 0)) ? 0 : -1;
+    if (small)
+      er[i] = (imul24(dx[i], Py0 - Y[i]) - imul24(dy[i], Px0 - X[i]) + bias) >> 8;
+    else
+      er[i] = edge_steps((long long)dx[i] * (Py0 - Y[i]) - (long long)dy[i] * (Px0 - X[i]) + bias);
   }
-  const long long Px0 = (long long)r.x0 * 256 + 128;
+  const float floor_z = depth_floor(zlo, z0, dzdx, dzdy);
+  const float fx0 = (float)(Px0 - X[0]);
+  float fy = (float)(Py0 - Y[0]);
+  int at = __mul24(r.y0 - rc.bin.y0, rc.B) + (r.x0 - rc.bin.x0);
+  const int w = r.x1 - r.x0 + 1;
   for (int py = r.y0; py <= r.y1; ++py) {
-    const long long Py = (long long)py * 256 + 128;
-    long long e[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const long long bias = (dy[i] < 0 || (dy[i] == 0 && dx[i] > 0)) ? 0 : -1;
-      e[i] = (long long)dx[i] * (Py - Y[i]) - (long long)dy[i] * (Px0 - X[i]) + bias;
-    }
-    for (int px = r.x0; px <= r.x1; ++px) {
-      if ((e[0] | e[1] | e[2]) >= 0) {
+    int32_t e0 = er[0], e1 = er[1], e2 = er[2];
+    const float zy = dzdy * fy;
+    float fx = fx0;
+    for (int i = 0; i < w; ++i) {
+      if ((e0 | e1 | e2) >= 0) {
         ++*rc.frags;
-        depth_key_min(rc, z0, dzdx, dzdy, zlo, X, Y, prim, px, py);
+        merge_key(rc.vis, at + i, z0 + dzdx * fx, zy, floor_z, prim);
       }
-#pragma unroll
-      for (int i = 0; i < 3; ++i) e[i] -= (long long)dy[i] * 256;
+      e0 -= dy[0];
+      e1 -= dy[1];
+      e2 -= dy[2];
+      fx += 256.0f;
     }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) er[i] += dx[i];
+    fy += 256.0f;
+    at += rc.B;
   }
 }
 
@@ -1114,14 +1121,14 @@ __device__ __forceinline__ int raster_classify(const RasterCtx& rc, const int32_
   r = tri_pixels(X, Y, rc.bin);
   if (r.x0 > r.x1 || r.y0 > r.y1) return 0;
   const int npx = (r.x1 - r.x0 + 1) * (r.y1 - r.y0 + 1);
+  *rc.pairs += (uint32_t)npx;
   if (npx > rc.lane_limit) {
     const int slot = atomicAdd(rc.nbig, 1);
     if (slot < kBigQueue) {
-      make_big(rc, X, Y, z0, dzdx, dzdy, zlo, prim, r, npx, rc.big[slot]);
+      make_big(rc, X, Y, z0, dzdx, dzdy, zlo, prim, r, rc.big[slot]);
       return -1;
     }
   }
-  *rc.pairs += (uint32_t)npx;
   return npx;
 }
 
@@ -1682,9 +1689,8 @@ __device__ __forceinline__ void overflow_rect(const FrameParams& p, const SceneD
 // short list spreads over the whole grid instead of filling a few waves:
 // the binning of a primitive close to the camera, which touches every bin
 // of its tile, is the longest part, and with 64 primitives in one wave and a
-// fan per lane it took 96 us a frame for 54 primitives at 640x480 (300 bins
-// a tile); this way 22 us, and 21 instead of 24 us on the plain 512-env frame
-// (1574 primitives, 16 bins a tile).
+// fan per lane it took 95 us a frame for 54 primitives at 640x480 (300 bins
+// a tile).
 constexpr int kClipBlock = 64;
 constexpr int kClipFans = kClipBlock * (kMaxPoly - 2);  // fan triangles of one wave at most
 
@@ -1953,12 +1959,37 @@ __device__ __forceinline__ uint32_t load_raster_rec(const FrameParams& p, unsign
 
 __device__ __forceinline__ void store_vis(const FrameParams& p, const BinInfo& b,
                                           const unsigned long long* s_vis, int B) {
+  const int tid = local_tid();
   const int bw = b.bin.x1 - b.bin.x0 + 1, bh = b.bin.y1 - b.bin.y0 + 1;
   const float inv_bw = 1.0f / (float)bw;
-  for (int l = threadIdx.x; l < bw * bh; l += kBlock) {
+  for (int l = tid; l < bw * bh; l += kBlock) {
     const int ly = div_small(l, inv_bw), lx = l - ly * bw;
     p.vis[(size_t)b.plane_offset + (size_t)(b.bin.y0 + ly) * b.stride + b.bin.x0 + lx] =
         s_vis[ly * B + lx];
+  }
+}
+
+// a bin's stored keys into an LDS tile of rows of B keys
+__device__ __forceinline__ void load_vis(const FrameParams& p, const BinInfo& b,
+                                         unsigned long long* tile, int B) {
+  const int tid = local_tid();
+  constexpr int kPer = kMaxBin * kMaxBin / kBlock;
+  const int bw = b.bin.x1 - b.bin.x0 + 1, bh = b.bin.y1 - b.bin.y0 + 1;
+  unsigned long long keys[kPer];
+  const float inv_bw = 1.0f / (float)bw;
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) {
+    const int l = tid + q * kBlock;
+    const int ly = div_small(l, inv_bw), lx = l - ly * bw;
+    keys[q] = l < bw * bh
+                  ? p.vis[(size_t)b.plane_offset + (size_t)(b.bin.y0 + ly) * b.stride + b.bin.x0 + lx]
+                  : 0ull;
+  }
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) {
+    const int l = tid + q * kBlock;
+    const int ly = div_small(l, inv_bw), lx = l - ly * bw;
+    if (l < bw * bh) tile[ly * B + lx] = keys[q];
   }
 }
 
@@ -2028,31 +2059,46 @@ __device__ __forceinline__ void add_raster_stats(const FrameParams& p, uint32_t 
   }
 }
 
+// the value of another lane of the same eight (a DPP control word)
+template <int kCtrl>
+__device__ __forceinline__ uint32_t lane_move(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, kCtrl, 0xF, 0xF, true);
+}
+
 // Depth pyramid of one 32x32 bin (s_vis rows of kMaxBin keys) from its final
 // phase-1 keys in LDS: max depth per level-0 block (2^kHiZ0 pixels square)
 // and over the bin (level 1), the same values k_hiz computes from the
 // stored keys.
 __device__ void bin_hiz(const FrameParams& p, const BinInfo& b, const unsigned long long* s_vis) {
+  const int tid = local_tid();
   constexpr int kN = kHiZPer * kHiZPer;
+  static_assert(kHiZ0 == 3 && kBlock / kMaxBin == 8, "a pass covers one row of blocks");
   __shared__ uint32_t s_max[kN];
-  if (threadIdx.x < kN) s_max[threadIdx.x] = 0u;
+  if (tid < kN) s_max[tid] = 0u;
   __syncthreads();
   const int bw = b.bin.x1 - b.bin.x0 + 1, bh = b.bin.y1 - b.bin.y0 + 1;
-  for (int l = threadIdx.x; l < kMaxBin * kMaxBin; l += kBlock) {
-    const int lx = l & 31, ly = l >> 5;
-    if (lx < bw && ly < bh)
-      atomicMax(&s_max[(ly >> kHiZ0) * kHiZPer + (lx >> kHiZ0)],
-                (uint32_t)(s_vis[ly * kMaxBin + lx] >> 32));
+  // eight neighbouring lanes hold a block's row: their maximum by lane
+  // moves, then one LDS atomic per row (an atomic per pixel puts 16 lanes on
+  // one address and took 4.8 us of a bin's 35)
+  const int lx = tid & 31;
+#pragma unroll
+  for (int q = 0; q < kMaxBin * kMaxBin / kBlock; ++q) {
+    const int ly = 8 * q + (tid >> 5);
+    uint32_t z = lx < bw && ly < bh ? (uint32_t)(s_vis[ly * kMaxBin + lx] >> 32) : 0u;
+    z = max(z, lane_move<0xB1>(z));   // lane ^ 1
+    z = max(z, lane_move<0x4E>(z));   // lane ^ 2
+    z = max(z, lane_move<0x141>(z));  // the other four of eight
+    if ((lx & 7) == 0) atomicMax(&s_max[q * kHiZPer + (lx >> kHiZ0)], z);
   }
   __syncthreads();
   const int rx = b.bin.x0 >> kHiZ1, ry = b.bin.y0 >> kHiZ1;
   float* h = p.hiz + (size_t)b.scene * p.hiz_stride;
-  if (threadIdx.x < kN) {
-    const int bx = rx * kHiZPer + (int)(threadIdx.x % kHiZPer),
-              by = ry * kHiZPer + (int)(threadIdx.x / kHiZPer);
-    if (bx < p.hiz_w0 && by < p.hiz_h0) h[by * p.hiz_w0 + bx] = __uint_as_float(s_max[threadIdx.x]);
+  if (tid < kN) {
+    const int bx = rx * kHiZPer + (int)(tid % kHiZPer),
+              by = ry * kHiZPer + (int)(tid / kHiZPer);
+    if (bx < p.hiz_w0 && by < p.hiz_h0) h[by * p.hiz_w0 + bx] = __uint_as_float(s_max[tid]);
   }
-  if (threadIdx.x == 0) {
+  if (tid == 0) {
     uint32_t m = 0;
     for (int k = 0; k < kN; ++k) m = max(m, s_max[k]);
     h[p.hiz_w0 * p.hiz_h0 + ry * p.hiz_w1 + rx] = __uint_as_float(m);
@@ -2072,13 +2118,24 @@ __device__ void bin_hiz(const FrameParams& p, const BinInfo& b, const unsigned l
 // resolves in place, resolves them from their phase-1 keys).
 // --------------------------------------------------------------------------
 
+// a range of the queue: its first bin, heavy bins, entries, and the number
+// of workgroups whose first bin it gives
+struct RasterRange {
+  uint32_t first, heavy, total, fixed;
+};
+
 struct RasterLds {
   unsigned long long vis[kMaxBin * kMaxBin];
   BigTri big[kBigQueue];
   float lut[256];  // unorm8 -> float, for resolving in place
   int nbig[2];     // queue fill of even / odd batches
-  int next[2];     // next queue entry to claim, even / odd batches
+  uint32_t next;   // the bin to rasterise next (kNoBin: none)
+  RasterRange ranges[kRasterParts];  // the queue's ranges, this workgroup's own first
 };
+
+// A raster queue entry: the bin, with kRestBin set when it comes from the
+// range's bins in order (it may then be a heavy bin, taken from that list).
+constexpr uint32_t kNoBin = ~0u, kRestBin = 0x80000000u;
 
 template <bool kLights>
 __device__ void resolve_tile(const FrameParams& p, const RasterItem& it,
@@ -2098,11 +2155,12 @@ __host__ __device__ __forceinline__ bool resolves_in_place(const FrameParams& p,
 template <bool kResolve>
 __device__ void raster_bin(const FrameParams& p, const RasterItem& item, int phase, RasterLds& L,
                            uint32_t& pairs, uint32_t& frags) {
+  const int tid = local_tid();
   const BinInfo b = bin_info(item);
   const uint32_t* entries = p.bin_entries + b.entries;
   // the first entries load beside the count (both addresses are known; an
   // entry at or past the count is never used)
-  const uint32_t e_first = threadIdx.x < b.bin_cap ? entries[threadIdx.x] : 0u;
+  const uint32_t e_first = tid < b.bin_cap ? entries[tid] : 0u;
   const uint32_t n = p.bin_count[b.gbin];
   if (n > b.bin_cap) return;  // overflowed: k_raster_full rescans this bin
   // with kResolve every bin is resolved here, also those without new
@@ -2120,7 +2178,7 @@ __device__ void raster_bin(const FrameParams& p, const RasterItem& item, int pha
   // the first batch's records are in flight while the tile is set up
   RasterRec rr_first = {};
   uint32_t prim_first = 0;
-  if (threadIdx.x < n) prim_first = fetch_raster_rec(p, b.rec_base, e_first, rr_first);
+  if (tid < n) prim_first = fetch_raster_rec(p, b.rec_base, e_first, rr_first);
   const int bw = b.bin.x1 - b.bin.x0 + 1, bh = b.bin.y1 - b.bin.y0 + 1;
   if (phase == 2) {
     constexpr int kPer = kMaxBin * kMaxBin / kBlock;
@@ -2128,7 +2186,7 @@ __device__ void raster_bin(const FrameParams& p, const RasterItem& item, int pha
     const float inv_bw = 1.0f / (float)bw;
 #pragma unroll
     for (int q = 0; q < kPer; ++q) {
-      const int l = threadIdx.x + q * kBlock;
+      const int l = tid + q * kBlock;
       const int ly = div_small(l, inv_bw), lx = l - ly * bw;
       keys[q] = l < bw * bh
                     ? p.vis[(size_t)b.plane_offset + (size_t)(b.bin.y0 + ly) * b.stride + b.bin.x0 + lx]
@@ -2136,14 +2194,14 @@ __device__ void raster_bin(const FrameParams& p, const RasterItem& item, int pha
     }
 #pragma unroll
     for (int q = 0; q < kPer; ++q) {
-      const int l = threadIdx.x + q * kBlock;
+      const int l = tid + q * kBlock;
       const int ly = div_small(l, inv_bw), lx = l - ly * bw;
       if (l < bw * bh) L.vis[ly * B + lx] = keys[q];
     }
   } else {
-    for (int i = threadIdx.x; i < B * B; i += kBlock) L.vis[i] = kClearKey;
+    for (int i = tid; i < B * B; i += kBlock) L.vis[i] = kClearKey;
   }
-  if (threadIdx.x == 0) L.nbig[0] = L.nbig[1] = L.next[0] = L.next[1] = 0;
+  if (tid == 0) L.nbig[0] = L.nbig[1] = 0;
   __syncthreads();
   // per batch of kBlock entries: lanes append large rectangles to the queue
   // (fill and claim counters of this batch's parity; the other ones, read
@@ -2151,9 +2209,9 @@ __device__ void raster_bin(const FrameParams& p, const RasterItem& item, int pha
   // batch), then the waves take the queued triangles one at a time
   int parity = 0;
   for (uint32_t base = 0; base < n; base += kBlock, parity ^= 1) {
-    const uint32_t k = base + threadIdx.x;
+    const uint32_t k = base + tid;
     rc.nbig = &L.nbig[parity];
-    if (threadIdx.x == 0) L.nbig[parity ^ 1] = L.next[parity ^ 1] = 0;
+    if (tid == 0) L.nbig[parity ^ 1] = 0;
     if (k < n) {
       int32_t X[3], Y[3];
       float z0, dzdx, dzdy, zlo;
@@ -2167,7 +2225,7 @@ __device__ void raster_bin(const FrameParams& p, const RasterItem& item, int pha
       raster_planed(rc, X, Y, z0, dzdx, dzdy, zlo, prim);
     }
     __syncthreads();
-    raster_big_waves(rc, L.big, min(L.nbig[parity], kBigQueue), &L.next[parity]);
+    raster_big_waves(rc, L.big, min(L.nbig[parity], kBigQueue));
     __syncthreads();
   }
   if (kResolve) {
@@ -2176,17 +2234,15 @@ __device__ void raster_bin(const FrameParams& p, const RasterItem& item, int pha
     store_vis(p, b, L.vis, B);
     if (phase == 1 && p.hiz_fused) bin_hiz(p, b, L.vis);
   }
-  if (threadIdx.x == 0) p.bin_count[b.gbin] = 0;  // ready for the next frame
+  if (tid == 0) p.bin_count[b.gbin] = 0;  // ready for the next frame
 }
 
-// kWaves: the waves per SIMD the register allocation must allow.  Without
-// resolve 6 (80 VGPRs, no spills): the bins' chains of dependent global
-// loads are latency-bound, and 6 resident workgroups per CU rasterise the
-// first phase ~7% faster than 5 (at 7 the walk spills).  With the resolve,
-// 5 when the resolving phase is the only one (every bin rasterised: a few
-// spilled registers cost less than the lost occupancy, plain frame -4%)
-// and 4 (no spills) after the depth-pyramid phase, whose bins mostly only
-// resolve.
+// kWaves: the waves per SIMD the register allocation must allow.  A bin is a
+// chain of dependent loads and barriers, so resident workgroups are what the
+// kernel needs most: without the resolve 8 (64 VGPRs, 20 KB of LDS), measured
+// on the learned 512-env frame 148 / 139 / 133 us at 6 / 7 / 8; with the
+// resolve 5 (96 VGPRs, 4 spilled; 183 -> 173 us after the depth pyramid
+// against 4 without spills).
 template <bool kResolve, int kWaves>
 __global__ __launch_bounds__(kBlock, kWaves) void k_raster_lane(FrameParams p,
                                                         const RasterItem* __restrict__ items,
@@ -2362,7 +2418,7 @@ __global__ __launch_bounds__(kBlock) void k_raster_full(FrameParams p,
   __shared__ unsigned long long s_vis[kMaxBin * kMaxBin];
   __shared__ BigTri s_big[kBigQueue];
   __shared__ uint32_t s_base[kDrawCache];
-  __shared__ int s_nbig, s_next;
+  __shared__ int s_nbig;
   __shared__ float s_lut[256];
 
   const uint32_t n_over =
@@ -2389,7 +2445,7 @@ __global__ __launch_bounds__(kBlock) void k_raster_full(FrameParams p,
     if (sc.draw_count <= (uint32_t)kDrawCache)
       for (uint32_t i = threadIdx.x; i < sc.draw_count; i += kBlock)
         s_base[i] = p.draws[sc.draw_begin + i].prim_base;
-    if (threadIdx.x == 0) s_nbig = s_next = 0;
+    if (threadIdx.x == 0) s_nbig = 0;
     float PV[16];
     load_mat(p.cameras + (size_t)it.scene * 16, PV);
     __syncthreads();
@@ -2397,9 +2453,9 @@ __global__ __launch_bounds__(kBlock) void k_raster_full(FrameParams p,
       const uint32_t k = base + threadIdx.x;
       if (k < sc.prim_count) raster_prim(p, sc, PV, rc, s_base, k);
       __syncthreads();
-      raster_big_waves(rc, s_big, min(s_nbig, kBigQueue), &s_next);
+      raster_big_waves(rc, s_big, min(s_nbig, kBigQueue));
       __syncthreads();
-      if (threadIdx.x == 0) s_nbig = s_next = 0;
+      if (threadIdx.x == 0) s_nbig = 0;
       __syncthreads();
     }
     if (resolves_in_place(p, phase)) {
@@ -2430,6 +2486,7 @@ __global__ __launch_bounds__(kBlock) void k_raster_full(FrameParams p,
 template <bool kLights>
 __device__ void resolve_tile(const FrameParams& p, const RasterItem& it,
                              const unsigned long long* tile, int B, const float* s_lut) {
+  const int tid = local_tid();
   const BinInfo b = bin_info(it);
   const uint32_t frame = *p.frame;
   const float un0 = p.unprojections[2 * it.scene], un1 = p.unprojections[2 * it.scene + 1];
@@ -2439,7 +2496,7 @@ __device__ void resolve_tile(const FrameParams& p, const RasterItem& it,
   // in a full bin the pixels of a 2x2 quad sit in lanes {l, l^1, l^bw, l^1^bw}
   // of one wave (rows of bw pixels, bw in {8, 16, 32}, even bin origin)
   const bool quads = bw == p.bin_size && bh == p.bin_size;
-  const int lane = threadIdx.x & 63;
+  const int lane = tid & 63;
   const float hw = (float)b.width * 0.5f, hh = (float)b.height * 0.5f;
   const float ihw = 1.0f / hw, ihh = 1.0f / hh;
   const float inv_bw = 1.0f / (float)bw;
@@ -2449,7 +2506,7 @@ __device__ void resolve_tile(const FrameParams& p, const RasterItem& it,
   const bool want_lin = p.out_lindepth && (b.planes & GBR_PLANE_LINEAR_DEPTH);
   const bool want_sem = p.out_semantic && (b.planes & GBR_PLANE_SEMANTIC);
   for (int base = 0; base < npx; base += kBlock) {
-    const int l = base + (int)threadIdx.x;
+    const int l = base + tid;
     const bool valid = l < npx;
     const int ly = div_small(l, inv_bw), lx = l - ly * bw;
     const int px = b.bin.x0 + lx, py = b.bin.y0 + ly;
@@ -2515,29 +2572,6 @@ __device__ void resolve_tile(const FrameParams& p, const RasterItem& it,
       p.out_lindepth[o] = lin == far_depth ? 0.0f : lin;
     }
     if (want_sem) p.out_semantic[o] = d.semantic;
-  }
-}
-
-// a bin's stored keys into an LDS tile of rows of B keys
-__device__ __forceinline__ void load_vis(const FrameParams& p, const BinInfo& b,
-                                         unsigned long long* tile, int B) {
-  constexpr int kPer = kMaxBin * kMaxBin / kBlock;
-  const int bw = b.bin.x1 - b.bin.x0 + 1, bh = b.bin.y1 - b.bin.y0 + 1;
-  unsigned long long keys[kPer];
-  const float inv_bw = 1.0f / (float)bw;
-#pragma unroll
-  for (int q = 0; q < kPer; ++q) {
-    const int l = threadIdx.x + q * kBlock;
-    const int ly = div_small(l, inv_bw), lx = l - ly * bw;
-    keys[q] = l < bw * bh
-                  ? p.vis[(size_t)b.plane_offset + (size_t)(b.bin.y0 + ly) * b.stride + b.bin.x0 + lx]
-                  : 0ull;
-  }
-#pragma unroll
-  for (int q = 0; q < kPer; ++q) {
-    const int l = threadIdx.x + q * kBlock;
-    const int ly = div_small(l, inv_bw), lx = l - ly * bw;
-    if (l < bw * bh) tile[ly * B + lx] = keys[q];
   }
 }
 
@@ -3097,14 +3131,12 @@ hipError_t launch_clip(const FrameParams& p, uint32_t grid, int phase, hipStream
   return hipGetLastError();
 }
 
-// the lane rasteriser's workgroups per CU: kind 0 stores the keys, 1
-// resolves a frame's only raster phase, 2 resolves after the depth pyramid
-int raster_blocks_per_cu(int kind) {
+// the lane rasteriser's workgroups per CU, storing the keys or resolving
+int raster_blocks_per_cu(bool resolve) {
   int b = 0;
   const hipError_t e =
-      kind == 1   ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_raster_lane<true, 5>, kBlock, 0)
-      : kind == 2 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_raster_lane<true, 4>, kBlock, 0)
-                  : hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_raster_lane<false, 6>, kBlock, 0);
+      resolve ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_raster_lane<true, 5>, kBlock, 0)
+              : hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_raster_lane<false, 8>, kBlock, 0);
   if (e != hipSuccess || b < 1) b = 4;
   return b;
 }
@@ -3116,14 +3148,11 @@ hipError_t launch_raster(const FrameParams& p, const RasterItem* items, uint32_t
   if (n == 0) return hipSuccess;
   if (p.raster_mode == 1)
     hipLaunchKernelGGL(k_raster_pairs, dim3(n), dim3(kBlock), 0, s, p, items, phase);
-  else if (resolves_in_place(p, phase) && phase == 1)
+  else if (resolves_in_place(p, phase))
     hipLaunchKernelGGL((k_raster_lane<true, 5>), dim3(grid < n ? grid : n), dim3(kBlock), 0, s, p,
                        items, n, phase);
-  else if (resolves_in_place(p, phase))
-    hipLaunchKernelGGL((k_raster_lane<true, 4>), dim3(grid < n ? grid : n), dim3(kBlock), 0, s, p,
-                       items, n, phase);
   else
-    hipLaunchKernelGGL((k_raster_lane<false, 6>), dim3(grid < n ? grid : n), dim3(kBlock), 0, s, p,
+    hipLaunchKernelGGL((k_raster_lane<false, 8>), dim3(grid < n ? grid : n), dim3(kBlock), 0, s, p,
                        items, n, phase);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
