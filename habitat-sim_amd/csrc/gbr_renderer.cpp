@@ -494,7 +494,17 @@ gbr_status rebuild_structure(gbr_renderer* r) {
     tris += prim;
     const uint32_t nb = (uint32_t)(bins_x * bins_y);
     sd.bin_base = (uint32_t)bins;
+    // A camera sees its triangles unevenly: a bin of a scene with few
+    // triangles, or with many bins, gets several times the average, and an
+    // overflowed bin costs a rescan of the whole scene (54 us of a 145 us
+    // frame of 16 rooms, 250 of 1000 us on 512 uneven environments).  So a
+    // bin holds kSkew times its share, up to kSkewCap entries, at 64 bytes
+    // per triangle at most beside the 96 of its records.  A factor below 1
+    // asks for bins smaller than the average: it gets exactly its share.
+    constexpr double kSkew = 8.0, kSkewCap = 4096.0;
     double per_bin = (double)prim / nb * r->tun.bin_capacity_factor;
+    if (r->tun.bin_capacity_factor >= 1.0f)
+      per_bin = std::max(per_bin, std::min(kSkew * per_bin, kSkewCap));
     uint32_t cap = (uint32_t)std::min<double>(std::max<double>(per_bin, r->tun.min_bin_capacity), 1u << 24);
     cap = (cap + 63) & ~63u;
     sd.bin_cap = cap;
