@@ -276,10 +276,32 @@ struct alignas(16) LightDesc {
   float pad2;
 };
 
+// TextureDesc::filter
+enum : uint32_t {
+  kTexMagLinear = 1u,   // magnified: bilinear, else nearest
+  kTexMinLinear = 2u,   // minified: bilinear within a level, else nearest
+  kTexMipNone = 4u,     // minified: level 0 only
+  kTexMipNearest = 8u,  // minified: the nearest level (neither bit: two levels blended)
+  kTexMagHalf = 16u,    // magnification up to a level of detail of 0.5 (GL 4.6 8.14)
+  kTexWrapSlow = 32u,   // an axis is neither clamp-to-edge nor a power-of-two repeat
+};
+
+// One mip level: where it starts and the texels of one layer.
+struct alignas(16) TexLevel {
+  int64_t offset;  // byte offset into texels[]
+  uint32_t texels;
+  uint32_t pad;
+};
+
+// A texel index along a fast axis of w texels wraps as
+// clamp(i & ((w - 1) | wrap_or), 0, w - 1): wrap_or is 0 for a power-of-two
+// repeat (whose levels are powers of two as well) and -1 for clamp-to-edge.
 struct alignas(16) TextureDesc {
   int32_t width, height, layers, levels;
-  int32_t min_filter, mag_filter, wrap_s, wrap_t;
-  int64_t level_offset[16];  // byte offsets into texels[]
+  uint32_t filter;
+  int32_t wrap_or_s, wrap_or_t;
+  uint32_t wraps;  // GL wrap modes: s | t << 16 (kTexWrapSlow textures)
+  TexLevel level[16];
 };
 
 struct FrameParams {
@@ -295,6 +317,7 @@ struct FrameParams {
   // materials / textures
   const MaterialDesc* materials;
   const TextureDesc* textures;
+  uint32_t n_textures;
   const uint8_t* texels;
   const float* unorm_lut;  // i/255.0f, 256 entries
   // scenes

@@ -118,6 +118,27 @@ __device__ __forceinline__ int local_tid() {
   return t;
 }
 
+// 1 / x, correctly rounded, for 2^-126 <= |x| <= 2^126: the hardware
+// reciprocal (1 ulp) and one Newton step in fused arithmetic, three
+// instructions instead of the ten of the general division.  (Compared with
+// it over every float of that range.)
+__device__ __forceinline__ float rcp_exact(float x) {
+  const float r = __builtin_amdgcn_rcpf(x);
+  return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+}
+
+// a / b, correctly rounded, from r = rcp_exact(b), where a, b and a / b stay
+// within 2^+-60 (or a is 0): the quotient's remainder corrects it (Markstein
+// 1990)
+__device__ __forceinline__ float div_exact(float a, float b, float r) {
+  const float q = a * r;
+  return __builtin_fmaf(__builtin_fmaf(-b, q, a), r, q);
+}
+
+__device__ __forceinline__ bool in_range(float x, float lo, float hi) {
+  return __builtin_amdgcn_fmed3f(fabsf(x), lo, hi) == fabsf(x);
+}
+
 struct Snap {
   int32_t X, Y;
   float z;
@@ -1228,7 +1249,8 @@ __device__ __forceinline__ float gbr_log2(float x) {
   if (e == 0) return -126.0f;
   if (e == 0xff) return 128.0f;
   float m = __uint_as_float((bits & 0x7fffffu) | 0x3f800000u);
-  float y = (m - 1.0f) / (m + 1.0f);
+  const float d = m + 1.0f;
+  float y = div_exact(m - 1.0f, d, rcp_exact(d));  // (compared with the division for every m)
   float y2 = y * y;
   float s = y2 * (1.0f / 9.0f);
   s = s + (1.0f / 7.0f);
@@ -1243,8 +1265,9 @@ __device__ __forceinline__ float gbr_log2(float x) {
   return (float)(e - 127) + l;
 }
 
-// mirrored repeat, and repeat of a size that is not a power of two
+// a texel index on an axis of `size` texels under any wrap mode
 __device__ __noinline__ int wrap_coord_slow(int i, int size, int mode) {
+  if (mode == GL_CLAMP_TO_EDGE) return min(max(i, 0), size - 1);
   if (mode == GL_MIRRORED_REPEAT) {
     int pp = 2 * size;
     int m = i % pp;
@@ -1256,25 +1279,6 @@ __device__ __noinline__ int wrap_coord_slow(int i, int size, int mode) {
   return m;
 }
 
-// GL wrap of texel indices along one axis of one level, decided once per
-// level: clamp-to-edge and power-of-two repeat share one form,
-// clamp(i & mask, 0, size - 1) (mask = size - 1 for repeat, all ones for
-// clamp), the rest (mirrored repeat, repeat of other sizes) goes out of line.
-struct AxisWrap {
-  int size, mask, mode;
-  bool fast;
-};
-
-__device__ __forceinline__ AxisWrap axis_wrap(int size, int mode) {
-  const bool clamp = mode == GL_CLAMP_TO_EDGE;
-  AxisWrap a;
-  a.size = size;
-  a.mode = mode;
-  a.fast = clamp || (mode != GL_MIRRORED_REPEAT && (size & (size - 1)) == 0);
-  a.mask = clamp ? -1 : size - 1;
-  return a;
-}
-
 // min(max(x, 0), hi) in one instruction
 __device__ __forceinline__ int clamp0(int x, int hi) {
   int r;
@@ -1282,41 +1286,75 @@ __device__ __forceinline__ int clamp0(int x, int hi) {
   return r;
 }
 
-__device__ __forceinline__ int wrap_coord(const AxisWrap& a, int i) {
-  if (__builtin_expect(a.fast, 1)) return clamp0(i & a.mask, a.size - 1);
-  return wrap_coord_slow(i, a.size, a.mode);
+// floor of u clamped to [-2^30, 2^30], as an integer-valued float (the clamp
+// as one median; u is finite)
+__device__ __forceinline__ float floor_clamped(float u) {
+  return floorf(__builtin_amdgcn_fmed3f(u, -1073741824.0f, 1073741824.0f));
 }
 
-// floor of u clamped to [-2^30, 2^30] (the clamp as one median; u is finite)
-__device__ __forceinline__ int floor_to_int(float u) {
-  u = __builtin_amdgcn_fmed3f(u, -1073741824.0f, 1073741824.0f);
-  return (int)floorf(u);
+// What the resolve keeps in LDS: the unorm8 -> float table, and the
+// descriptors of the first kLdsTextures textures.  The resolve is bound by
+// the L1's accesses beside its VALU work (610 accesses per 64 pixels on the
+// 512-env frame), and a descriptor costs every pixel two dependent loads,
+// of the header and of the level.
+constexpr uint32_t kLdsTextures = 8;
+
+struct ResolveLds {
+  TextureDesc tex[kLdsTextures];
+  float lut[256];
+};
+
+// fills it (every thread of the workgroup; a barrier is left to the caller)
+__device__ __forceinline__ void resolve_lds_fill(const FrameParams& p, ResolveLds& L) {
+  static_assert(kBlock == 256 && sizeof(TextureDesc) % 16 == 0, "one LUT entry per thread");
+  L.lut[threadIdx.x] = p.unorm_lut[threadIdx.x];
+  const uint32_t words = min(p.n_textures, kLdsTextures) * (uint32_t)(sizeof(TextureDesc) / 16);
+  for (uint32_t i = threadIdx.x; i < words; i += kBlock)
+    reinterpret_cast<uint4*>(L.tex)[i] = reinterpret_cast<const uint4*>(p.textures)[i];
 }
 
-// A texture's header held in registers (one 32-byte load), and the byte
-// offset of the level being sampled: every field is read once per pixel
+// A texture's header held in registers: every field is read once per pixel
 // instead of once per use.
 struct TexHeader {
   int32_t width, height, layers, levels;
-  int32_t min_filter, mag_filter, wrap_s, wrap_t;
+  uint32_t filter;
+  int32_t wrap_or_s, wrap_or_t;
+  uint32_t wraps;
 };
 
-__device__ __forceinline__ TexHeader load_tex_header(const TextureDesc* t) {
-  const int4 a = *reinterpret_cast<const int4*>(t);
-  const int4 b = *(reinterpret_cast<const int4*>(t) + 1);
-  return TexHeader{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+__device__ __forceinline__ TexHeader load_tex_header(const FrameParams& p, const ResolveLds& L,
+                                                     uint32_t texture) {
+  int4 a, b;
+  if (__builtin_expect(texture < kLdsTextures, 1)) {
+    a = reinterpret_cast<const int4*>(&L.tex[texture])[0];
+    b = reinterpret_cast<const int4*>(&L.tex[texture])[1];
+  } else {
+    a = reinterpret_cast<const int4*>(p.textures + texture)[0];
+    b = reinterpret_cast<const int4*>(p.textures + texture)[1];
+  }
+  return TexHeader{a.x, a.y, a.z, a.w, (uint32_t)b.x, b.y, b.z, (uint32_t)b.w};
+}
+
+__device__ __forceinline__ TexLevel load_tex_level(const FrameParams& p, const ResolveLds& L,
+                                                   uint32_t texture, int level) {
+  if (__builtin_expect(texture < kLdsTextures, 1)) return L.tex[texture].level[level];
+  return p.textures[texture].level[level];
 }
 
 // texel `row + i` of a level whose first byte is `base`: row = (layer * h
 // + j) * w in 32-bit arithmetic, as the texel index always was
-__device__ __forceinline__ void fetch(const float* lut, const uint8_t* base, uint32_t row,
-                                      int i, float* out) {
-  const uint32_t idx = row + (uint32_t)i;
-  const uint32_t texel = *reinterpret_cast<const uint32_t*>(base + (size_t)idx * 4);
-  out[0] = lut[texel & 0xff];
-  out[1] = lut[(texel >> 8) & 0xff];
-  out[2] = lut[(texel >> 16) & 0xff];
-  out[3] = lut[texel >> 24];
+__device__ __forceinline__ uint32_t texel_at(const uint8_t* base, uint32_t row, int i) {
+  return *reinterpret_cast<const uint32_t*>(base + (size_t)(row + (uint32_t)i) * 4);
+}
+
+// Texels i and i + 1 of a row in one 8-byte load: a bilinear footprint, whose
+// second texel follows the first unless they wrap or clamp at an edge, takes
+// two such loads instead of four, and half the L1 accesses.  (The texel after
+// the blob's last one may be read, not used: the buffer has room for it.)
+typedef uint32_t TexelPair __attribute__((ext_vector_type(2), aligned(4)));
+
+__device__ __forceinline__ TexelPair texel_pair_at(const uint8_t* base, uint32_t row, int i) {
+  return *reinterpret_cast<const TexelPair*>(base + (size_t)(row + (uint32_t)i) * 4);
 }
 
 // (layer * h + j) * w mod 2^32 as layer_off + j * w, layer_off = layer * h * w
@@ -1326,38 +1364,58 @@ __device__ __forceinline__ uint32_t texel_row(uint32_t layer_off, int j, int w) 
   return layer_off + __umul24((uint32_t)j, (uint32_t)w);
 }
 
-__device__ void sample_level(const float* lut, const TexHeader& t, const uint8_t* base, int level,
-                             int layer, float s, float tc, bool linear, float* out) {
-  int w = max(t.width >> level, 1), h = max(t.height >> level, 1);
-  const AxisWrap ws = axis_wrap(w, t.wrap_s), wt = axis_wrap(h, t.wrap_t);
-  float u = s * (float)w;
-  float v = tc * (float)h;
-  const uint32_t layer_off = (uint32_t)layer * (uint32_t)h * (uint32_t)w;
+__device__ __forceinline__ void unpack_texel(const float* lut, uint32_t texel, float* out) {
+  out[0] = lut[texel & 0xff];
+  out[1] = lut[(texel >> 8) & 0xff];
+  out[2] = lut[(texel >> 16) & 0xff];
+  out[3] = lut[texel >> 24];
+}
+
+// one level of a texture, bilinear or nearest
+__device__ __forceinline__ void sample_level(const FrameParams& p, const ResolveLds& L,
+                                             const TexHeader& t, uint32_t texture, int level,
+                                             int layer, float s, float tc, bool linear, float* out) {
+  const float* lut = L.lut;
+  const int w = max(t.width >> level, 1), h = max(t.height >> level, 1);
+  const TexLevel lv = load_tex_level(p, L, texture, level);
+  const uint8_t* base = p.texels + lv.offset;
+  const uint32_t layer_off = (uint32_t)layer * lv.texels;
+  const float u = s * (float)w, v = tc * (float)h;
+  // nearest: the texel at floor(u), floor(v); bilinear: the four around
+  // u - 1/2, v - 1/2
+  const float uu = linear ? u - 0.5f : u, vv = linear ? v - 0.5f : v;
+  const float fi = floor_clamped(uu), fj = floor_clamped(vv);
+  const int i = (int)fi, j = (int)fj;
+  const int ms = (w - 1) | t.wrap_or_s, mt = (h - 1) | t.wrap_or_t;
+  int i0 = clamp0(i & ms, w - 1), i1 = clamp0((i + 1) & ms, w - 1);
+  int j0 = clamp0(j & mt, h - 1), j1 = clamp0((j + 1) & mt, h - 1);
+  if (__builtin_expect(t.filter & kTexWrapSlow, 0)) {
+    const int mode_s = (int)(t.wraps & 0xffffu), mode_t = (int)(t.wraps >> 16);
+    i0 = wrap_coord_slow(i, w, mode_s);
+    i1 = wrap_coord_slow(i + 1, w, mode_s);
+    j0 = wrap_coord_slow(j, h, mode_t);
+    j1 = wrap_coord_slow(j + 1, h, mode_t);
+  }
+  const uint32_t r0 = texel_row(layer_off, j0, w);
   if (!linear) {
-    int i = wrap_coord(ws, floor_to_int(u));
-    int j = wrap_coord(wt, floor_to_int(v));
-    fetch(lut, base, texel_row(layer_off, j, w), i, out);
+    unpack_texel(lut, texel_at(base, r0, i0), out);
     return;
   }
-  float uu = u - 0.5f;
-  float vv = v - 0.5f;
-  int i0 = floor_to_int(uu);
-  int j0 = floor_to_int(vv);
-  float a = uu - (float)i0;
-  float b = vv - (float)j0;
-  int i1 = wrap_coord(ws, i0 + 1);
-  int j1 = wrap_coord(wt, j0 + 1);
-  i0 = wrap_coord(ws, i0);
-  j0 = wrap_coord(wt, j0);
-  const uint32_t r0 = texel_row(layer_off, j0, w), r1 = texel_row(layer_off, j1, w);
+  const uint32_t r1 = texel_row(layer_off, j1, w);
+  TexelPair x0 = texel_pair_at(base, r0, i0), x1 = texel_pair_at(base, r1, i0);
+  asm("" : "+v"(x0), "+v"(x1));  // (both halves, or the compiler loads the second ones apart)
+  if (i1 != i0 + 1) {
+    x0.y = texel_at(base, r0, i1);
+    x1.y = texel_at(base, r1, i1);
+  }
+  const float a = uu - fi, b = vv - fj;
+  const float ia = 1.0f - a, ib = 1.0f - b;
+  const float w00 = ia * ib, w10 = a * ib, w01 = ia * b, w11 = a * b;
   float t00[4], t10[4], t01[4], t11[4];
-  fetch(lut, base, r0, i0, t00);
-  fetch(lut, base, r0, i1, t10);
-  fetch(lut, base, r1, i0, t01);
-  fetch(lut, base, r1, i1, t11);
-  float ia = 1.0f - a;
-  float ib = 1.0f - b;
-  float w00 = ia * ib, w10 = a * ib, w01 = ia * b, w11 = a * b;
+  unpack_texel(lut, x0.x, t00);
+  unpack_texel(lut, x0.y, t10);
+  unpack_texel(lut, x1.x, t01);
+  unpack_texel(lut, x1.y, t11);
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     float r = w00 * t00[c];
@@ -1371,102 +1429,83 @@ __device__ void sample_level(const float* lut, const TexHeader& t, const uint8_t
   }
 }
 
-__device__ __forceinline__ const uint8_t* level_base(const FrameParams& p, const TextureDesc* td,
-                                                     int level) {
-  return p.texels + td->level_offset[level];
-}
-
-__device__ void sample_tex(const FrameParams& p, const float* lut, const TextureDesc* td,
-                           const TexHeader& t, int layer, float s, float tc, float lambda,
-                           float* out) {
-  if (layer < 0) layer = 0;
-  if (layer >= t.layers) layer = t.layers - 1;
-  float c = 0.0f;
-  if (t.mag_filter == GL_LINEAR &&
-      (t.min_filter == GL_NEAREST_MIPMAP_NEAREST || t.min_filter == GL_NEAREST_MIPMAP_LINEAR))
-    c = 0.5f;
-  if (lambda <= c) {
-    sample_level(lut, t, level_base(p, td, 0), 0, layer, s, tc, t.mag_filter == GL_LINEAR, out);
-    return;
-  }
+// GL 4.6 section 8.14: the level or levels and their filter are decided
+// first, so that every pixel of a wave takes the same one or two passes of
+// sample_level() whatever its level of detail
+__device__ __forceinline__ void sample_tex(const FrameParams& p, const ResolveLds& L,
+                                           uint32_t texture, const TexHeader& t, int layer,
+                                           float s, float tc, float lambda, float* out) {
+  layer = clamp0(layer, t.layers - 1);
+  const bool mag = lambda <= ((t.filter & kTexMagHalf) ? 0.5f : 0.0f);
+  const bool linear = (t.filter & (mag ? kTexMagLinear : kTexMinLinear)) != 0;
   const int q = t.levels - 1;
-  switch (t.min_filter) {
-    case GL_NEAREST:
-    case GL_LINEAR:
-      sample_level(lut, t, level_base(p, td, 0), 0, layer, s, tc, t.min_filter == GL_LINEAR, out);
-      return;
-    case GL_NEAREST_MIPMAP_NEAREST:
-    case GL_LINEAR_MIPMAP_NEAREST: {
-      int dlev;
-      if (lambda <= 0.5f)
-        dlev = 0;
-      else {
-        float f = ceilf(lambda + 0.5f) - 1.0f;
-        dlev = f > (float)q ? q : (int)f;
-      }
-      sample_level(lut, t, level_base(p, td, dlev), dlev, layer, s, tc,
-                   t.min_filter == GL_LINEAR_MIPMAP_NEAREST, out);
-      return;
+  int level = 0;
+  float f = 0.0f;
+  bool two = false;
+  if (!mag && !(t.filter & kTexMipNone)) {
+    if (t.filter & kTexMipNearest) {
+      const float d = lambda <= 0.5f ? 0.0f : ceilf(lambda + 0.5f) - 1.0f;
+      level = d > (float)q ? q : (int)d;
+    } else if (lambda >= (float)q) {
+      level = q;
+    } else {
+      const float fl = floorf(lambda);
+      level = (int)fl;
+      f = lambda - fl;
+      two = true;
     }
-    default: {
-      bool lin = t.min_filter == GL_LINEAR_MIPMAP_LINEAR;
-      if (lambda >= (float)q) {
-        sample_level(lut, t, level_base(p, td, q), q, layer, s, tc, lin, out);
-        return;
-      }
-      float fl = floorf(lambda);
-      int d1 = (int)fl;
-      float f = lambda - fl;
-      const uint8_t* b1 = level_base(p, td, d1);
-      const uint8_t* b2 = level_base(p, td, d1 + 1);
-      float t1[4], t2[4];
-      sample_level(lut, t, b1, d1, layer, s, tc, lin, t1);
-      sample_level(lut, t, b2, d1 + 1, layer, s, tc, lin, t2);
-      float g = 1.0f - f;
+  }
+  sample_level(p, L, t, texture, level, layer, s, tc, linear, out);
+  if (two) {
+    float t2[4];
+    sample_level(p, L, t, texture, level + 1, layer, s, tc, linear, t2);
+    const float g = 1.0f - f;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        float x1 = g * t1[k];
-        float x2 = f * t2[k];
-        out[k] = x1 + x2;
-      }
-      return;
+    for (int k = 0; k < 4; ++k) {
+      float x1 = g * out[k];
+      float x2 = f * t2[k];
+      out[k] = x1 + x2;
     }
   }
 }
 
 // ---- resolve ----------------------------------------------------------------
 
-struct TriAttr {
-  float s[3], t[3];
-  float e[3][3];  // homogeneous barycentric rows (bary_rows_of)
+// Perspective-correct barycentrics at one pixel centre from the three
+// homogeneous forms l evaluated there (their sum is 1 / w up to a factor)
+struct BaryPoint {
+  float l[3];
+  float sum;
 };
 
-__device__ __forceinline__ void bary_at(const TriAttr& A, float hw, float hh, float ihw, float ihh,
-                                        float fx, float fy, float* b) {
-  float nx = fx - hw;
-  nx = nx * ihw;
-  float ny = fy - hh;
-  ny = ny * ihh;
-  float l[3];
+__device__ __forceinline__ BaryPoint bary_point(const float* px, const float* py, const float* e2) {
+  BaryPoint b;
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
-    float v = A.e[i][0] * nx;
-    float v2 = A.e[i][1] * ny;
-    v = v + v2;
-    v = v + A.e[i][2];
-    l[i] = v;
+    const float v = px[i] + py[i];
+    b.l[i] = v + e2[i];
   }
-  float S = l[0] + l[1];
-  S = S + l[2];
-  if (S == 0.0f) {
-    b[0] = 1.0f; b[1] = 0.0f; b[2] = 0.0f;
-    return;
-  }
-  float r = 1.0f / S;
-  b[0] = l[0] * r;
-  b[1] = l[1] * r;
-  b[2] = l[2] * r;
+  const float s = b.l[0] + b.l[1];
+  b.sum = s + b.l[2];
+  return b;
 }
+
+// 1 / sum for any sum; a sum of 0 stands for the first vertex
+__device__ __forceinline__ float bary_rcp_any(BaryPoint& b) {
+  if (b.sum == 0.0f) {
+    b.l[0] = 1.0f; b.l[1] = 0.0f; b.l[2] = 0.0f;
+    return 1.0f;
+  }
+  return 1.0f / b.sum;
+}
+
+__device__ __forceinline__ void bary_of(const BaryPoint& b, float r, float* out) {
+  out[0] = b.l[0] * r;
+  out[1] = b.l[1] * r;
+  out[2] = b.l[2] * r;
+}
+
+constexpr float kRcpLo = 0x1p-126f, kRcpHi = 0x1p126f;  // rcp_exact()'s range
 
 __device__ __forceinline__ float interp3(const float* b, float a0, float a1, float a2) {
   float v = b[0] * a0;
@@ -1483,16 +1522,6 @@ __device__ __forceinline__ uint32_t to_unorm8(float c) {
   v = v + 0.5f;
   return (uint32_t)(int)v;
 }
-
-// colour of the visible primitive at a pixel.  A holds the triangle's rows,
-// b the pixel's barycentrics, (s, t) its texture coordinates; q00/q10/q01
-// the texture coordinates at the centres of its 2x2 quad (derivatives for
-// the level of detail) where a quad neighbour already computed them for the
-// same primitive (has_*), else they are evaluated here.
-struct QuadST {
-  float s00, t00, s10, t10, s01, t01;
-  bool h00, h10, h01;
-};
 
 // Phong diffuse term of the scene's lights (no specular) for a shaded
 // material, in world space: per light, intensity = max(0, N.L) * attenuation
@@ -1581,35 +1610,63 @@ __device__ void add_lights(const FrameParams& p, const DrawDesc& d, uint32_t pri
   c[3] = c[3] + dd[3];
 }
 
+// Colour of the visible primitive at pixel (px, py): its record rs, its
+// draw d.  The texture coordinates are evaluated at the pixel and at three
+// centres of its 2x2 quad (the coarse derivatives of the level of detail),
+// with the primitive's own rows: the products of the rows with the quad's
+// two columns and two rows are shared by the four points, and no other
+// pixel's value is needed.
 template <bool kLights>
-__device__ uint32_t shade_pixel(const FrameParams& p, const float* lut, float hw, float hh,
-                               float ihw, float ihh, const TriAttr& A, const float* b, float s,
-                               float t, bool textured, const QuadST& q, const DrawDesc& d,
-                               uint32_t prim, uint32_t scene, int px, int py) {
+__device__ __forceinline__ uint32_t shade_pixel(const FrameParams& p, const ResolveLds& L, float hw,
+                                                float hh, float ihw, float ihh, const ResolveRec& rs,
+                                                const DrawDesc& d, uint32_t prim, uint32_t scene,
+                                                int px, int py) {
   float c[4] = {d.ambient[0], d.ambient[1], d.ambient[2], d.ambient[3]};
   float texc[4] = {1.0f, 1.0f, 1.0f, 1.0f};
   float vc[4] = {1.0f, 1.0f, 1.0f, 1.0f};
-  if (textured) {
-    const TextureDesc* tdp = p.textures + d.texture;
-    const TexHeader td = load_tex_header(tdp);
-    const int qx = px & ~1, qy = py & ~1;
-    float s00 = q.s00, t00 = q.t00, s10 = q.s10, t10 = q.t10, s01 = q.s01, t01 = q.t01;
-    float bq[3];
-    if (!q.h00) {
-      bary_at(A, hw, hh, ihw, ihh, (float)qx + 0.5f, (float)qy + 0.5f, bq);
-      s00 = interp3(bq, A.s[0], A.s[1], A.s[2]);
-      t00 = interp3(bq, A.t[0], A.t[1], A.t[2]);
+  float b[3];
+  const uint32_t cf = (d.flags >> kDrawColorShift) & 3u;
+  const float fx = (float)(px & ~1), fy = (float)(py & ~1);
+  float nx0 = fx + 0.5f; nx0 = nx0 - hw; nx0 = nx0 * ihw;
+  float nx1 = fx + 1.5f; nx1 = nx1 - hw; nx1 = nx1 * ihw;
+  float ny0 = fy + 0.5f; ny0 = ny0 - hh; ny0 = ny0 * ihh;
+  float ny1 = fy + 1.5f; ny1 = ny1 - hh; ny1 = ny1 * ihh;
+  const bool odd_x = px & 1, odd_y = py & 1;
+  float ex0[3], ex1[3], ey0[3], ey1[3], e2[3], exo[3], eyo[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    ex0[i] = rs.e[3 * i] * nx0;
+    ex1[i] = rs.e[3 * i] * nx1;
+    ey0[i] = rs.e[3 * i + 1] * ny0;
+    ey1[i] = rs.e[3 * i + 1] * ny1;
+    e2[i] = rs.e[3 * i + 2];
+    exo[i] = odd_x ? ex1[i] : ex0[i];
+    eyo[i] = odd_y ? ey1[i] : ey0[i];
+  }
+  BaryPoint own = bary_point(exo, eyo, e2);
+  if (!p.no_textures && d.texture > 0) {
+    BaryPoint p00 = bary_point(ex0, ey0, e2), p10 = bary_point(ex1, ey0, e2),
+              p01 = bary_point(ex0, ey1, e2);
+    float r = rcp_exact(own.sum), r00 = rcp_exact(p00.sum), r10 = rcp_exact(p10.sum),
+          r01 = rcp_exact(p01.sum);
+    const float lo = fminf(fminf(fabsf(own.sum), fabsf(p00.sum)), fminf(fabsf(p10.sum), fabsf(p01.sum)));
+    const float hi = fmaxf(fmaxf(fabsf(own.sum), fabsf(p00.sum)), fmaxf(fabsf(p10.sum), fabsf(p01.sum)));
+    if (!(lo >= kRcpLo && hi <= kRcpHi)) {
+      r = bary_rcp_any(own);
+      r00 = bary_rcp_any(p00);
+      r10 = bary_rcp_any(p10);
+      r01 = bary_rcp_any(p01);
     }
-    if (!q.h10) {
-      bary_at(A, hw, hh, ihw, ihh, (float)qx + 1.5f, (float)qy + 0.5f, bq);
-      s10 = interp3(bq, A.s[0], A.s[1], A.s[2]);
-      t10 = interp3(bq, A.t[0], A.t[1], A.t[2]);
-    }
-    if (!q.h01) {
-      bary_at(A, hw, hh, ihw, ihh, (float)qx + 0.5f, (float)qy + 1.5f, bq);
-      s01 = interp3(bq, A.s[0], A.s[1], A.s[2]);
-      t01 = interp3(bq, A.t[0], A.t[1], A.t[2]);
-    }
+    float q[3];
+    bary_of(p00, r00, q);
+    const float s00 = interp3(q, rs.s0, rs.s1, rs.s2), t00 = interp3(q, rs.t0, rs.t1, rs.t2);
+    bary_of(p10, r10, q);
+    const float s10 = interp3(q, rs.s0, rs.s1, rs.s2), t10 = interp3(q, rs.t0, rs.t1, rs.t2);
+    bary_of(p01, r01, q);
+    const float s01 = interp3(q, rs.s0, rs.s1, rs.s2), t01 = interp3(q, rs.t0, rs.t1, rs.t2);
+    bary_of(own, r, b);
+    const float s = interp3(b, rs.s0, rs.s1, rs.s2), t = interp3(b, rs.t0, rs.t1, rs.t2);
+    const TexHeader td = load_tex_header(p, L, (uint32_t)d.texture);
     const float fw = (float)td.width, fh = (float)td.height;
     float dux = s10 - s00; dux = dux * fw;
     float dvx = t10 - t00; dvx = dvx * fh;
@@ -1620,15 +1677,13 @@ __device__ uint32_t shade_pixel(const FrameParams& p, const float* lut, float hw
     const float r2 = rx > ry ? rx : ry;
     float lambda = gbr_log2(r2);
     lambda = lambda * 0.5f;
-    float tc[4];
-    sample_tex(p, lut, tdp, td, (int)d.layer, s, t, lambda, tc);
+    sample_tex(p, L, (uint32_t)d.texture, td, (int)d.layer, s, t, lambda, texc);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      texc[k] = tc[k];
-      c[k] = c[k] * tc[k];
-    }
+    for (int k = 0; k < 4; ++k) c[k] = c[k] * texc[k];
+  } else if (cf != kColorNone || kLights) {
+    const float r = bary_rcp_any(own);
+    bary_of(own, r, b);
   }
-  const uint32_t cf = (d.flags >> kDrawColorShift) & 3u;
   if (cf != kColorNone) {
     const uint32_t* ip = p.indices + d.index_base + 3 * (prim - d.prim_base);
     float col[3][4];
@@ -1636,11 +1691,7 @@ __device__ uint32_t shade_pixel(const FrameParams& p, const float* lut, float hw
     for (int k = 0; k < 3; ++k) {
       const uint32_t v = ip[k];
       if (cf == kColorU8) {
-        const uint32_t u8 = p.col8[v];
-        col[k][0] = lut[u8 & 0xff];
-        col[k][1] = lut[(u8 >> 8) & 0xff];
-        col[k][2] = lut[(u8 >> 16) & 0xff];
-        col[k][3] = lut[u8 >> 24];
+        unpack_texel(L.lut, p.col8[v], col[k]);
       } else {
         const float4 f = p.col32[v];
         col[k][0] = f.x; col[k][1] = f.y; col[k][2] = f.z; col[k][3] = f.w;
@@ -2118,28 +2169,15 @@ __device__ void bin_hiz(const FrameParams& p, const BinInfo& b, const unsigned l
 // resolves in place, resolves them from their phase-1 keys).
 // --------------------------------------------------------------------------
 
-// a range of the queue: its first bin, heavy bins, entries, and the number
-// of workgroups whose first bin it gives
-struct RasterRange {
-  uint32_t first, heavy, total, fixed;
-};
-
 struct RasterLds {
   unsigned long long vis[kMaxBin * kMaxBin];
   BigTri big[kBigQueue];
-  float lut[256];  // unorm8 -> float, for resolving in place
   int nbig[2];     // queue fill of even / odd batches
-  uint32_t next;   // the bin to rasterise next (kNoBin: none)
-  RasterRange ranges[kRasterParts];  // the queue's ranges, this workgroup's own first
 };
-
-// A raster queue entry: the bin, with kRestBin set when it comes from the
-// range's bins in order (it may then be a heavy bin, taken from that list).
-constexpr uint32_t kNoBin = ~0u, kRestBin = 0x80000000u;
 
 template <bool kLights>
 __device__ void resolve_tile(const FrameParams& p, const RasterItem& it,
-                             const unsigned long long* tile, int B, const float* s_lut);
+                             const unsigned long long* tile, int B, const ResolveLds& R);
 
 // the raster phase after which no pass changes the keys
 __host__ __device__ __forceinline__ bool final_phase(const FrameParams& p, int phase) {
@@ -2154,7 +2192,7 @@ __host__ __device__ __forceinline__ bool resolves_in_place(const FrameParams& p,
 // kResolve: the phase resolves its bins in place (resolves_in_place)
 template <bool kResolve>
 __device__ void raster_bin(const FrameParams& p, const RasterItem& item, int phase, RasterLds& L,
-                           uint32_t& pairs, uint32_t& frags) {
+                           const ResolveLds* R, uint32_t& pairs, uint32_t& frags) {
   const int tid = local_tid();
   const BinInfo b = bin_info(item);
   const uint32_t* entries = p.bin_entries + b.entries;
@@ -2229,7 +2267,7 @@ __device__ void raster_bin(const FrameParams& p, const RasterItem& item, int pha
     __syncthreads();
   }
   if (kResolve) {
-    resolve_tile<false>(p, item, L.vis, B, L.lut);
+    resolve_tile<false>(p, item, L.vis, B, *R);
   } else {
     store_vis(p, b, L.vis, B);
     if (phase == 1 && p.hiz_fused) bin_hiz(p, b, L.vis);
@@ -2252,8 +2290,12 @@ __global__ __launch_bounds__(kBlock, kWaves) void k_raster_lane(FrameParams p,
   // phase 1 visits every bin (each gets its keys and pyramid); phase 2 only
   // the bins that received entries, unless it resolves (then every bin)
   const bool active_only = phase == 2 && !kResolve;
-  static_assert(kBlock == 256, "one LUT entry per thread");
-  if (kResolve) L.lut[threadIdx.x] = p.unorm_lut[threadIdx.x];
+  ResolveLds* R = nullptr;
+  if constexpr (kResolve) {
+    __shared__ ResolveLds s_resolve;
+    R = &s_resolve;
+    resolve_lds_fill(p, s_resolve);
+  }
   uint32_t pairs = 0, frags = 0;
   // thread 0's position in the queue ranges: its own XCD's range first
   // (workgroups are dispatched to the XCDs round robin), then the next ones
@@ -2292,7 +2334,7 @@ __global__ __launch_bounds__(kBlock, kWaves) void k_raster_lane(FrameParams p,
     __syncthreads();  // s_claim is rewritten by the next claim; the LDS tile is free
     if (claim == ~0u) break;
     if (claim & 0x80000000u) continue;
-    raster_bin<kResolve>(p, items[claim], phase, L, pairs, frags);
+    raster_bin<kResolve>(p, items[claim], phase, L, R, pairs, frags);
   }
   add_raster_stats(p, pairs, frags);
 }
@@ -2419,12 +2461,12 @@ __global__ __launch_bounds__(kBlock) void k_raster_full(FrameParams p,
   __shared__ BigTri s_big[kBigQueue];
   __shared__ uint32_t s_base[kDrawCache];
   __shared__ int s_nbig;
-  __shared__ float s_lut[256];
+  __shared__ ResolveLds s_resolve;
 
   const uint32_t n_over =
       min(p.counters[(phase == 2 ? kCtrOverflow2 : kCtrOverflow1) * kCtrStride], n);
   if (blockIdx.x >= n_over) return;  // (whole workgroup)
-  if (p.fuse_resolve) s_lut[threadIdx.x] = p.unorm_lut[threadIdx.x];  // (kBlock == 256)
+  if (p.fuse_resolve) resolve_lds_fill(p, s_resolve);
   __syncthreads();
   const int B = p.bin_size;
   uint32_t pairs = 0, frags = 0;
@@ -2459,7 +2501,7 @@ __global__ __launch_bounds__(kBlock) void k_raster_full(FrameParams p,
       __syncthreads();
     }
     if (resolves_in_place(p, phase)) {
-      resolve_tile<false>(p, it, s_vis, B, s_lut);
+      resolve_tile<false>(p, it, s_vis, B, s_resolve);
     } else {
       store_vis(p, b, s_vis, B);
       if (phase == 1 && p.hiz_fused) bin_hiz(p, b, s_vis);
@@ -2479,13 +2521,13 @@ __global__ __launch_bounds__(kBlock) void k_raster_full(FrameParams p,
 // --------------------------------------------------------------------------
 
 // The outputs of one bin from its final visibility keys: `tile` holds them
-// in rows of B keys (an LDS tile), s_lut the unorm8 -> float table.  Called
+// in rows of B keys (an LDS tile), R the resolve's tables.  Called
 // by every thread of the workgroup.  kLights: the renderer has lights
 // enabled (a separate instance, so that renderers without lights keep the
 // smaller register footprint).
 template <bool kLights>
 __device__ void resolve_tile(const FrameParams& p, const RasterItem& it,
-                             const unsigned long long* tile, int B, const float* s_lut) {
+                             const unsigned long long* tile, int B, const ResolveLds& R) {
   const int tid = local_tid();
   const BinInfo b = bin_info(it);
   const uint32_t frame = *p.frame;
@@ -2493,10 +2535,6 @@ __device__ void resolve_tile(const FrameParams& p, const RasterItem& it,
   const float far_depth = un1 / (1.0f + un0);
   const int bw = b.bin.x1 - b.bin.x0 + 1, bh = b.bin.y1 - b.bin.y0 + 1;
   const int npx = bw * bh;
-  // in a full bin the pixels of a 2x2 quad sit in lanes {l, l^1, l^bw, l^1^bw}
-  // of one wave (rows of bw pixels, bw in {8, 16, 32}, even bin origin)
-  const bool quads = bw == p.bin_size && bh == p.bin_size;
-  const int lane = tid & 63;
   const float hw = (float)b.width * 0.5f, hh = (float)b.height * 0.5f;
   const float ihw = 1.0f / hw, ihh = 1.0f / hh;
   const float inv_bw = 1.0f / (float)bw;
@@ -2505,73 +2543,46 @@ __device__ void resolve_tile(const FrameParams& p, const RasterItem& it,
   const bool want_depth = p.out_depth && (b.planes & GBR_PLANE_DEPTH);
   const bool want_lin = p.out_lindepth && (b.planes & GBR_PLANE_LINEAR_DEPTH);
   const bool want_sem = p.out_semantic && (b.planes & GBR_PLANE_SEMANTIC);
-  for (int base = 0; base < npx; base += kBlock) {
-    const int l = base + tid;
-    const bool valid = l < npx;
+  for (int l = tid; l < npx; l += kBlock) {
     const int ly = div_small(l, inv_bw), lx = l - ly * bw;
     const int px = b.bin.x0 + lx, py = b.bin.y0 + ly;
-    const unsigned long long key = valid ? tile[ly * B + lx] : kClearKey;
-    const bool drawn = key != kClearKey;
-    const uint32_t prim = (uint32_t)key;
-    ResolveRec rs;
-    DrawDesc d;
-    TriAttr A;
-    float bc[3] = {1.0f, 0.0f, 0.0f};
-    float s = 0.0f, t = 0.0f;
-    bool textured = false;
-    if (drawn) {
-      rs = p.srecs[(size_t)b.rec_base + prim];
-      // every drawn primitive's record was written this frame; the clamp
-      // only keeps the lookups in bounds
-      const uint32_t item = min(rs.item, p.n_items - 1u);
-      d = p.item_draws[item];
-      if (p.item_vis) p.item_vis[item] = frame;  // visibility feedback for the next frame
-#pragma unroll
-      for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int k = 0; k < 3; ++k) A.e[i][k] = rs.e[3 * i + k];
-      A.s[0] = rs.s0; A.t[0] = rs.t0;
-      A.s[1] = rs.s1; A.t[1] = rs.t1;
-      A.s[2] = rs.s2; A.t[2] = rs.t2;
-      bary_at(A, hw, hh, ihw, ihh, (float)px + 0.5f, (float)py + 0.5f, bc);
-      textured = !p.no_textures && d.texture > 0;
-      if (textured) {
-        s = interp3(bc, A.s[0], A.s[1], A.s[2]);
-        t = interp3(bc, A.t[0], A.t[1], A.t[2]);
-      }
-    }
-    QuadST q = {};
-    if (quads) {
-      const uint32_t tag = textured ? prim : 0xffffffffu;
-      const int l00 = lane & ~1 & ~bw, l10 = (lane | 1) & ~bw, l01 = (lane & ~1) | bw;
-      const uint32_t g00 = __shfl(tag, l00), g10 = __shfl(tag, l10), g01 = __shfl(tag, l01);
-      q.s00 = __shfl(s, l00); q.t00 = __shfl(t, l00);
-      q.s10 = __shfl(s, l10); q.t10 = __shfl(t, l10);
-      q.s01 = __shfl(s, l01); q.t01 = __shfl(t, l01);
-      q.h00 = textured && g00 == prim;
-      q.h10 = textured && g10 == prim;
-      q.h01 = textured && g01 == prim;
-    }
-    if (!valid) continue;
+    const unsigned long long key = tile[ly * B + lx];
     const int row = p.top_down ? (b.height - 1 - py) : py;
     const size_t o = (size_t)b.plane_offset + (size_t)row * b.stride + px;
-    if (!drawn) {
+    if (key == kClearKey) {
       if (want_color) p.out_color[o] = kClearColor;
       if (want_depth) p.out_depth[o] = 1.0f;
       if (want_lin) p.out_lindepth[o] = 0.0f;
       if (want_sem) p.out_semantic[o] = 0u;
       continue;
     }
+    const uint32_t prim = (uint32_t)key;
+    const ResolveRec* rec = p.srecs + (size_t)b.rec_base + prim;
+    // the whole record, or (no colour wanted) its work item alone
+    ResolveRec rs;
+    if (want_color) rs = *rec;
+    else rs.item = rec->item;
+    // every drawn primitive's record was written this frame; the clamp
+    // only keeps the lookups in bounds
+    const uint32_t item = min(rs.item, p.n_items - 1u);
+    const DrawDesc& d = p.item_draws[item];
+    // visibility feedback for the next frame, once per run of pixels (the
+    // lane before has the same item, or is in another row of 16, or idle)
+    if (p.item_vis && __builtin_amdgcn_update_dpp((int)~item, (int)item, 0x111, 0xF, 0xF, false) != (int)item)
+      p.item_vis[item] = frame;
     const float z = __uint_as_float((uint32_t)(key >> 32));
-    if (want_color)
-      p.out_color[o] = shade_pixel<kLights>(p, s_lut, hw, hh, ihw, ihh, A, bc, s, t, textured, q, d, prim,
-                                            it.scene, px, py);
     if (want_depth) p.out_depth[o] = z;
     if (want_lin) {
-      const float lin = un1 / (z + un0);
+      const float den = z + un0;
+      float lin = div_exact(un1, den, rcp_exact(den));
+      if (!(in_range(den, 0x1p-60f, 0x1p60f) && in_range(un1, 0x1p-60f, 0x1p60f) &&
+            in_range(lin, 0x1p-60f, 0x1p60f)))
+        lin = un1 / den;
       p.out_lindepth[o] = lin == far_depth ? 0.0f : lin;
     }
     if (want_sem) p.out_semantic[o] = d.semantic;
+    if (want_color)
+      p.out_color[o] = shade_pixel<kLights>(p, R, hw, hh, ihw, ihh, rs, d, prim, it.scene, px, py);
   }
 }
 
@@ -2581,14 +2592,13 @@ __device__ void resolve_tile(const FrameParams& p, const RasterItem& it,
 template <bool kLights>
 __global__ __launch_bounds__(kBlock) void k_resolve(FrameParams p,
                                                     const RasterItem* __restrict__ items) {
-  __shared__ float s_lut[256];
+  __shared__ ResolveLds s_resolve;
   __shared__ unsigned long long s_tile[kMaxBin * kMaxBin];
-  static_assert(kBlock >= 256, "one LUT entry per thread");
-  if (threadIdx.x < 256) s_lut[threadIdx.x] = p.unorm_lut[threadIdx.x];
+  resolve_lds_fill(p, s_resolve);
   const RasterItem it = items[blockIdx.x];
   load_vis(p, bin_info(it), s_tile, p.bin_size);
   __syncthreads();
-  resolve_tile<kLights>(p, it, s_tile, p.bin_size, s_lut);
+  resolve_tile<kLights>(p, it, s_tile, p.bin_size, s_resolve);
 }
 
 // --------------------------------------------------------------------------

@@ -314,6 +314,37 @@ std::vector<std::vector<uint8_t>> generate_mips(const uint8_t* level0, int w, in
   return out;
 }
 
+// the device form of a texture's GL filters and wrap modes (GL enums; its
+// size is set already)
+void set_sampler(TextureDesc& td, uint32_t min_filter, uint32_t mag_filter, uint32_t wrap_s,
+                 uint32_t wrap_t) {
+  constexpr uint32_t kLinear = 9729, kNearest = 9728, kNearestMipNearest = 9984,
+                     kLinearMipNearest = 9985, kNearestMipLinear = 9986, kLinearMipLinear = 9987;
+  constexpr uint32_t kClamp = 33071, kMirror = 33648;
+  td.filter = 0;
+  if (mag_filter == kLinear) td.filter |= kTexMagLinear;
+  if (min_filter == kLinear || min_filter == kLinearMipNearest || min_filter == kLinearMipLinear)
+    td.filter |= kTexMinLinear;
+  if (min_filter == kNearest || min_filter == kLinear) td.filter |= kTexMipNone;
+  if (min_filter == kNearestMipNearest || min_filter == kLinearMipNearest)
+    td.filter |= kTexMipNearest;
+  if (mag_filter == kLinear &&
+      (min_filter == kNearestMipNearest || min_filter == kNearestMipLinear))
+    td.filter |= kTexMagHalf;
+  auto axis = [&](uint32_t mode, int32_t size, int32_t& wrap_or) {
+    wrap_or = mode == kClamp ? -1 : 0;
+    if (mode != kClamp && (mode == kMirror || (size & (size - 1)) != 0)) td.filter |= kTexWrapSlow;
+  };
+  axis(wrap_s, td.width, td.wrap_or_s);
+  axis(wrap_t, td.height, td.wrap_or_t);
+  td.wraps = (wrap_s & 0xffffu) | (wrap_t << 16);
+}
+
+void set_level(TextureDesc& td, int level, size_t offset) {
+  td.level[level].offset = (int64_t)offset;
+  td.level[level].texels = (uint32_t)std::max(td.width >> level, 1) * (uint32_t)std::max(td.height >> level, 1);
+}
+
 uint32_t batch_id(Scene& sc, uint32_t vcolor, uint32_t mesh, uint32_t tex) {
   for (size_t i = 0; i < sc.batches.size(); ++i)
     if (sc.batches[i].vcolor == vcolor && sc.batches[i].mesh == mesh && sc.batches[i].texture == tex)
@@ -380,6 +411,7 @@ gbr_status upload_assets(gbr_renderer* r) {
   TRY(upload(r->d_col32, r->col32, s));
   if (r->cfg.max_light_count) TRY(upload(r->d_nrm, r->nrm, s));
   TRY(upload(r->d_indices, r->indices, s));
+  TRY(r->d_texels.reserve(r->texels.size() + sizeof(uint32_t)));  // (a texel pair's second half)
   TRY(upload(r->d_texels, r->texels, s));
   TRY(upload(r->d_textures, r->textures, s));
   TRY(upload(r->d_materials, r->materials, s));
@@ -771,6 +803,7 @@ gbr_status do_draw(gbr_renderer* r) {
   p.indices = r->d_indices.ptr;
   p.materials = r->d_materials.ptr;
   p.textures = r->d_textures.ptr;
+  p.n_textures = (uint32_t)r->textures.size();
   p.texels = r->d_texels.ptr;
   p.unorm_lut = r->d_lut.ptr;
   p.draws = r->d_draws.ptr;
@@ -1154,10 +1187,8 @@ gbr_status gbr_create(const gbr_config* config, gbr_renderer** out) {
   // texture 0 = white pixel, material 0 = white ambient (Renderer.cpp:287-304)
   TextureDesc white{};
   white.width = white.height = white.layers = white.levels = 1;
-  white.min_filter = 9728;
-  white.mag_filter = 9728;
-  white.wrap_s = white.wrap_t = 10497;
-  white.level_offset[0] = 0;
+  set_sampler(white, 9728, 9728, 10497, 10497);
+  set_level(white, 0, 0);
   r->textures.push_back(white);
   r->texels.insert(r->texels.end(), {255, 255, 255, 255});
   MaterialDesc m0{};
@@ -1292,17 +1323,14 @@ gbr_status gbr_add_file_data(gbr_renderer* r, const gbr_file_desc* f, uint32_t f
       td.width = (int)t.width;
       td.height = (int)t.height;
       td.layers = (int)t.layers;
-      td.min_filter = (int)t.min_filter;
-      td.mag_filter = (int)t.mag_filter;
-      td.wrap_s = (int)t.wrap_s;
-      td.wrap_t = (int)t.wrap_t;
+      set_sampler(td, t.min_filter, t.mag_filter, t.wrap_s, t.wrap_t);
       const bool gen = t.levels == 1 && (flags & GBR_FILE_GENERATE_MIPMAP) && !t.compressed;
       if (gen) {
         int nl = 1;
         auto lv = generate_mips(t.texels, td.width, td.height, td.layers, nl);
         td.levels = nl;
         for (int l = 0; l < nl; ++l) {
-          td.level_offset[l] = (int64_t)r->texels.size();
+          set_level(td, l, r->texels.size());
           r->texels.insert(r->texels.end(), lv[l].begin(), lv[l].end());
         }
       } else {
@@ -1310,7 +1338,7 @@ gbr_status gbr_add_file_data(gbr_renderer* r, const gbr_file_desc* f, uint32_t f
         size_t off = 0;
         for (int l = 0; l < td.levels; ++l) {
           const size_t sz = (size_t)std::max(td.width >> l, 1) * std::max(td.height >> l, 1) * td.layers * 4;
-          td.level_offset[l] = (int64_t)r->texels.size();
+          set_level(td, l, r->texels.size());
           r->texels.insert(r->texels.end(), t.texels + off, t.texels + off + sz);
           off += sz;
         }
