@@ -311,6 +311,19 @@ __device__ __forceinline__ unsigned long long block_sum(unsigned long long v,
   return t;
 }
 
+// The frame parameters (a kernel's first argument) read from the argument
+// segment again: the persistent kernels use some forty of its fields, and
+// fields loaded before their loops stay in scalar registers, which overflow
+// into vector lanes (a v_readlane for each use: 245 of the 2155 vector
+// instructions of k_setup_bin).  Through a pointer the compiler cannot see
+// through, each loop iteration loads what it uses by scalar loads.
+__device__ __forceinline__ const FrameParams& params_again() {
+  typedef const __attribute__((address_space(4))) FrameParams* Segment;
+  Segment k = (Segment)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(k));
+  return *(const FrameParams*)k;
+}
+
 // --------------------------------------------------------------------------
 // k_nodes: absolute node transforms
 // --------------------------------------------------------------------------
@@ -672,7 +685,7 @@ __device__ __forceinline__ void note_heavy(const FrameParams& p, uint32_t gbin, 
 
 // at least 5 waves per SIMD (96 VGPRs): one register more costs a fifth
 // of the resident waves and ~15% of the setup time
-__global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams p,
+__global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams params,
                                                       const uint32_t* __restrict__ list,
                                                       uint32_t list_ctr, uint32_t queue_ctr) {
   __shared__ int32_t s_x[kVertexCache];
@@ -684,10 +697,10 @@ __global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams p,
   __shared__ float s_cw[kVertexCache];
   __shared__ float s_s[kVertexCache];
   __shared__ float s_t[kVertexCache];
-  // per-bin counters and bases: 2 * p.lds_bins words of dynamic LDS
+  // per-bin counters and bases: 2 * params.lds_bins words of dynamic LDS
   extern __shared__ uint32_t s_bins[];
   uint32_t* const s_bcount = s_bins;
-  uint32_t* const s_bbase = s_bins + p.lds_bins;
+  uint32_t* const s_bbase = s_bins + params.lds_bins;
   __shared__ uint32_t s_pair[kPairCap];  // bin << 21 | local slot << 10 | triangle in chunk
   __shared__ uint32_t s_npairs;
   __shared__ uint32_t s_item;
@@ -698,9 +711,9 @@ __global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams p,
   unsigned long long tri_acc = 0, vtx_acc = 0;  // triangles / vertices set up (uniform)
   uint32_t grab = 0, grab_end = 0;  // items claimed from the queue (uniform)
   const int phase = queue_ctr == kCtrQueue2 ? 2 : 1;
-  const bool hiz_test = phase == 2 && p.hiz != nullptr;
+  const bool hiz_test = phase == 2 && params.hiz != nullptr;
   // the whole frame, or the work items listed for this phase
-  const uint32_t n_items = list ? min(p.counters[list_ctr * kCtrStride], p.n_items) : p.n_items;
+  const uint32_t n_items = list ? min(params.counters[list_ctr * kCtrStride], params.n_items) : params.n_items;
 
   bool have_pre = false;
   uint32_t pre_item = 0;
@@ -708,7 +721,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams p,
   // items per claim: queue_grain, down to 1 when there are fewer than 8
   // claims' worth per workgroup (a short list balances better item by item)
   const uint32_t grain =
-      max(1u, min((uint32_t)p.queue_grain, n_items / (gridDim.x * 8u)));
+      max(1u, min((uint32_t)params.queue_grain, n_items / (gridDim.x * 8u)));
   // this workgroup's stripe of the list and its claim counter (every stripe
   // has workgroups: a grid smaller than kQueueStripes uses fewer stripes)
   const uint32_t nstripes = min(kQueueStripes, gridDim.x);
@@ -716,7 +729,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams p,
   const uint32_t s_begin = (uint32_t)((unsigned long long)n_items * stripe / nstripes);
   const uint32_t s_end = (uint32_t)((unsigned long long)n_items * (stripe + 1) / nstripes);
   uint32_t* const claim_ctr =
-      &p.counters[(kCtrStripes + (queue_ctr == kCtrQueue2 ? kQueueStripes : 0u) + stripe) * kCtrStride];
+      &params.counters[(kCtrStripes + (queue_ctr == kCtrQueue2 ? kQueueStripes : 0u) + stripe) * kCtrStride];
   // thread 0 claims the next chunk one chunk ahead, so the claim's round
   // trip overlaps the current chunk (the last, unused claim only moves the
   // counter past the end)
@@ -734,6 +747,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams p,
       __syncthreads();  // s_item may be rewritten only after everyone read it
       if (grab >= s_end) break;
     }
+    const FrameParams& p = params_again();
     uint32_t item;
     WorkItem wi;
     if (have_pre) {  // fetched during the previous item
@@ -928,10 +942,10 @@ __global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams p,
   const unsigned long long wsum = block_sum(written, s_red);
   if (threadIdx.x == 0) {
     const uint32_t st = queue_ctr == kCtrQueue2 ? 4u : 2u;
-    if (wsum) add_stat(p.stats, 0, wsum);
+    if (wsum) add_stat(params.stats, 0, wsum);
     if (tri_acc) {
-      add_stat(p.stats, st, tri_acc);
-      add_stat(p.stats, st + 1, vtx_acc);
+      add_stat(params.stats, st, tri_acc);
+      add_stat(params.stats, st + 1, vtx_acc);
     }
   }
 }
@@ -1045,7 +1059,7 @@ __device__ __forceinline__ float uniform(float v) {
 // the functions are linear); lanes 0-15 test the bin's at most 16 blocks at
 // once.  A block step is then three additions (block offset, a scalar, plus
 // the lane's own offset), the depth and the LDS atomicMin.
-__device__ void raster_big_waves(const RasterCtx& rc, const BigTri* big, int nb) {
+__device__ __forceinline__ void raster_big_waves(const RasterCtx& rc, const BigTri* big, int nb) {
   const int tid = local_tid();
   const int lane = tid & 63;
   const int lx = lane & 7, ly = lane >> 3;          // pixel in a block
@@ -1091,7 +1105,7 @@ __device__ void raster_big_waves(const RasterCtx& rc, const BigTri* big, int nb)
 // a known depth plane row by row, edge functions stepped by additions.  The
 // depth plane's pixel offsets are integers below 2^24, so stepping them by
 // 256 as floats is exact.
-__device__ void raster_walk(const RasterCtx& rc, const int32_t* X, const int32_t* Y, float z0,
+__device__ __forceinline__ void raster_walk(const RasterCtx& rc, const int32_t* X, const int32_t* Y, float z0,
                             float dzdx, float dzdy, float zlo, uint32_t prim, const PixRect& r) {
   int32_t dx[3], dy[3], er[3];
   const int32_t Px0 = (r.x0 << 8) | 128, Py0 = (r.y0 << 8) | 128;
@@ -1324,21 +1338,31 @@ struct TexHeader {
 
 __device__ __forceinline__ TexHeader load_tex_header(const FrameParams& p, const ResolveLds& L,
                                                      uint32_t texture) {
-  int4 a, b;
+  // (the words from memory pass through an empty asm: the compiler would
+  // else merge the two places' loads into flat ones)
+  typedef int Words __attribute__((ext_vector_type(4)));
+  Words a, b;
   if (__builtin_expect(texture < kLdsTextures, 1)) {
-    a = reinterpret_cast<const int4*>(&L.tex[texture])[0];
-    b = reinterpret_cast<const int4*>(&L.tex[texture])[1];
+    a = reinterpret_cast<const Words*>(&L.tex[texture])[0];
+    b = reinterpret_cast<const Words*>(&L.tex[texture])[1];
   } else {
-    a = reinterpret_cast<const int4*>(p.textures + texture)[0];
-    b = reinterpret_cast<const int4*>(p.textures + texture)[1];
+    a = reinterpret_cast<const Words*>(p.textures + texture)[0];
+    b = reinterpret_cast<const Words*>(p.textures + texture)[1];
+    asm volatile("" : "+v"(a), "+v"(b));
   }
   return TexHeader{a.x, a.y, a.z, a.w, (uint32_t)b.x, b.y, b.z, (uint32_t)b.w};
 }
 
 __device__ __forceinline__ TexLevel load_tex_level(const FrameParams& p, const ResolveLds& L,
                                                    uint32_t texture, int level) {
-  if (__builtin_expect(texture < kLdsTextures, 1)) return L.tex[texture].level[level];
-  return p.textures[texture].level[level];
+  TexLevel v;
+  if (__builtin_expect(texture < kLdsTextures, 1)) {
+    v = L.tex[texture].level[level];
+  } else {
+    v = p.textures[texture].level[level];
+    asm volatile("" : "+v"(v.offset), "+v"(v.texels));
+  }
+  return v;
 }
 
 // texel `row + i` of a level whose first byte is `base`: row = (layer * h
@@ -2120,7 +2144,7 @@ __device__ __forceinline__ uint32_t lane_move(uint32_t v) {
 // phase-1 keys in LDS: max depth per level-0 block (2^kHiZ0 pixels square)
 // and over the bin (level 1), the same values k_hiz computes from the
 // stored keys.
-__device__ void bin_hiz(const FrameParams& p, const BinInfo& b, const unsigned long long* s_vis) {
+__device__ __forceinline__ void bin_hiz(const FrameParams& p, const BinInfo& b, const unsigned long long* s_vis) {
   const int tid = local_tid();
   constexpr int kN = kHiZPer * kHiZPer;
   static_assert(kHiZ0 == 3 && kBlock / kMaxBin == 8, "a pass covers one row of blocks");
@@ -2176,7 +2200,7 @@ struct RasterLds {
 };
 
 template <bool kLights>
-__device__ void resolve_tile(const FrameParams& p, const RasterItem& it,
+__device__ __forceinline__ void resolve_tile(const FrameParams& p, const RasterItem& it,
                              const unsigned long long* tile, int B, const ResolveLds& R);
 
 // the raster phase after which no pass changes the keys
@@ -2191,7 +2215,7 @@ __host__ __device__ __forceinline__ bool resolves_in_place(const FrameParams& p,
 
 // kResolve: the phase resolves its bins in place (resolves_in_place)
 template <bool kResolve>
-__device__ void raster_bin(const FrameParams& p, const RasterItem& item, int phase, RasterLds& L,
+__device__ __forceinline__ void raster_bin(const FrameParams& p, const RasterItem& item, int phase, RasterLds& L,
                            const ResolveLds* R, uint32_t& pairs, uint32_t& frags) {
   const int tid = local_tid();
   const BinInfo b = bin_info(item);
@@ -2282,7 +2306,7 @@ __device__ void raster_bin(const FrameParams& p, const RasterItem& item, int pha
 // resolve 5 (96 VGPRs, 4 spilled; 183 -> 173 us after the depth pyramid
 // against 4 without spills).
 template <bool kResolve, int kWaves>
-__global__ __launch_bounds__(kBlock, kWaves) void k_raster_lane(FrameParams p,
+__global__ __launch_bounds__(kBlock, kWaves) void k_raster_lane(FrameParams params,
                                                         const RasterItem* __restrict__ items,
                                                         uint32_t n_ritems, int phase) {
   __shared__ RasterLds L;
@@ -2294,7 +2318,7 @@ __global__ __launch_bounds__(kBlock, kWaves) void k_raster_lane(FrameParams p,
   if constexpr (kResolve) {
     __shared__ ResolveLds s_resolve;
     R = &s_resolve;
-    resolve_lds_fill(p, s_resolve);
+    resolve_lds_fill(params, s_resolve);
   }
   uint32_t pairs = 0, frags = 0;
   // thread 0's position in the queue ranges: its own XCD's range first
@@ -2302,6 +2326,7 @@ __global__ __launch_bounds__(kBlock, kWaves) void k_raster_lane(FrameParams p,
   const uint32_t home = blockIdx.x % kRasterParts;
   uint32_t tried = 0;
   for (;;) {
+    const FrameParams& p = params_again();
     if (threadIdx.x == 0) {
       uint32_t claim = ~0u;  // every range is drained
       for (; tried < kRasterParts; ++tried) {
@@ -2336,7 +2361,7 @@ __global__ __launch_bounds__(kBlock, kWaves) void k_raster_lane(FrameParams p,
     if (claim & 0x80000000u) continue;
     raster_bin<kResolve>(p, items[claim], phase, L, R, pairs, frags);
   }
-  add_raster_stats(p, pairs, frags);
+  add_raster_stats(params, pairs, frags);
 }
 
 // --------------------------------------------------------------------------
@@ -2526,7 +2551,7 @@ __global__ __launch_bounds__(kBlock) void k_raster_full(FrameParams p,
 // enabled (a separate instance, so that renderers without lights keep the
 // smaller register footprint).
 template <bool kLights>
-__device__ void resolve_tile(const FrameParams& p, const RasterItem& it,
+__device__ __forceinline__ void resolve_tile(const FrameParams& p, const RasterItem& it,
                              const unsigned long long* tile, int B, const ResolveLds& R) {
   const int tid = local_tid();
   const BinInfo b = bin_info(it);
