@@ -65,6 +65,8 @@ struct alignas(16) SceneDesc {
   unsigned long long rec_base;    // first primitive record of this scene
   int32_t stride;                 // row stride of the scene's planes (the tile width)
   uint32_t planes;                // GBR_PLANE_* written for this scene
+  float guard_x, guard_y;         // kGuardPx over half the viewport's width and height
+  uint32_t pad[2];
 };
 
 // One chunk of <= kChunkTris consecutive triangles of a draw; everything a

@@ -172,7 +172,9 @@ __device__ __forceinline__ float plane_dist(float4 v, int plane, float gx, float
 
 __device__ __forceinline__ void project(float4 v, float hw, float hh, int32_t& X, int32_t& Y,
                                         float& Z) {
-  float iw = 1.0f / v.w;
+  // (w > 0: the vertex is inside the clip volume)
+  float iw = rcp_exact(v.w);
+  if (!(v.w >= 0x1p-126f && v.w <= 0x1p126f)) iw = 1.0f / v.w;
   float nx = v.x * iw, ny = v.y * iw, nz = v.z * iw;
   float xw = nx * hw;
   xw = xw + hw;
@@ -622,6 +624,17 @@ __device__ __forceinline__ T uniform_load(const T* ptr, uint32_t i) {
   return out;
 }
 
+// AND of v over the wave, in every lane's scalar view (lane moves within
+// rows of 16, then the four rows)
+__device__ __forceinline__ uint32_t wave_and(uint32_t v) {
+  v &= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true);   // lane ^ 1
+  v &= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true);   // lane ^ 2
+  v &= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, true);  // half mirror: 8 lanes
+  v &= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x140, 0xF, 0xF, true);  // mirror: 16 lanes
+  return (uint32_t)(__builtin_amdgcn_readlane((int)v, 0) & __builtin_amdgcn_readlane((int)v, 16) &
+                    __builtin_amdgcn_readlane((int)v, 32) & __builtin_amdgcn_readlane((int)v, 48));
+}
+
 __device__ __forceinline__ void append_ref(const FrameParams& p, uint32_t counter, bool flag,
                                            PrimRef ref, const ClipFast& fast, int lane,
                                            unsigned long long lt_mask) {
@@ -685,6 +698,7 @@ __device__ __forceinline__ void note_heavy(const FrameParams& p, uint32_t gbin, 
 
 // at least 5 waves per SIMD (96 VGPRs): one register more costs a fifth
 // of the resident waves and ~15% of the setup time
+template <bool kAll>
 __global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams params,
                                                       const uint32_t* __restrict__ list,
                                                       uint32_t list_ctr, uint32_t queue_ctr) {
@@ -704,6 +718,8 @@ __global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams params,
   __shared__ uint32_t s_pair[kPairCap];  // bin << 21 | local slot << 10 | triangle in chunk
   __shared__ uint32_t s_npairs;
   __shared__ uint32_t s_item;
+  __shared__ uint4 s_out[2];  // per wave, the planes every vertex of the item is outside of
+  static_assert(kBlock == 256, "four waves");
 
   const int lane = threadIdx.x & 63;
   const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
@@ -713,9 +729,11 @@ __global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams params,
   const int phase = queue_ctr == kCtrQueue2 ? 2 : 1;
   const bool hiz_test = phase == 2 && params.hiz != nullptr;
   // the whole frame, or the work items listed for this phase
-  const uint32_t n_items = list ? min(params.counters[list_ctr * kCtrStride], params.n_items) : params.n_items;
+  const uint32_t n_items =
+      kAll ? params.n_items : min(params.counters[list_ctr * kCtrStride], params.n_items);
 
   bool have_pre = false;
+  int parity = 0;  // of the items, for s_out
   uint32_t pre_item = 0;
   WorkItem pre_wi = {};
   // items per claim: queue_grain, down to 1 when there are fewer than 8
@@ -754,7 +772,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams params,
       item = pre_item;
       wi = pre_wi;
     } else {
-      item = list ? uniform_load(list, grab) : grab;
+      item = kAll ? grab : uniform_load(list, grab);
       wi = uniform_load(p.items, item);
     }
     ++grab;
@@ -763,7 +781,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams params,
     // the end of this item's vertex stage)
     const bool prefetch = grab < grab_end;
     if (prefetch) {
-      pre_item = list ? uniform_load(list, grab) : grab;
+      pre_item = kAll ? grab : uniform_load(list, grab);
       pre_wi = uniform_load(p.items, pre_item);
     }
     tri_acc += wi.tri_count;
@@ -780,7 +798,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams params,
 #pragma unroll
     for (int q = 0; q < 9; ++q) tm[q] = mat.texmat[q];
     const float hw = (float)sc.width * 0.5f, hh = (float)sc.height * 0.5f;
-    const float gx = kGuardPx / hw, gy = kGuardPx / hh;
+    const float gx = sc.guard_x, gy = sc.guard_y;
     const bool cached = wi.vcount <= (uint32_t)kVertexCache;
     // scenes with more bins than the LDS counters hold append every pair
     // straight to the global bins
@@ -801,6 +819,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams params,
         ix[k][2] = ip[2];
       }
     }
+    uint32_t out_all = 63u;
     if (cached) {
 #pragma unroll
       for (int q = 0; q < kVtxPerThread; ++q) {
@@ -815,6 +834,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams params,
         s_y[v] = s.Y;
         s_z[v] = s.z;
         s_f[v] = s.flags;
+        if (kAll) out_all &= s.flags;
         s_cx[v] = c.x;
         s_cy[v] = c.y;
         s_cw[v] = c.w;
@@ -823,8 +843,25 @@ __global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams params,
         s_s[v] = ss;
         s_t[v] = tt;
       }
+    } else {
+      out_all = 0u;  // (k_setup_clip takes the item whole)
+    }
+    if constexpr (kAll) {
+      out_all = wave_and(out_all);
+      if (lane == 0) reinterpret_cast<uint32_t*>(&s_out[parity])[threadIdx.x >> 6] = out_all;
     }
     __syncthreads();
+    have_pre = prefetch;
+    // Without culling five of six items have every vertex outside one plane:
+    // each of their triangles would be rejected on its own, so the item ends
+    // here (plain 512-env frame, setup 638 -> 612 us).  After culling such
+    // items are rare and the test costs more than it saves.  The next
+    // item writes the other s_out, so no barrier is needed before it.
+    if constexpr (kAll) {
+      const uint4 o = s_out[parity];
+      parity ^= 1;
+      if (__builtin_amdgcn_readfirstlane(o.x & o.y & o.z & o.w) != 0u) continue;
+    }
 
     const PixRect tile = {0, 0, sc.width - 1, sc.height - 1};
     const int sh = p.bin_shift;
@@ -916,7 +953,6 @@ __global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams params,
                  ClipFast{wi.scene, wi.node, {ix[k][0], ix[k][1], ix[k][2]}, {0u, 0u, 0u}}, lane,
                  lt_mask);
     }
-    have_pre = prefetch;
     __syncthreads();
     // one global reservation per touched bin
     for (int b = threadIdx.x; b < nlb; b += kBlock) {
@@ -1218,7 +1254,7 @@ __device__ void raster_prim(const FrameParams& p, const SceneDesc& sc, const flo
   }
   if (outcode(c[0]) & outcode(c[1]) & outcode(c[2])) return;
   const float hw = (float)sc.width * 0.5f, hh = (float)sc.height * 0.5f;
-  const float gx = kGuardPx / hw, gy = kGuardPx / hh;
+  const float gx = sc.guard_x, gy = sc.guard_y;
   bool need = false;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
@@ -1831,7 +1867,7 @@ __global__ __launch_bounds__(kClipBlock) void k_setup_clip(FrameParams p, int ph
       load_mat(p.abs_nodes + (size_t)node * 16, M);
       load_mat(p.cameras + (size_t)scene * 16, PV);
       const float hw = (float)sc.width * 0.5f, hh = (float)sc.height * 0.5f;
-      const float gx = kGuardPx / hw, gy = kGuardPx / hh;
+      const float gx = sc.guard_x, gy = sc.guard_y;
       float4* poly = s_poly[0] + tid;
       float4 c[3];
 #pragma unroll
@@ -2884,7 +2920,7 @@ __global__ __launch_bounds__(kListBlock) void k_cull(FrameParams p) {
     abs_bound(M, PV, fmaxf(fabsf(bb.lo[0]), fabsf(bb.hi[0])), fmaxf(fabsf(bb.lo[1]), fabsf(bb.hi[1])),
               fmaxf(fabsf(bb.lo[2]), fabsf(bb.hi[2])), e);
     const float hw = (float)sc.width * 0.5f, hh = (float)sc.height * 0.5f;
-    const float gx = kGuardPx / hw, gy = kGuardPx / hh;
+    const float gx = sc.guard_x, gy = sc.guard_y;
     const float mx = 2.0f * (e[0] + e[3]), my = 2.0f * (e[1] + e[3]), mz = 2.0f * (e[2] + e[3]);
     uint32_t out_all = 63u;
     bool inner = true;  // strictly inside near, far and the guard band
@@ -3144,7 +3180,7 @@ hipError_t launch_nodes(const int32_t* parents, const float* local, float* abs_o
 
 int setup_blocks_per_cu(uint32_t lds_bins) {
   int b = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_setup_bin, kBlock,
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_setup_bin<false>, kBlock,
                                                    2 * lds_bins * sizeof(uint32_t)) != hipSuccess ||
       b < 1)
     b = 4;
@@ -3156,8 +3192,12 @@ int setup_blocks_per_cu(uint32_t lds_bins) {
 hipError_t launch_setup(const FrameParams& p, const uint32_t* list, uint32_t list_ctr,
                         uint32_t queue_ctr, uint32_t grid, hipStream_t s) {
   if (p.n_items == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_setup_bin, dim3(grid < p.n_items ? grid : p.n_items), dim3(kBlock),
-                     2 * p.lds_bins * sizeof(uint32_t), s, p, list, list_ctr, queue_ctr);
+  const dim3 blocks(grid < p.n_items ? grid : p.n_items);
+  const uint32_t lds = 2 * p.lds_bins * (uint32_t)sizeof(uint32_t);
+  if (list)
+    hipLaunchKernelGGL(k_setup_bin<false>, blocks, dim3(kBlock), lds, s, p, list, list_ctr, queue_ctr);
+  else
+    hipLaunchKernelGGL(k_setup_bin<true>, blocks, dim3(kBlock), lds, s, p, list, list_ctr, queue_ctr);
   return hipGetLastError();
 }
 

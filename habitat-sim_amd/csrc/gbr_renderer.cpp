@@ -471,6 +471,8 @@ gbr_status rebuild_structure(gbr_renderer* r) {
     const int bins_x = (vw + B - 1) / B, bins_y = (vh + B - 1) / B;
     sd.width = vw;
     sd.height = vh;
+    sd.guard_x = kGuardPx / ((float)vw * 0.5f);
+    sd.guard_y = kGuardPx / ((float)vh * 0.5f);
     sd.stride = W;
     sd.planes = sc.planes ? (sc.planes & r->cfg.planes) : r->cfg.planes;
     sd.bins_x = bins_x;
@@ -529,14 +531,16 @@ gbr_status rebuild_structure(gbr_renderer* r) {
     // A camera sees its triangles unevenly: a bin of a scene with few
     // triangles, or with many bins, gets several times the average, and an
     // overflowed bin costs a rescan of the whole scene (54 us of a 145 us
-    // frame of 16 rooms, 250 of 1000 us on 512 uneven environments).  So a
-    // bin holds kSkew times its share, up to kSkewCap entries, at 64 bytes
-    // per triangle at most beside the 96 of its records.  A factor below 1
+    // frame of 16 rooms, 150 to 250 of 1000 us on 512 uneven environments).
+    // So a bin holds all triangles of its scene, up to kSkewCap, as long as
+    // the scene's entries stay within 2 MB or kSkew times their number (64
+    // bytes per triangle, beside the 96 of its records).  A factor below 1
     // asks for bins smaller than the average: it gets exactly its share.
-    constexpr double kSkew = 8.0, kSkewCap = 4096.0;
+    constexpr double kSkew = 8.0, kSkewCap = 4096.0, kSceneEntries = 1 << 19;
     double per_bin = (double)prim / nb * r->tun.bin_capacity_factor;
     if (r->tun.bin_capacity_factor >= 1.0f)
-      per_bin = std::max(per_bin, std::min(kSkew * per_bin, kSkewCap));
+      per_bin = std::max(per_bin, std::min({(double)prim, kSkewCap,
+                                            std::max(kSkew * per_bin, kSceneEntries / nb)}));
     uint32_t cap = (uint32_t)std::min<double>(std::max<double>(per_bin, r->tun.min_bin_capacity), 1u << 24);
     cap = (cap + 63) & ~63u;
     sd.bin_cap = cap;
