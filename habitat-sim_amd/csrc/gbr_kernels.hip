@@ -3136,30 +3136,35 @@ __global__ __launch_bounds__(kListBlock) void k_cull_hiz(FrameParams p) {
 
 
 __global__ __launch_bounds__(kBlock) void k_gather(GatherArgs g) {
-  const long long i = (long long)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= (long long)g.w * g.h) return;
-  const int lx = (int)(i % g.w), ly = (int)(i / g.w);
-  const int fx = g.x0 + lx, fy = g.y0 + ly;
-  const int tx = fx / g.tile_w, ty = fy / g.tile_h;
-  const int scene = ty * g.tiles_x + tx;
-  const int px = fx - tx * g.tile_w, py = fy - ty * g.tile_h;
-  uint32_t v = (uint32_t)g.fill;
-  if (scene < g.scene_count) {
-    // the scene's viewport is the bottom-left of its tile; the rest is clear
-    const int vw = g.scenes[scene].width, vh = g.scenes[scene].height;
-    if (px < vw && py < vh) {
-      const int row = g.top_down ? (vh - 1 - py) : py;
-      v = *reinterpret_cast<const uint32_t*>(
-          g.plane + (((long long)scene * g.tile_h + row) * g.tile_w + px) * 4);
+  // a workgroup takes kBlock pixels of a row, and rows gridDim.y apart
+  const int lx = (int)(blockIdx.x * kBlock + threadIdx.x);
+  if (lx >= g.w) return;
+  const int fx = g.x0 + lx;
+  const int tx = fx / g.tile_w;
+  const int px = fx - tx * g.tile_w;
+  for (int ly = (int)blockIdx.y; ly < g.h; ly += (int)gridDim.y) {
+    const int fy = g.y0 + ly;
+    const int ty = fy / g.tile_h;
+    const int scene = ty * g.tiles_x + tx;
+    const int py = fy - ty * g.tile_h;
+    uint32_t v = (uint32_t)g.fill;
+    if (scene < g.scene_count) {
+      // the scene's viewport is the bottom-left of its tile; the rest is clear
+      const int vw = g.scenes[scene].width, vh = g.scenes[scene].height;
+      if (px < vw && py < vh) {
+        const int row = g.top_down ? (vh - 1 - py) : py;
+        v = *reinterpret_cast<const uint32_t*>(
+            g.plane + (((long long)scene * g.tile_h + row) * g.tile_w + px) * 4);
+      }
     }
-  }
-  uint8_t* d = g.dst + (long long)ly * g.dst_stride + (long long)lx * g.dst_bytes;
-  if (g.dst_bytes == 4) {
-    *reinterpret_cast<uint32_t*>(d) = v;
-  } else {
-    d[0] = v & 0xff;
-    d[1] = (v >> 8) & 0xff;
-    d[2] = (v >> 16) & 0xff;
+    uint8_t* d = g.dst + (long long)ly * g.dst_stride + (long long)lx * g.dst_bytes;
+    if (g.dst_bytes == 4) {
+      *reinterpret_cast<uint32_t*>(d) = v;
+    } else {
+      d[0] = v & 0xff;
+      d[1] = (v >> 8) & 0xff;
+      d[2] = (v >> 16) & 0xff;
+    }
   }
 }
 
@@ -3284,9 +3289,9 @@ hipError_t launch_cull_hiz(const FrameParams& p, hipStream_t s) {
 }
 
 hipError_t launch_gather(const GatherArgs& g, hipStream_t s) {
-  long long n = (long long)g.w * g.h;
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_gather, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, g);
+  if (g.w <= 0 || g.h <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_gather, dim3((unsigned)((g.w + kBlock - 1) / kBlock), (unsigned)(g.h < 32768 ? g.h : 32768)),
+                     dim3(kBlock), 0, s, g);
   return hipGetLastError();
 }
 
