@@ -399,6 +399,21 @@ struct FrameParams {
   int32_t no_textures;
 };
 
+// One frame's host inputs, in pinned memory: kInputParts runs of 16-byte
+// words that go to device arrays one after the other, then the local
+// transforms that changed (4 words each) with their node indices.
+constexpr uint32_t kInputParts = 6;
+
+struct InputArgs {
+  const uint4* src;
+  uint4* dst[kInputParts];
+  uint32_t end[kInputParts];  // of each run, in words from src
+  const uint32_t* nodes;      // node index of each changed transform
+  const uint4* transforms;
+  uint4* local;               // [node] of 4 words
+  uint32_t n_nodes;
+};
+
 struct GatherArgs {
   const uint8_t* plane;
   const SceneDesc* scenes;  // per-scene viewports

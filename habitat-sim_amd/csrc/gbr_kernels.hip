@@ -392,6 +392,29 @@ __device__ __forceinline__ void node_transform(const int32_t* __restrict__ paren
   }
 }
 
+// The frame's host inputs (cameras, lights, changed local transforms) read
+// by the GPU from one pinned block: a launch in place of four to six copies
+// of a few KB, each of which costs the host a submission and the stream a
+// blit kernel and the gap before it (4.4 us + 4 us apiece on a one-room frame),
+// and of one pageable copy per scene with moved objects.
+__global__ __launch_bounds__(kBlock) void k_inputs(InputArgs a) {
+  const uint32_t fixed = a.end[kInputParts - 1], total = fixed + 4u * a.n_nodes;
+  for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < total; i += gridDim.x * kBlock) {
+    if (i < fixed) {
+      const uint4 v = a.src[i];
+      uint32_t begin = 0;
+#pragma unroll
+      for (uint32_t k = 0; k < kInputParts; ++k) {
+        if (i >= begin && i < a.end[k]) a.dst[k][i - begin] = v;
+        begin = a.end[k];
+      }
+    } else {
+      const uint32_t j = i - fixed;
+      a.local[4 * (size_t)a.nodes[j >> 2] + (j & 3u)] = a.transforms[j];
+    }
+  }
+}
+
 __global__ __launch_bounds__(kBlock) void k_nodes(const int32_t* __restrict__ parents,
                                                   const float* __restrict__ local,
                                                   float* __restrict__ abs_out, uint32_t n,
@@ -406,7 +429,7 @@ __global__ __launch_bounds__(kBlock) void k_nodes(const int32_t* __restrict__ pa
   if (i0 < kCtrTotal) counters[i0 * kCtrStride] = 0u;
   if (i0 == 0) *frame += 1u;
   for (uint32_t j = i0; j < kStatCount * kStatStripes; j += gridDim.x * kBlock) stats[j] = 0ull;
-  // the host uploads *dirty with the cameras of every frame: 0 when no local
+  // *dirty comes with the host inputs of every frame: 0 when no local
   // transform and no node list changed since the previous frame, whose
   // absolute transforms (and normal matrices) are still in place.  The
   // grid is capped (a frame without changes then dispatches few
@@ -3171,6 +3194,14 @@ __global__ __launch_bounds__(kBlock) void k_gather(GatherArgs g) {
 // --------------------------------------------------------------------------
 // Host-side launchers
 // --------------------------------------------------------------------------
+
+hipError_t launch_inputs(const InputArgs& a, uint32_t max_blocks, hipStream_t s) {
+  const uint64_t words = (uint64_t)a.end[kInputParts - 1] + 4ull * a.n_nodes;
+  const uint64_t blocks = (words + kBlock - 1) / kBlock;
+  hipLaunchKernelGGL(k_inputs, dim3((uint32_t)(blocks < max_blocks ? (blocks ? blocks : 1) : max_blocks)),
+                     dim3(kBlock), 0, s, a);
+  return hipGetLastError();
+}
 
 hipError_t launch_nodes(const int32_t* parents, const float* local, float* abs_out, uint32_t n,
                         uint32_t* counters, unsigned long long* stats, uint32_t* frame,

@@ -32,6 +32,7 @@
 #pragma STDC FP_CONTRACT OFF
 
 namespace gbr {
+hipError_t launch_inputs(const InputArgs& a, uint32_t max_blocks, hipStream_t s);
 hipError_t launch_nodes(const int32_t* parents, const float* local, float* abs_out, uint32_t n,
                         uint32_t* counters, unsigned long long* stats, uint32_t* frame,
                         float* nrm_out, const uint32_t* dirty, uint32_t max_blocks, hipStream_t s);
@@ -142,6 +143,7 @@ struct Light {
 struct Scene {
   std::vector<int32_t> parents;
   std::vector<Mat4> transforms;
+  std::vector<Mat4> uploaded;  // the transforms as the device has them
   std::vector<Batch> batches;
   std::vector<Draw> draws;
   std::vector<Light> lights;
@@ -249,21 +251,25 @@ struct gbr_renderer {
   DevBuf<uint32_t> d_color, d_sem;
   DevBuf<float> d_depth, d_lin;
   DevBuf<uint8_t> d_fb_color, d_fb_depth, d_stage;
-  // pinned per-frame staging for cameras
-  float* h_cam = nullptr;
-  size_t h_cam_cap = 0;
+  // pinned memory of the frames' host inputs, in blocks taken in turn: a
+  // block is written again once its frame's k_inputs has read it
+  struct InputBlock {
+    hipEvent_t read = nullptr;
+    bool pending = false;
+  };
+  std::array<InputBlock, 3> inputs;
+  uint8_t* h_inputs = nullptr;
+  size_t input_cap = 0;  // of a block
+  size_t input_next = 0;
+  std::vector<uint32_t> moved;  // nodes whose local transform changed since the last frame
   uint8_t* h_read = nullptr;  // pinned staging of host readbacks (kReadbackBytes, or one row)
   size_t h_read_cap = 0;
-  uint8_t* h_light = nullptr;  // pinned per-frame staging for lights
-  size_t h_light_cap = 0;
-  hipEvent_t cam_event = nullptr;
   // optional per-stage timing of gbr_draw (tuning.timing): one event set per
   // frame since the last gbr_frame_timings(), up to kTimingFrames frames
   std::vector<std::array<hipEvent_t, 2 * GBR_TIMING_SLOTS>> t_pool;
   std::vector<std::array<bool, GBR_TIMING_SLOTS>> t_used;
   size_t t_frames = 0;
   int t_cur = -1;
-  bool cam_event_pending = false;
 
   uint64_t tile_pixels() const { return (uint64_t)cfg.tile_size[0] * cfg.tile_size[1]; }
   uint32_t scene_count() const { return (uint32_t)scenes.size(); }
@@ -462,6 +468,7 @@ gbr_status rebuild_structure(gbr_renderer* r) {
       local.insert(local.end(), sc.transforms[i].m, sc.transforms[i].m + 16);
     }
     sc.xform_dirty = false;
+    sc.uploaded = sc.transforms;
     // counting sort of draws by batch id, stable (Renderer.cpp:1151-1188)
     std::vector<uint32_t> order;
     order.reserve(sc.draws.size());
@@ -635,72 +642,100 @@ gbr_status rebuild_structure(gbr_renderer* r) {
   return GBR_OK;
 }
 
-gbr_status upload_dirty_transforms(gbr_renderer* r) {
+// The nodes of scenes handed out for writing whose local transform differs
+// from the device's: a program that moves a few objects gets a view of all of
+// the scene's nodes, and only the moved ones are sent.
+void find_moved(gbr_renderer* r) {
+  r->moved.clear();
   for (uint32_t si = 0; si < r->scene_count(); ++si) {
     Scene& sc = r->scenes[si];
     if (!sc.xform_dirty) continue;
     sc.xform_dirty = false;
-    if (sc.transforms.empty()) continue;
-    r->nodes_dirty = true;
-    HIP_TRY(hipMemcpyAsync(r->d_local.ptr + (size_t)r->scene_node_base[si] * 16, sc.transforms.data(),
-                           sc.transforms.size() * sizeof(Mat4), hipMemcpyHostToDevice, r->stream));
+    for (size_t i = 0; i < sc.transforms.size(); ++i)
+      if (std::memcmp(&sc.transforms[i], &sc.uploaded[i], sizeof(Mat4)) != 0) {
+        sc.uploaded[i] = sc.transforms[i];
+        r->moved.push_back(r->scene_node_base[si] + (uint32_t)i);
+      }
   }
-  return GBR_OK;
+  if (!r->moved.empty()) r->nodes_dirty = true;
 }
 
-gbr_status upload_cameras(gbr_renderer* r) {
+// Cameras, lights and moved nodes into a pinned block, and the kernel that
+// takes them to their arrays.
+gbr_status upload_inputs(gbr_renderer* r) {
   const size_t n = r->scene_count();
-  // projection*view, unprojection, camera position + forward, then the
-  // frame's node-recompute flag
-  const size_t need = n * 26 + 1;
-  if (r->cam_event_pending) {
-    HIP_TRY(hipEventSynchronize(r->cam_event));
-    r->cam_event_pending = false;
-  }
-  if (r->h_cam_cap < need) {
-    if (r->h_cam) (void)hipHostFree(r->h_cam);
-    r->h_cam = nullptr;
-    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&r->h_cam), need * sizeof(float)));
-    r->h_cam_cap = need;
-  }
-  for (size_t i = 0; i < n; ++i) {
-    std::memcpy(r->h_cam + i * 16, r->scenes[i].camera.m, 64);
-    r->h_cam[n * 16 + 2 * i] = r->scenes[i].unproj[0];
-    r->h_cam[n * 16 + 2 * i + 1] = r->scenes[i].unproj[1];
-    std::memcpy(r->h_cam + n * 18 + 8 * i, r->scenes[i].cam_info, 32);
-  }
-  TRY(r->d_cameras.reserve(n * 16 + 16));
-  TRY(r->d_unproj.reserve(n * 2 + 2));
-  TRY(r->d_caminfo.reserve(n * 8 + 8));
-  HIP_TRY(hipMemcpyAsync(r->d_cameras.ptr, r->h_cam, n * 64, hipMemcpyHostToDevice, r->stream));
-  HIP_TRY(hipMemcpyAsync(r->d_unproj.ptr, r->h_cam + n * 16, n * 8, hipMemcpyHostToDevice, r->stream));
-  HIP_TRY(hipMemcpyAsync(r->d_caminfo.ptr, r->h_cam + n * 18, n * 32, hipMemcpyHostToDevice,
-                         r->stream));
-  {
-    const uint32_t flag = r->nodes_dirty ? 1u : 0u;
-    std::memcpy(r->h_cam + n * 26, &flag, sizeof flag);
-    TRY(r->d_nodes_dirty.reserve(1));
-    HIP_TRY(hipMemcpyAsync(r->d_nodes_dirty.ptr, r->h_cam + n * 26, sizeof flag,
-                           hipMemcpyHostToDevice, r->stream));
-    r->nodes_dirty = false;
-  }
-  if (r->cfg.max_light_count) {
-    // per scene its first light and light count (at most max_light_count,
-    // the count the reference's shaders are compiled for), then the lights
-    // with their nodes as global indices
-    size_t nl = 0;
+  auto padded = [](size_t bytes) { return (bytes + 15) & ~size_t(15); };
+  // lights: per scene the first one and their count (at most
+  // max_light_count, the count the reference's shaders are compiled for),
+  // then the lights with their nodes as global indices
+  const bool lit = r->cfg.max_light_count != 0;
+  size_t nl = 0;
+  if (lit)
     for (size_t i = 0; i < n; ++i)
       nl += std::min<size_t>(r->scenes[i].lights.size(), r->cfg.max_light_count);
-    const size_t head = (n * 2 * sizeof(uint32_t) + 15) & ~size_t(15);
-    const size_t bytes = head + std::max<size_t>(nl, 1) * sizeof(LightDesc);
-    if (r->h_light_cap < bytes) {
-      if (r->h_light) (void)hipHostFree(r->h_light);
-      r->h_light = nullptr;
-      HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&r->h_light), bytes));
-      r->h_light_cap = bytes;
+  const size_t part_bytes[kInputParts] = {
+      n * 64,           // projection * view
+      padded(n * 8),    // unprojection
+      n * 32,           // camera position, forward
+      16,               // the node-recompute flag
+      lit ? padded(n * 2 * sizeof(uint32_t)) : 0, nl * sizeof(LightDesc)};
+  static_assert(sizeof(LightDesc) % 16 == 0, "whole words");
+  size_t fixed = 0;
+  for (size_t b : part_bytes) fixed += b;
+  const size_t nm = r->moved.size();
+  const size_t need = fixed + nm * sizeof(Mat4) + nm * sizeof(uint32_t);
+
+  if (r->input_cap < need) {
+    // all blocks at once, with room for moved nodes, so that frames after
+    // the first do not allocate
+    const size_t room = std::max<size_t>({nm, std::min<size_t>(r->n_nodes, 4096), r->n_nodes / 16});
+    const size_t cap = padded(fixed + room * (sizeof(Mat4) + sizeof(uint32_t)));
+    for (auto& b : r->inputs) {
+      if (b.pending) HIP_TRY(hipEventSynchronize(b.read));
+      b.pending = false;
     }
-    uint32_t* ranges = reinterpret_cast<uint32_t*>(r->h_light);
-    LightDesc* lights = reinterpret_cast<LightDesc*>(r->h_light + head);
+    if (r->h_inputs) (void)hipHostFree(r->h_inputs);
+    r->h_inputs = nullptr;
+    r->input_cap = 0;
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&r->h_inputs), cap * r->inputs.size()));
+    r->input_cap = cap;
+  }
+  gbr_renderer::InputBlock& blk = r->inputs[r->input_next];
+  uint8_t* const block = r->h_inputs + r->input_next * r->input_cap;
+  r->input_next = (r->input_next + 1) % r->inputs.size();
+  if (blk.pending) {
+    HIP_TRY(hipEventSynchronize(blk.read));
+    blk.pending = false;
+  }
+  TRY(r->d_cameras.reserve(n * 16 + 16));
+  TRY(r->d_unproj.reserve(n * 2 + 4));
+  TRY(r->d_caminfo.reserve(n * 8 + 8));
+  TRY(r->d_nodes_dirty.reserve(4));
+  if (lit) {
+    TRY(r->d_scene_lights.reserve(n * 2 + 4));
+    TRY(r->d_lights.reserve(std::max<size_t>(nl, 1)));
+  }
+
+  uint8_t* at = block;
+  float* cam = reinterpret_cast<float*>(at);
+  at += part_bytes[0];
+  float* un = reinterpret_cast<float*>(at);
+  at += part_bytes[1];
+  float* info = reinterpret_cast<float*>(at);
+  at += part_bytes[2];
+  for (size_t i = 0; i < n; ++i) {
+    const Scene& sc = r->scenes[i];
+    std::memcpy(cam + 16 * i, sc.camera.m, 64);
+    un[2 * i] = sc.unproj[0];
+    un[2 * i + 1] = sc.unproj[1];
+    std::memcpy(info + 8 * i, sc.cam_info, 32);
+  }
+  const uint32_t flag[4] = {r->nodes_dirty ? 1u : 0u, 0u, 0u, 0u};
+  std::memcpy(at, flag, sizeof flag);
+  at += part_bytes[3];
+  if (lit) {
+    uint32_t* ranges = reinterpret_cast<uint32_t*>(at);
+    LightDesc* lights = reinterpret_cast<LightDesc*>(at + part_bytes[4]);
     uint32_t k = 0;
     for (size_t i = 0; i < n; ++i) {
       const Scene& sc = r->scenes[i];
@@ -717,16 +752,36 @@ gbr_status upload_cameras(gbr_renderer* r) {
         std::memcpy(d.color, L.color, sizeof d.color);
       }
     }
-    TRY(r->d_scene_lights.reserve(n * 2 + 2));
-    TRY(r->d_lights.reserve(std::max<size_t>(nl, 1)));
-    HIP_TRY(hipMemcpyAsync(r->d_scene_lights.ptr, ranges, n * 2 * sizeof(uint32_t),
-                           hipMemcpyHostToDevice, r->stream));
-    if (nl)
-      HIP_TRY(hipMemcpyAsync(r->d_lights.ptr, lights, nl * sizeof(LightDesc),
-                             hipMemcpyHostToDevice, r->stream));
   }
-  HIP_TRY(hipEventRecord(r->cam_event, r->stream));
-  r->cam_event_pending = true;
+  at = block + fixed;
+  Mat4* mats = reinterpret_cast<Mat4*>(at);
+  uint32_t* nodes = reinterpret_cast<uint32_t*>(at + nm * sizeof(Mat4));
+  size_t si = 0;
+  for (size_t k = 0; k < nm; ++k) {  // (ascending nodes)
+    while (si + 1 < n && r->scene_node_base[si + 1] <= r->moved[k]) ++si;
+    mats[k] = r->scenes[si].uploaded[r->moved[k] - r->scene_node_base[si]];
+    nodes[k] = r->moved[k];
+  }
+
+  InputArgs a{};
+  a.src = reinterpret_cast<const uint4*>(block);
+  void* const dst[kInputParts] = {r->d_cameras.ptr,     r->d_unproj.ptr,       r->d_caminfo.ptr,
+                                  r->d_nodes_dirty.ptr, r->d_scene_lights.ptr, r->d_lights.ptr};
+  uint32_t words = 0;
+  for (uint32_t k = 0; k < kInputParts; ++k) {
+    words += (uint32_t)(part_bytes[k] / 16);
+    a.dst[k] = static_cast<uint4*>(dst[k]);
+    a.end[k] = words;
+  }
+  a.transforms = reinterpret_cast<const uint4*>(mats);
+  a.nodes = nodes;
+  a.local = reinterpret_cast<uint4*>(r->d_local.ptr);
+  a.n_nodes = (uint32_t)nm;
+  HIP_TRY(launch_inputs(a, (uint32_t)r->cu_count, r->stream));
+  HIP_TRY(hipEventRecord(blk.read, r->stream));
+  blk.pending = true;
+  r->nodes_dirty = false;
+  r->moved.clear();
   return GBR_OK;
 }
 
@@ -791,8 +846,14 @@ gbr_status do_draw(gbr_renderer* r) {
   TRY(ensure_planes(r));
   if (r->assets_dirty) TRY(upload_assets(r));
   if (r->structure_dirty) TRY(rebuild_structure(r));
-  else TRY(upload_dirty_transforms(r));
-  TRY(upload_cameras(r));
+  else find_moved(r);
+  {
+    const gbr_status st = upload_inputs(r);
+    if (st != GBR_OK) {
+      r->structure_dirty = true;  // moved nodes were not sent: the next draw sends everything
+      return st;
+    }
+  }
   TRY(r->d_stats.reserve(kStatCount * kStatStripes));
   TRY(r->d_counters.reserve(kCtrTotal * kCtrStride));
   TRY(r->d_vis.reserve((size_t)r->scene_count() * r->tile_pixels()));
@@ -1213,8 +1274,12 @@ gbr_status gbr_create(const gbr_config* config, gbr_renderer** out) {
   const uint64_t n = (uint64_t)config->tile_count[0] * config->tile_count[1];
   r->scenes.resize(n);
   hipError_t e = hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipEventCreateWithFlags(&r->cam_event, hipEventDisableTiming);
+  for (auto& blk : r->inputs)
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&blk.read, hipEventDisableTiming);
   if (e != hipSuccess) {
+    for (auto& blk : r->inputs)
+      if (blk.read) (void)hipEventDestroy(blk.read);
+    if (r->stream) (void)hipStreamDestroy(r->stream);
     delete r;
     return fail(GBR_ERR_DEVICE, std::string("gbr_create: ") + hipGetErrorString(e));
   }
@@ -1278,10 +1343,10 @@ gbr_status gbr_destroy(gbr_renderer* r) {
   r->d_nmat.release();
   r->d_lights.release();
   r->d_scene_lights.release();
-  if (r->h_cam) (void)hipHostFree(r->h_cam);
-  if (r->h_light) (void)hipHostFree(r->h_light);
+  if (r->h_inputs) (void)hipHostFree(r->h_inputs);
+  for (auto& blk : r->inputs)
+    if (blk.read) (void)hipEventDestroy(blk.read);
   if (r->h_read) (void)hipHostFree(r->h_read);
-  if (r->cam_event) (void)hipEventDestroy(r->cam_event);
   for (auto& set : r->t_pool)
     for (hipEvent_t e : set)
       if (e) (void)hipEventDestroy(e);
