@@ -1,16 +1,18 @@
 // Chunk-visibility MLP (32 -> 256 -> 256 -> 1, ReLU) on gfx950 MFMA:
 // BF16 operands, FP32 accumulation, FP32 master weights with Adam.
 //
-// Every matrix product is an "NT" GEMM, C[M][N] = sum_k A[M][K] * Bt[N][K],
-// with both operands K-contiguous so that a wave's MFMA fragments are single
-// 16-byte loads:
-//   forward   H1 = relu(X  W1^T + b1)        A = X   [B][32],  Bt = W1  [256][32]
-//             H2 = relu(H1 W2^T + b2)        A = H1  [B][256], Bt = W2  [256][256]
-//   backward  dW2 = dH2^T H1                 A = dH2^T [256][B], Bt = H1^T [256][B]
-//             dH1 = (dH2 W2) o [H1 > 0]      A = dH2 [B][256], Bt = W2^T [256][256]
-//             dW1 = dH1^T X                  A = dH1^T [256][B], Bt = X^T  [32][B]
-// The last layer (256 -> 1), the loss and the bias gradients are reductions
-// (no atomics: each output has one writer).
+// A training step is four launches (it was nineteen):
+//   k_train_forward  per 32 rows of the minibatch: the rows from the training
+//                    set, both layers, the logits, the loss and its gradient
+//                    by the logits, dH2 = [H2 > 0] dl w3
+//   k_train_grads    dW2 = dH2^T H1, dH1 = (dH2 W2) o [H1 > 0] and the sums over
+//                    the batch for w3, b2, b3 and the loss
+//   k_train_grads1   dW1 = dH1^T X and the sums for b1
+//   k_adam           the weights, and their bf16 copies
+// Every product is an "NT" one, C[M][N] = sum_k A[M][K] * Bt[N][K], with both
+// operands K-contiguous so that a wave's MFMA fragments are single 16-byte
+// loads.  The sums are reductions with one writer per output (no atomics),
+// and every sum runs in a fixed order, whatever the launch geometry.
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
@@ -38,152 +40,301 @@ __device__ __forceinline__ int rows_of(int M, const uint32_t* M_dev) {
   return M_dev ? min(M, (int)*M_dev) : M;
 }
 
+// four bf16 in one 8-byte store
+__device__ __forceinline__ void store4(uint16_t* dst, uint16_t a, uint16_t b, uint16_t c, uint16_t d) {
+  *reinterpret_cast<uint2*>(dst) =
+      make_uint2((uint32_t)a | ((uint32_t)b << 16), (uint32_t)c | ((uint32_t)d << 16));
+}
+
 // --------------------------------------------------------------------------
-// NT GEMM, one 32x32 output tile per wave (v_mfma_f32_32x32x16_bf16):
+// One 32x32 tile of an NT product by one wave (v_mfma_f32_32x32x16_bf16):
 // lane l supplies A[m0 + l%32][k + 8*(l/32) .. +8] and Bt[n0 + l%32][same k];
-// accumulator v holds C[m0 + 8*(v/4) + 4*(l/32) + v%4][n0 + l%32].
-// Requirements (checked on the host): K % 16 == 0, lda % 8 == 0,
-// ldb % 8 == 0, 16-byte aligned base pointers.
+// accumulator v holds C[m0 + 8*(v/4) + 4*(l/32) + v%4][n0 + l%32].  The K
+// steps run in order, k = 0, 16, ...
+//
+// A weight gradient is a chain of K / 16 = 256 such steps (4096 rows) in 64
+// waves, so what bounds it is the latency of the fragments' loads: kAhead
+// steps' fragments are in flight at any time (128 registers), 68 us down to
+// 9 for dW2 at 4096 rows against one step's loads at a time.
+// Requirements (the callers'): K % 16 == 0, rows of 16-byte alignment.
 // --------------------------------------------------------------------------
+constexpr int kAhead = 16;
 
-__global__ __launch_bounds__(256) void k_gemm_nt(GemmArgs g) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int M = rows_of(g.M, g.M_dev);
-  const int tiles_n = (g.N + 31) / 32;
-  const int tile = blockIdx.x * 4 + wave;
-  const int tiles_m = (M + 31) / 32;
-  if (tile >= tiles_m * tiles_n) return;
-  const int m0 = (tile / tiles_n) * 32, n0 = (tile % tiles_n) * 32;
-  const int am = m0 + (lane & 31), bn = n0 + (lane & 31);
+__device__ __forceinline__ floatx16 tile_product(const uint16_t* __restrict__ A, size_t lda,
+                                                 const uint16_t* __restrict__ Bt, size_t ldb, int K,
+                                                 int m0, int n0, int lane) {
   const int kofs = 8 * (lane >> 5);
-  const bool arow = am < M, brow = bn < g.N;
-  const uint16_t* ap = g.A + (size_t)am * g.lda + kofs;
-  const uint16_t* bp = g.Bt + (size_t)bn * g.ldb + kofs;
-  floatx16 acc = {};
-  for (int k = 0; k < g.K; k += 16) {
-    bf16x8 a = {}, b = {};
-    if (arow) a = *reinterpret_cast<const bf16x8*>(ap + k);
-    if (brow) b = *reinterpret_cast<const bf16x8*>(bp + k);
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-  }
-  const int n = bn;
-  if (n >= g.N) return;
+  const uint16_t* ap = A + (size_t)(m0 + (lane & 31)) * lda + kofs;
+  const uint16_t* bp = Bt + (size_t)(n0 + (lane & 31)) * ldb + kofs;
+  const int steps = K / 16;
+  bf16x8 a[kAhead], b[kAhead];
 #pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int m = m0 + 8 * (v / 4) + 4 * (lane >> 5) + (v % 4);
-    if (m >= M) continue;
-    float x = acc[v] * g.alpha;
-    if (g.C) g.C[(size_t)m * g.ldc + n] = x;
-    if (g.bias) x = x + g.bias[n];
-    if (g.mask) x = bf2f(g.mask[(size_t)m * g.ldmask + n]) > 0.0f ? x : 0.0f;
-    if (g.relu) x = x > 0.0f ? x : 0.0f;
-    if (g.D) g.D[(size_t)m * g.ldd + n] = f2bf(x);
-    if (g.Dt) g.Dt[(size_t)n * g.lddt + m] = f2bf(x);
+  for (int u = 0; u < kAhead; ++u)
+    if (u < steps) {
+      a[u] = *reinterpret_cast<const bf16x8*>(ap + 16 * u);
+      b[u] = *reinterpret_cast<const bf16x8*>(bp + 16 * u);
+    }
+  floatx16 acc = {};
+  int s0 = 0;
+  for (; s0 + 2 * kAhead <= steps; s0 += kAhead) {
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[u], b[u], acc, 0, 0, 0);
+      a[u] = *reinterpret_cast<const bf16x8*>(ap + 16 * (size_t)(s0 + u + kAhead));
+      b[u] = *reinterpret_cast<const bf16x8*>(bp + 16 * (size_t)(s0 + u + kAhead));
+    }
   }
-}
-
-// logit[r] = sum_k H2[r][k] * w3[k] + b3, one wave per row
-__global__ __launch_bounds__(256) void k_last_layer(const uint16_t* __restrict__ H2,
-                                                    const uint16_t* __restrict__ w3,
-                                                    const float* __restrict__ b3,
-                                                    float* __restrict__ logits, int rows,
-                                                    const uint32_t* __restrict__ rows_dev) {
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (row >= rows_of(rows, rows_dev)) return;
-  float s = 0.0f;
-  for (int k = lane; k < kMlpHidden; k += 64)
-    s += bf2f(H2[(size_t)row * kMlpHidden + k]) * bf2f(w3[k]);
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-  if (lane == 0) logits[row] = s + *b3;
-}
-
-// weighted binary cross-entropy with logits, per row:
-//   loss_r = w_r [log(1 + e^-|z|) + max(z, 0) - z y],  dl_r = w_r (sigmoid(z) - y) / rows
-// with w_r = pos_weight for visible rows, 1 otherwise
-__global__ __launch_bounds__(256) void k_head(const float* __restrict__ logits,
-                                              const uint8_t* __restrict__ labels, float pos_weight,
-                                              int rows, float* __restrict__ dl,
-                                              float* __restrict__ loss) {
-  const int r = blockIdx.x * 256 + threadIdx.x;
-  if (r >= rows) return;
-  const float z = logits[r];
-  const float y = labels[r] ? 1.0f : 0.0f;
-  const float w = labels[r] ? pos_weight : 1.0f;
-  const float sig = 1.0f / (1.0f + expf(-z));
-  dl[r] = w * (sig - y) / (float)rows;
-  loss[r] = w * (log1pf(expf(-fabsf(z))) + fmaxf(z, 0.0f) - z * y);
-}
-
-// dH2 = [H2 > 0] dl[r] w3[k], row-major [rows][256] and transposed [256][rows]
-// (two passes so that each store is coalesced)
-__global__ __launch_bounds__(256) void k_dh2(const uint16_t* __restrict__ H2,
-                                             const uint16_t* __restrict__ H2t,
-                                             const float* __restrict__ dl,
-                                             const uint16_t* __restrict__ w3, int rows,
-                                             uint16_t* __restrict__ dH2,
-                                             uint16_t* __restrict__ dH2t) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  const size_t n = (size_t)rows * kMlpHidden;
-  if (i < n) {
-    const size_t r = i / kMlpHidden, k = i % kMlpHidden;
-    dH2[i] = bf2f(H2[i]) > 0.0f ? f2bf(dl[r] * bf2f(w3[k])) : (uint16_t)0;
-  } else if (i < 2 * n) {
-    const size_t j = i - n, k = j / rows, r = j % rows;
-    dH2t[j] = bf2f(H2t[j]) > 0.0f ? f2bf(dl[r] * bf2f(w3[k])) : (uint16_t)0;
+  for (; s0 < steps; s0 += kAhead) {
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      if (s0 + u < steps) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[u], b[u], acc, 0, 0, 0);
+      if (s0 + u + kAhead < steps) {
+        a[u] = *reinterpret_cast<const bf16x8*>(ap + 16 * (size_t)(s0 + u + kAhead));
+        b[u] = *reinterpret_cast<const bf16x8*>(bp + 16 * (size_t)(s0 + u + kAhead));
+      }
+    }
   }
+  return acc;
 }
 
-// out[j] = sum_r Mt[j][r] * (w ? w[r] : 1), one wave per j
-__global__ __launch_bounds__(256) void k_row_sums(const uint16_t* __restrict__ Mt,
-                                                  const float* __restrict__ w, int n, int rows,
-                                                  float* __restrict__ out) {
-  const int j = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (j >= n) return;
+__device__ __forceinline__ void store_tile(const floatx16& acc, float* __restrict__ C, int ldc, int m0,
+                                           int n0, int lane) {
+  const int n = n0 + (lane & 31);
+#pragma unroll
+  for (int v = 0; v < 16; ++v)
+    C[(size_t)(m0 + 8 * (v / 4) + 4 * (lane >> 5) + v % 4) * ldc + n] = acc[v];
+}
+
+// sum_r row[r] * (w ? w[r] : 1) by one wave: lane l adds r = l, l + 64, ...,
+// then a butterfly (sixteen loads in flight at a time)
+__device__ __forceinline__ float row_sum(const uint16_t* __restrict__ row, const float* __restrict__ w,
+                                         int rows, int lane) {
   float s = 0.0f;
-  for (int r = lane; r < rows; r += 64) {
-    const float x = bf2f(Mt[(size_t)j * rows + r]);
-    s += w ? x * w[r] : x;
+  int r = lane;
+  for (; r - lane + 1024 <= rows; r += 1024) {
+    uint16_t x[16];
+    float y[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      x[q] = row[r + 64 * q];
+      y[q] = w ? w[r + 64 * q] : 1.0f;
+    }
+#pragma unroll
+    for (int q = 0; q < 16; ++q) s += w ? bf2f(x[q]) * y[q] : bf2f(x[q]);
   }
+  for (; r < rows; r += 64) s += w ? bf2f(row[r]) * w[r] : bf2f(row[r]);
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-  if (lane == 0) out[j] = s;
+  return s;
 }
 
-// out[0] = sum of v[0..n) (one workgroup)
-__global__ __launch_bounds__(256) void k_sum(const float* __restrict__ v, int n,
-                                             float* __restrict__ out) {
-  __shared__ float s_part[4];
-  float s = 0.0f;
-  for (int i = threadIdx.x; i < n; i += 256) s += v[i];
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-  if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) out[0] = (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
+// sum of v[0..n) by one wave, as four partial sums of 256-strided elements
+__device__ __forceinline__ float quarter_sums(const float* __restrict__ v, int n, int lane) {
+  float part[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    float s = 0.0f;
+#pragma unroll 8
+    for (int i = 64 * q + lane; i < n; i += 256) s += v[i];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    part[q] = s;
+  }
+  return (part[0] + part[1]) + (part[2] + part[3]);
 }
 
-// minibatch: row i of the batch = dataset row hash(seed, step, i) mod total,
-// copied row-major and transposed, with its label
+// minibatch: row i of the batch = dataset row hash(seed, step, i) mod total
 __device__ __forceinline__ uint64_t mix64(uint64_t z) {
   z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
   z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
   return z ^ (z >> 31);
 }
 
-__global__ __launch_bounds__(256) void k_gather(const uint16_t* __restrict__ X,
-                                                const uint8_t* __restrict__ Y, uint64_t total,
-                                                uint64_t seed, uint64_t step, int batch,
-                                                uint16_t* __restrict__ Xb,
-                                                uint16_t* __restrict__ Xbt,
-                                                uint8_t* __restrict__ Yb) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= batch) return;
-  const uint64_t src = mix64(seed ^ mix64(step * 0x9e3779b97f4a7c15ull + (uint64_t)i)) % total;
-#pragma unroll 4
-  for (int k = 0; k < kMlpIn; ++k) {
-    const uint16_t x = X[src * kMlpIn + k];
-    Xb[(size_t)i * kMlpIn + k] = x;
-    Xbt[(size_t)k * batch + i] = x;
+constexpr int kTrainRows = 32;                  // rows per workgroup of k_train_forward
+constexpr int kTrainThreads = kMlpHidden / 32 * 64;
+constexpr int kTrainStride = kMlpHidden + 8;    // padded LDS row of bf16
+constexpr int kTrainPart = kMlpHidden + 4;      // padded LDS row of fp32
+
+// A workgroup of 8 waves takes 32 rows through the forward pass, wave w the
+// hidden columns [32w, 32w + 32) of both layers, and leaves behind what the
+// gradients read: X, H1, H2 and dH2 transposed, and dH2.
+//   loss_r = w_r [log(1 + e^-|z|) + max(z, 0) - z y],  dl_r = w_r (sigmoid(z) - y) / rows
+// with w_r = pos_weight for visible rows, 1 otherwise; dH2 = [H2 > 0] dl[r] w3[k].
+// The arithmetic and its order are the scorer's (k_mlp_score).  As six
+// launches the same work took 105 us at 4096 rows; 128 workgroups here, 10 us.
+__global__ __launch_bounds__(kTrainThreads) void k_train_forward(TrainArgs t) {
+  __shared__ uint16_t s_h[kTrainRows * kTrainStride];  // H1, then dH2
+  __shared__ float s_part[kTrainRows * kTrainPart];
+  __shared__ uint64_t s_src[kTrainRows];
+  __shared__ float s_dl[kTrainRows];
+  __shared__ uint8_t s_y[kTrainRows];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int lr = lane & 31, kh = 8 * (lane >> 5), hi = lane >> 5;
+  const int n = wave * 32 + lr;  // this lane's hidden column
+  const int row0 = blockIdx.x * kTrainRows;
+  const size_t B = (size_t)t.batch;
+  if (threadIdx.x < kTrainRows) {
+    const uint64_t i = (uint64_t)(row0 + (int)threadIdx.x);
+    // (total 0: the batch's rows as they are)
+    const uint64_t src =
+        t.total ? mix64(t.seed ^ mix64(t.step * 0x9e3779b97f4a7c15ull + i)) % t.total : i;
+    s_src[threadIdx.x] = src;
+    s_y[threadIdx.x] = t.Y[src];
   }
-  Yb[i] = Y[src];
+  bf16x8 w1f[2], w2f[kMlpHidden / 16];
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+    w1f[s] = *reinterpret_cast<const bf16x8*>(t.W1 + (size_t)n * kMlpIn + 16 * s + kh);
+#pragma unroll
+  for (int s = 0; s < kMlpHidden / 16; ++s)
+    w2f[s] = *reinterpret_cast<const bf16x8*>(t.W2 + (size_t)n * kMlpHidden + 16 * s + kh);
+  const float bias1 = t.b1[n], bias2 = t.b2[n], wn = bf2f(t.w3[n]), bias3 = *t.b3;
+  __syncthreads();
+  bf16x8 xa[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+    xa[s] = *reinterpret_cast<const bf16x8*>(t.X + s_src[lr] * kMlpIn + 16 * s + kh);
+  if (wave == 0) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const __bf16 x = xa[s][k];
+        t.Xt[(size_t)(16 * s + kh + k) * B + row0 + lr] = __builtin_bit_cast(uint16_t, x);
+      }
+  }
+  // layer 1
+  floatx16 acc = {};
+#pragma unroll
+  for (int s = 0; s < 2; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[s], w1f[s], acc, 0, 0, 0);
+  uint16_t h[16];
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int m = 8 * (v / 4) + 4 * hi + (v % 4);
+    float x = acc[v] + bias1;
+    x = x > 0.0f ? x : 0.0f;
+    h[v] = f2bf(x);
+    s_h[m * kTrainStride + n] = h[v];
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    store4(t.H1t + (size_t)n * B + row0 + 8 * q + 4 * hi, h[4 * q], h[4 * q + 1], h[4 * q + 2], h[4 * q + 3]);
+  __syncthreads();
+  // layer 2
+  acc = floatx16{};
+#pragma unroll
+  for (int s = 0; s < kMlpHidden / 16; ++s) {
+    const bf16x8 a = *reinterpret_cast<const bf16x8*>(s_h + lr * kTrainStride + 16 * s + kh);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, w2f[s], acc, 0, 0, 0);
+  }
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int m = 8 * (v / 4) + 4 * hi + (v % 4);
+    float x = acc[v] + bias2;
+    x = x > 0.0f ? x : 0.0f;
+    h[v] = f2bf(x);
+    s_part[m * kTrainPart + n] = bf2f(h[v]) * wn;
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    store4(t.H2t + (size_t)n * B + row0 + 8 * q + 4 * hi, h[4 * q], h[4 * q + 1], h[4 * q + 2], h[4 * q + 3]);
+  __syncthreads();
+  // logits, loss and its gradient: wave w takes rows w, w + 8, ...; lane l
+  // adds columns l, l + 64, l + 128, l + 192, then a butterfly
+#pragma unroll
+  for (int q = 0; q < kTrainRows / (kTrainThreads / 64); ++q) {
+    const int m = wave + q * (kTrainThreads / 64);
+    float sum = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kMlpHidden; k += 64) sum += s_part[m * kTrainPart + k + lane];
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+    if (lane == 0) {
+      const float z = sum + bias3;
+      const float y = s_y[m] ? 1.0f : 0.0f;
+      const float w = s_y[m] ? t.pos_weight : 1.0f;
+      const float sig = 1.0f / (1.0f + expf(-z));
+      const float d = w * (sig - y) / (float)t.batch;
+      s_dl[m] = d;
+      t.dl[row0 + m] = d;
+      t.loss[row0 + m] = w * (log1pf(expf(-fabsf(z))) + fmaxf(z, 0.0f) - z * y);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int m = 8 * (v / 4) + 4 * hi + (v % 4);
+    h[v] = bf2f(h[v]) > 0.0f ? f2bf(s_dl[m] * wn) : (uint16_t)0;
+    s_h[m * kTrainStride + n] = h[v];
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    store4(t.dH2t + (size_t)n * B + row0 + 8 * q + 4 * hi, h[4 * q], h[4 * q + 1], h[4 * q + 2], h[4 * q + 3]);
+  __syncthreads();
+  // dH2 by rows, 32 bytes a thread
+  static_assert(kTrainThreads * 16 == kTrainRows * kMlpHidden, "one pass");
+  const int row = threadIdx.x / (kMlpHidden / 16), col = threadIdx.x % (kMlpHidden / 16) * 16;
+  const uint4* src = reinterpret_cast<const uint4*>(s_h + row * kTrainStride + col);
+  uint4* dst = reinterpret_cast<uint4*>(t.dH2 + (size_t)(row0 + row) * kMlpHidden + col);
+  dst[0] = src[0];
+  dst[1] = src[1];
+}
+
+// One wave per workgroup; by workgroup index: the 64 tiles of dW2 (the
+// longest chains, first), the row sums for w3 and b2, the sums for b3 and the
+// loss, then the tiles of dH1.
+constexpr int kDw2Tiles = kMlpHidden / 32 * (kMlpHidden / 32);
+
+__global__ __launch_bounds__(64) void k_train_grads(TrainArgs t) {
+  const int lane = threadIdx.x;
+  const size_t B = (size_t)t.batch;
+  int i = (int)blockIdx.x;
+  if (i < kDw2Tiles) {
+    const int m0 = i / (kMlpHidden / 32) * 32, n0 = i % (kMlpHidden / 32) * 32;
+    store_tile(tile_product(t.dH2t, B, t.H1t, B, t.batch, m0, n0, lane), t.gW2, kMlpHidden, m0, n0, lane);
+    return;
+  }
+  i -= kDw2Tiles;
+  if (i < 2 * kMlpHidden) {
+    const bool w3 = i < kMlpHidden;
+    const int j = w3 ? i : i - kMlpHidden;
+    const float s = w3 ? row_sum(t.H2t + j * B, t.dl, t.batch, lane)
+                       : row_sum(t.dH2t + j * B, nullptr, t.batch, lane);
+    if (lane == 0) (w3 ? t.gw3 : t.gb2)[j] = s;
+    return;
+  }
+  i -= 2 * kMlpHidden;
+  if (i < 2) {
+    const float s = quarter_sums(i ? t.dl : t.loss, t.batch, lane);
+    if (lane == 0) *(i ? t.gb3 : t.loss_sum) = s;
+    return;
+  }
+  i -= 2;
+  const int m0 = i / (kMlpHidden / 32) * 32, n0 = i % (kMlpHidden / 32) * 32;
+  const floatx16 acc = tile_product(t.dH2, kMlpHidden, t.W2t, kMlpHidden, kMlpHidden, m0, n0, lane);
+  const size_t at = (size_t)(n0 + (lane & 31)) * B + m0 + 4 * (lane >> 5);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const uint2 mask = *reinterpret_cast<const uint2*>(t.H1t + at + 8 * q);
+    uint16_t d[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const uint16_t hm = (uint16_t)((k < 2 ? mask.x : mask.y) >> (16 * (k & 1)));
+      d[k] = f2bf(bf2f(hm) > 0.0f ? acc[4 * q + k] : 0.0f);
+    }
+    store4(t.dH1t + at + 8 * q, d[0], d[1], d[2], d[3]);
+  }
+}
+
+// the 8 tiles of dW1, then the row sums for b1
+__global__ __launch_bounds__(64) void k_train_grads1(TrainArgs t) {
+  const int lane = threadIdx.x;
+  const size_t B = (size_t)t.batch;
+  const int i = (int)blockIdx.x;
+  if (i < kMlpHidden / 32) {
+    store_tile(tile_product(t.dH1t, B, t.Xt, B, t.batch, 32 * i, 0, lane), t.gW1, kMlpIn, 32 * i, 0, lane);
+    return;
+  }
+  const int j = i - kMlpHidden / 32;
+  const float s = row_sum(t.dH1t + j * B, nullptr, t.batch, lane);
+  if (lane == 0) t.gb1[j] = s;
 }
 
 // float -> bf16 conversion (weights after the optimiser step), optionally
@@ -198,74 +349,40 @@ __global__ __launch_bounds__(256) void k_to_bf16(const float* __restrict__ in, s
   if (out_t) out_t[(i % cols) * rows + i / cols] = b;
 }
 
-// Adam (Kingma & Ba 2015) on fp32 master weights; bc1/bc2 = bias corrections
-__global__ __launch_bounds__(256) void k_adam(float* __restrict__ w, const float* __restrict__ g,
-                                              float* __restrict__ m, float* __restrict__ v,
-                                              size_t n, float lr, float b1, float b2, float eps,
-                                              float bc1, float bc2) {
+// Adam (Kingma & Ba 2015) on fp32 master weights; bc1/bc2 = bias corrections.
+// Writes the new weights' bf16 copies as well.
+__global__ __launch_bounds__(256) void k_adam(AdamArgs a) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.0f - b1) * gi;
-  const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  w[i] -= lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
+  if (i >= a.n) return;
+  const float gi = a.g[i];
+  const float mi = a.b1 * a.m[i] + (1.0f - a.b1) * gi;
+  const float vi = a.b2 * a.v[i] + (1.0f - a.b2) * gi * gi;
+  a.m[i] = mi;
+  a.v[i] = vi;
+  const float w = a.w[i] - a.lr * (mi / a.bc1) / (sqrtf(vi / a.bc2) + a.eps);
+  a.w[i] = w;
+  const uint16_t b = f2bf(w);
+  if (i >= a.at_w1 && i < a.at_w1 + (size_t)kMlpHidden * kMlpIn) a.W1[i - a.at_w1] = b;
+  if (i >= a.at_w2 && i < a.at_w2 + (size_t)kMlpHidden * kMlpHidden) {
+    const size_t j = i - a.at_w2;
+    a.W2[j] = b;
+    a.W2t[j % kMlpHidden * kMlpHidden + j / kMlpHidden] = b;
+  }
+  if (i >= a.at_w3 && i < a.at_w3 + kMlpHidden) a.w3[i - a.at_w3] = b;
 }
 
 // ---- launchers --------------------------------------------------------------
 
 static unsigned blocks_for(size_t n) { return (unsigned)((n + 255) / 256); }
 
-hipError_t mlp_gemm(const GemmArgs& g, hipStream_t s) {
-  const int tiles = ((g.M + 31) / 32) * ((g.N + 31) / 32);
-  if (tiles == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_gemm_nt, dim3((tiles + 3) / 4), dim3(256), 0, s, g);
-  return hipGetLastError();
-}
-
-hipError_t mlp_last_layer(const uint16_t* H2, const uint16_t* w3, const float* b3, float* logits,
-                          int rows, const uint32_t* rows_dev, hipStream_t s) {
-  if (rows == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_last_layer, dim3((rows + 3) / 4), dim3(256), 0, s, H2, w3, b3, logits, rows,
-                     rows_dev);
-  return hipGetLastError();
-}
-
-hipError_t mlp_head(const float* logits, const uint8_t* labels, float pos_weight, int rows,
-                    float* dl, float* loss, hipStream_t s) {
-  if (rows == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_head, dim3(blocks_for(rows)), dim3(256), 0, s, logits, labels, pos_weight,
-                     rows, dl, loss);
-  return hipGetLastError();
-}
-
-hipError_t mlp_dh2(const uint16_t* H2, const uint16_t* H2t, const float* dl, const uint16_t* w3,
-                   int rows, uint16_t* dH2, uint16_t* dH2t, hipStream_t s) {
-  if (rows == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_dh2, dim3(blocks_for(2 * (size_t)rows * kMlpHidden)), dim3(256), 0, s, H2,
-                     H2t, dl, w3, rows, dH2, dH2t);
-  return hipGetLastError();
-}
-
-hipError_t mlp_row_sums(const uint16_t* Mt, const float* w, int n, int rows, float* out,
-                        hipStream_t s) {
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_row_sums, dim3((n + 3) / 4), dim3(256), 0, s, Mt, w, n, rows, out);
-  return hipGetLastError();
-}
-
-hipError_t mlp_sum(const float* v, int n, float* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_sum, dim3(1), dim3(256), 0, s, v, n, out);
-  return hipGetLastError();
-}
-
-hipError_t mlp_gather(const uint16_t* X, const uint8_t* Y, uint64_t total, uint64_t seed,
-                      uint64_t step, int batch, uint16_t* Xb, uint16_t* Xbt, uint8_t* Yb,
-                      hipStream_t s) {
-  if (batch == 0 || total == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_gather, dim3(blocks_for(batch)), dim3(256), 0, s, X, Y, total, seed, step,
-                     batch, Xb, Xbt, Yb);
+hipError_t mlp_train(const TrainArgs& t, hipStream_t s) {
+  // the batch is a multiple of 32 rows (checked by the callers)
+  if (t.batch < kTrainRows || t.batch % kTrainRows) return hipErrorInvalidValue;
+  const unsigned row_tiles = (unsigned)(t.batch / kTrainRows);
+  hipLaunchKernelGGL(k_train_forward, dim3(row_tiles), dim3(kTrainThreads), 0, s, t);
+  hipLaunchKernelGGL(k_train_grads, dim3(kDw2Tiles + 2 * kMlpHidden + 2 + row_tiles * (kMlpHidden / 32)),
+                     dim3(64), 0, s, t);
+  hipLaunchKernelGGL(k_train_grads1, dim3(kMlpHidden / 32 + kMlpHidden), dim3(64), 0, s, t);
   return hipGetLastError();
 }
 
@@ -276,11 +393,9 @@ hipError_t mlp_to_bf16(const float* in, size_t n, uint16_t* out, uint16_t* out_t
   return hipGetLastError();
 }
 
-hipError_t mlp_adam(float* w, const float* g, float* m, float* v, size_t n, float lr, float b1,
-                    float b2, float eps, float bc1, float bc2, hipStream_t s) {
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_adam, dim3(blocks_for(n)), dim3(256), 0, s, w, g, m, v, n, lr, b1, b2, eps,
-                     bc1, bc2);
+hipError_t mlp_adam(const AdamArgs& a, hipStream_t s) {
+  if (a.n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_adam, dim3(blocks_for(a.n)), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
@@ -297,9 +412,9 @@ namespace gbr {
 // v_mfma_f32_32x32x16_bf16) -> bias, ReLU, bf16 -> the tile's H1 in LDS;
 // layer 2 (K = 256, 16 MFMAs, A fragments from LDS) -> bias, ReLU, bf16,
 // times w3 -> per-column products in LDS; then each row's logit is summed in
-// k_last_layer's order (lane l: columns l, l+64, l+128, l+192, then a
-// butterfly over 64 lanes).  The K loops run k = 0, 16, ... like k_gemm_nt,
-// so H1, H2 and the logits equal the training forward's bit for bit.
+// k_train_forward's order (lane l: columns l, l+64, l+128, l+192, then a
+// butterfly over 64 lanes).  The K loops run k = 0, 16, ... like its own, so
+// H1, H2 and the logits equal the training forward's bit for bit.
 // --------------------------------------------------------------------------
 
 constexpr int kScoreRows = 32;                  // rows per tile
@@ -379,7 +494,7 @@ __global__ __launch_bounds__(kScoreThreads) void k_mlp_score(const uint16_t* __r
       s_part[m * kPartStride + n] = bf2f(f2bf(x)) * wn;
     }
     __syncthreads();  // products complete; H1 may be rewritten
-    // logits: wave w sums rows w, w + 8, ... in k_last_layer's order
+    // logits: wave w sums rows w, w + 8, ... in k_train_forward's order
 #pragma unroll
     for (int q = 0; q < kScoreRows / kScoreWaves; ++q) {
       const int m = wave + q * kScoreWaves;

@@ -22,24 +22,12 @@ uint16_t host_f2bf(float f) {
   return (uint16_t)(u >> 16);
 }
 
-GemmArgs gemm(const uint16_t* A, int lda, const uint16_t* Bt, int ldb, int M, int N, int K) {
-  GemmArgs g;
-  g.A = A;
-  g.lda = lda;
-  g.Bt = Bt;
-  g.ldb = ldb;
-  g.M = M;
-  g.N = N;
-  g.K = K;
-  return g;
-}
-
 }  // namespace
 
 void VisModel::release() {
-  for (DevBuf<float>* b : {&w, &g, &m, &v, &logits, &dl, &lossr, &red, &logits_i}) b->release();
-  for (DevBuf<uint16_t>* b : {&W1b, &W2b, &W2tb, &w3b, &Xd, &Xb, &Xbt, &H1, &H1t, &H2, &H2t, &dH2,
-                              &dH2t, &dH1, &dH1t, &Xi})
+  for (DevBuf<float>* b : {&w, &g, &m, &v, &logits, &dl, &lossr, &losses, &logits_i}) b->release();
+  for (DevBuf<uint16_t>* b : {&W1b, &W2b, &W2tb, &w3b, &Xd, &Xb, &Xbt, &H1t, &H2t, &dH2, &dH2t,
+                              &dH1t, &Xi})
     b->release();
   Yd.release();
   Yb.release();
@@ -128,39 +116,13 @@ gbr_status VisModel::reserve_batch(int batch) {
   const size_t b = (size_t)batch;
   TRY(Xb.reserve(b * kMlpIn));
   TRY(Xbt.reserve(b * kMlpIn));
-  for (DevBuf<uint16_t>* x : {&H1, &H1t, &H2, &H2t, &dH2, &dH2t, &dH1, &dH1t})
+  for (DevBuf<uint16_t>* x : {&H1t, &H2t, &dH2, &dH2t, &dH1t})
     TRY(x->reserve(b * kMlpHidden));
   TRY(Yb.reserve(b));
   TRY(logits.reserve(b));
   TRY(dl.reserve(b));
   TRY(lossr.reserve(b));
-  TRY(red.reserve(4));
   bcap = batch;
-  return GBR_OK;
-}
-
-gbr_status VisModel::forward(const uint16_t* X, int nrows, const uint32_t* rows_dev,
-                             uint16_t* H1o, uint16_t* H1to, uint16_t* H2o, uint16_t* H2to,
-                             float* out, hipStream_t s) {
-  GemmArgs g1 = gemm(X, kMlpIn, W1b.ptr, kMlpIn, nrows, kMlpHidden, kMlpIn);
-  g1.M_dev = rows_dev;
-  g1.bias = w.ptr + kVisB1;
-  g1.relu = 1;
-  g1.D = H1o;
-  g1.ldd = kMlpHidden;
-  g1.Dt = H1to;
-  g1.lddt = nrows;
-  HIP_TRY(mlp_gemm(g1, s));
-  GemmArgs g2 = gemm(H1o, kMlpHidden, W2b.ptr, kMlpHidden, nrows, kMlpHidden, kMlpHidden);
-  g2.M_dev = rows_dev;
-  g2.bias = w.ptr + kVisB2;
-  g2.relu = 1;
-  g2.D = H2o;
-  g2.ldd = kMlpHidden;
-  g2.Dt = H2to;
-  g2.lddt = nrows;
-  HIP_TRY(mlp_gemm(g2, s));
-  HIP_TRY(mlp_last_layer(H2o, w3b.ptr, w.ptr + kVisB3, out, nrows, rows_dev, s));
   return GBR_OK;
 }
 
@@ -171,46 +133,68 @@ gbr_status VisModel::score(const uint16_t* X, int nrows, const uint32_t* rows_de
   return GBR_OK;
 }
 
-// gradients of the mean weighted loss over the batch in Xb/Xbt/Yb; the loss
-// lands in red[0]
-gbr_status VisModel::backward(int b, float pos_weight, hipStream_t s) {
-  TRY(forward(Xb.ptr, b, nullptr, H1.ptr, H1t.ptr, H2.ptr, H2t.ptr, logits.ptr, s));
-  HIP_TRY(mlp_head(logits.ptr, Yb.ptr, pos_weight, b, dl.ptr, lossr.ptr, s));
-  HIP_TRY(mlp_sum(lossr.ptr, b, red.ptr, s));
-  HIP_TRY(mlp_sum(dl.ptr, b, g.ptr + kVisB3, s));
-  HIP_TRY(mlp_row_sums(H2t.ptr, dl.ptr, kMlpHidden, b, g.ptr + kVisW3, s));
-  HIP_TRY(mlp_dh2(H2.ptr, H2t.ptr, dl.ptr, w3b.ptr, b, dH2.ptr, dH2t.ptr, s));
-  // dW2 = dH2^T H1
-  GemmArgs gw2 = gemm(dH2t.ptr, b, H1t.ptr, b, kMlpHidden, kMlpHidden, b);
-  gw2.C = g.ptr + kVisW2;
-  gw2.ldc = kMlpHidden;
-  HIP_TRY(mlp_gemm(gw2, s));
-  HIP_TRY(mlp_row_sums(dH2t.ptr, nullptr, kMlpHidden, b, g.ptr + kVisB2, s));
-  // dH1 = (dH2 W2) o [H1 > 0]
-  GemmArgs gh1 = gemm(dH2.ptr, kMlpHidden, W2tb.ptr, kMlpHidden, b, kMlpHidden, kMlpHidden);
-  gh1.mask = H1.ptr;
-  gh1.ldmask = kMlpHidden;
-  gh1.D = dH1.ptr;
-  gh1.ldd = kMlpHidden;
-  gh1.Dt = dH1t.ptr;
-  gh1.lddt = b;
-  HIP_TRY(mlp_gemm(gh1, s));
-  // dW1 = dH1^T X
-  GemmArgs gw1 = gemm(dH1t.ptr, b, Xbt.ptr, b, kMlpHidden, kMlpIn, b);
-  gw1.C = g.ptr + kVisW1;
-  gw1.ldc = kMlpIn;
-  HIP_TRY(mlp_gemm(gw1, s));
-  HIP_TRY(mlp_row_sums(dH1t.ptr, nullptr, kMlpHidden, b, g.ptr + kVisB1, s));
+// gradients of the mean weighted loss over a batch of rows of X, Y (hashed by
+// seed and step out of `total` rows, or the first `b` with total 0); the
+// batch's loss lands in *loss_sum
+gbr_status VisModel::backward(const uint16_t* X, const uint8_t* Y, uint64_t total, uint64_t seed,
+                              uint64_t step, int b, float pos_weight, float* loss_sum, hipStream_t s) {
+  TrainArgs t{};
+  t.batch = b;
+  t.X = X;
+  t.Y = Y;
+  t.total = total;
+  t.seed = seed;
+  t.step = step;
+  t.pos_weight = pos_weight;
+  t.W1 = W1b.ptr;
+  t.W2 = W2b.ptr;
+  t.W2t = W2tb.ptr;
+  t.w3 = w3b.ptr;
+  t.b1 = w.ptr + kVisB1;
+  t.b2 = w.ptr + kVisB2;
+  t.b3 = w.ptr + kVisB3;
+  t.Xt = Xbt.ptr;
+  t.H1t = H1t.ptr;
+  t.H2t = H2t.ptr;
+  t.dH2t = dH2t.ptr;
+  t.dH1t = dH1t.ptr;
+  t.dH2 = dH2.ptr;
+  t.dl = dl.ptr;
+  t.loss = lossr.ptr;
+  t.gW1 = g.ptr + kVisW1;
+  t.gb1 = g.ptr + kVisB1;
+  t.gW2 = g.ptr + kVisW2;
+  t.gb2 = g.ptr + kVisB2;
+  t.gw3 = g.ptr + kVisW3;
+  t.gb3 = g.ptr + kVisB3;
+  t.loss_sum = loss_sum;
+  HIP_TRY(mlp_train(t, s));
   return GBR_OK;
 }
 
 gbr_status VisModel::adam_step(const gbr_vis_fit_params& fp, hipStream_t s) {
   ++adam_t;
-  const float bc1 = 1.0f - std::pow(fp.beta1, (float)adam_t);
-  const float bc2 = 1.0f - std::pow(fp.beta2, (float)adam_t);
-  HIP_TRY(mlp_adam(w.ptr, g.ptr, m.ptr, v.ptr, kVisParams, fp.learning_rate, fp.beta1, fp.beta2,
-                   fp.eps, bc1, bc2, s));
-  return refresh_bf16(s);
+  AdamArgs a{};
+  a.w = w.ptr;
+  a.g = g.ptr;
+  a.m = m.ptr;
+  a.v = v.ptr;
+  a.n = kVisParams;
+  a.lr = fp.learning_rate;
+  a.b1 = fp.beta1;
+  a.b2 = fp.beta2;
+  a.eps = fp.eps;
+  a.bc1 = 1.0f - std::pow(fp.beta1, (float)adam_t);
+  a.bc2 = 1.0f - std::pow(fp.beta2, (float)adam_t);
+  a.at_w1 = kVisW1;
+  a.at_w2 = kVisW2;
+  a.at_w3 = kVisW3;
+  a.W1 = W1b.ptr;
+  a.W2 = W2b.ptr;
+  a.W2t = W2tb.ptr;
+  a.w3 = w3b.ptr;
+  HIP_TRY(mlp_adam(a, s));
+  return GBR_OK;
 }
 
 gbr_status VisModel::fit(const gbr_vis_fit_params& fp, gbr_vis_fit_report* rep, hipStream_t s) {
@@ -219,27 +203,22 @@ gbr_status VisModel::fit(const gbr_vis_fit_params& fp, gbr_vis_fit_report* rep, 
   if (fp.steps < 1 || fp.batch < 32 || fp.batch > 65536 || fp.batch % 32)
     return fail(GBR_ERR_ARGUMENT, "vis_fit: steps >= 1 and batch a multiple of 32 in [32, 65536]");
   TRY(reserve_batch(fp.batch));
-  std::vector<float> losses((size_t)fp.steps, 0.0f);
-  DevBuf<float> dloss;
-  TRY(dloss.reserve((size_t)fp.steps));
+  std::vector<float> sums((size_t)fp.steps, 0.0f);
+  TRY(losses.reserve((size_t)fp.steps));
   for (int k = 0; k < fp.steps; ++k) {
-    HIP_TRY(mlp_gather(Xd.ptr, Yd.ptr, rows, fp.seed, (uint64_t)k, fp.batch, Xb.ptr, Xbt.ptr,
-                       Yb.ptr, s));
-    TRY(backward(fp.batch, fp.pos_weight, s));
-    HIP_TRY(hipMemcpyAsync(dloss.ptr + k, red.ptr, sizeof(float), hipMemcpyDeviceToDevice, s));
+    TRY(backward(Xd.ptr, Yd.ptr, rows, fp.seed, (uint64_t)k, fp.batch, fp.pos_weight, losses.ptr + k, s));
     TRY(adam_step(fp, s));
   }
-  HIP_TRY(hipMemcpyAsync(losses.data(), dloss.ptr, losses.size() * sizeof(float),
+  HIP_TRY(hipMemcpyAsync(sums.data(), losses.ptr, sums.size() * sizeof(float),
                          hipMemcpyDeviceToHost, s));
   uint32_t pos = 0;
   HIP_TRY(hipMemcpyAsync(&pos, positives.ptr, sizeof pos, hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
-  dloss.release();
   if (rep) {
-    rep->loss_first = losses[0] / (float)fp.batch;
+    rep->loss_first = sums[0] / (float)fp.batch;
     const int tail = std::max(1, fp.steps / 10);
     double t = 0.0;
-    for (int k = fp.steps - tail; k < fp.steps; ++k) t += losses[(size_t)k];
+    for (int k = fp.steps - tail; k < fp.steps; ++k) t += sums[(size_t)k];
     rep->loss_last = (float)(t / tail / fp.batch);
     rep->rows = rows;
     rep->positives = pos;
@@ -253,19 +232,14 @@ gbr_status VisModel::loss_grad(const float* X, const uint8_t* labels, int n, flo
   if (n < 32 || n > 65536 || n % 32)
     return fail(GBR_ERR_ARGUMENT, "vis_loss_grad: rows must be a multiple of 32 in [32, 65536]");
   TRY(reserve_batch(n));
-  std::vector<uint16_t> xb((size_t)n * kMlpIn), xbt((size_t)n * kMlpIn);
-  for (int r = 0; r < n; ++r)
-    for (int k = 0; k < kMlpIn; ++k) {
-      const uint16_t b = host_f2bf(X[(size_t)r * kMlpIn + k]);
-      xb[(size_t)r * kMlpIn + k] = b;
-      xbt[(size_t)k * n + r] = b;
-    }
+  TRY(losses.reserve(1));
+  std::vector<uint16_t> xb((size_t)n * kMlpIn);
+  for (size_t i = 0; i < xb.size(); ++i) xb[i] = host_f2bf(X[i]);
   HIP_TRY(hipMemcpyAsync(Xb.ptr, xb.data(), xb.size() * 2, hipMemcpyHostToDevice, s));
-  HIP_TRY(hipMemcpyAsync(Xbt.ptr, xbt.data(), xbt.size() * 2, hipMemcpyHostToDevice, s));
   HIP_TRY(hipMemcpyAsync(Yb.ptr, labels, (size_t)n, hipMemcpyHostToDevice, s));
-  TRY(backward(n, pos_weight, s));
+  TRY(backward(Xb.ptr, Yb.ptr, 0, 0, 0, n, pos_weight, losses.ptr, s));
   float l = 0.0f;
-  HIP_TRY(hipMemcpyAsync(&l, red.ptr, sizeof l, hipMemcpyDeviceToHost, s));
+  HIP_TRY(hipMemcpyAsync(&l, losses.ptr, sizeof l, hipMemcpyDeviceToHost, s));
   HIP_TRY(hipMemcpyAsync(grad, g.ptr, kVisParams * sizeof(float), hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
   *loss = l / (float)n;

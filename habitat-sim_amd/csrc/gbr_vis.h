@@ -35,9 +35,10 @@ struct VisModel {
 
   // minibatch scratch
   int bcap = 0;
-  DevBuf<uint16_t> Xb, Xbt, H1, H1t, H2, H2t, dH2, dH2t, dH1, dH1t;
+  DevBuf<uint16_t> Xb, Xbt, H1t, H2t, dH2, dH2t, dH1t;
   DevBuf<uint8_t> Yb;
-  DevBuf<float> logits, dl, lossr, red;
+  DevBuf<float> logits, dl, lossr;
+  DevBuf<float> losses;  // summed loss of each step of a fit
 
   // per-frame inference scratch (rows = candidate work items)
   DevBuf<uint16_t> Xi;
@@ -49,14 +50,12 @@ struct VisModel {
   gbr_status get_weights(float* host, hipStream_t s);
   gbr_status reserve_dataset(uint64_t rows_cap);
   gbr_status reserve_infer(size_t rows);
-  // forward over rows [0, min(rows, *rows_dev)) of X into logits
-  gbr_status forward(const uint16_t* X, int rows, const uint32_t* rows_dev, uint16_t* H1o,
-                     uint16_t* H1to, uint16_t* H2o, uint16_t* H2to, float* out, hipStream_t s);
   // rendering: logits of rows [0, min(rows, *rows_dev)) of X, fused
   gbr_status score(const uint16_t* X, int rows, const uint32_t* rows_dev, float* out,
                    int max_blocks, hipStream_t s);
-  // loss and gradients (into g) of the batch already in Xb/Xbt/Yb
-  gbr_status backward(int batch, float pos_weight, hipStream_t s);
+  // loss and gradients (into g) of a batch of rows
+  gbr_status backward(const uint16_t* X, const uint8_t* Y, uint64_t total, uint64_t seed,
+                      uint64_t step, int batch, float pos_weight, float* loss_sum, hipStream_t s);
   gbr_status adam_step(const gbr_vis_fit_params& fp, hipStream_t s);
   gbr_status refresh_bf16(hipStream_t s);
   gbr_status fit(const gbr_vis_fit_params& fp, gbr_vis_fit_report* rep, hipStream_t s);
