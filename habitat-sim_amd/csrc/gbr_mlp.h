@@ -21,8 +21,9 @@ struct TrainArgs {
   // weights
   const uint16_t *W1, *W2, *W2t, *w3;
   const float *b1, *b2, *b3;
-  // scratch: X, H1, H2, dH2, dH1 transposed ([column][batch]), dH2, and per row
-  // the loss and its gradient by the logit
+  // scratch: X, H1, H2, dH2, dH1 in fragment order ([columns][batch] values;
+  // frag_at() in gbr_mlp.hip), dH2 by rows, and per row the loss and its
+  // gradient by the logit
   uint16_t *Xt, *H1t, *H2t, *dH2t, *dH1t, *dH2;
   float *dl, *loss;
   // gradients of the mean weighted loss, and the loss summed over the batch

@@ -9,9 +9,8 @@
 //                    the batch for w3, b2, b3 and the loss
 //   k_train_grads1   dW1 = dH1^T X and the sums for b1
 //   k_adam           the weights, and their bf16 copies
-// Every product is an "NT" one, C[M][N] = sum_k A[M][K] * Bt[N][K], with both
-// operands K-contiguous so that a wave's MFMA fragments are single 16-byte
-// loads.  The sums are reductions with one writer per output (no atomics),
+// Every product is an "NT" one, C[M][N] = sum_k A[M][K] * Bt[N][K], with the
+// eight k of an MFMA fragment's lane contiguous in both operands.  The sums are reductions with one writer per output (no atomics),
 // and every sum runs in a fixed order, whatever the launch geometry.
 #include <hip/hip_runtime.h>
 
@@ -46,33 +45,41 @@ __device__ __forceinline__ void store4(uint16_t* dst, uint16_t a, uint16_t b, ui
       make_uint2((uint32_t)a | ((uint32_t)b << 16), (uint32_t)c | ((uint32_t)d << 16));
 }
 
+// The batch matrices that a weight gradient contracts over the batch (X, H1,
+// dH2, dH1 transposed) are kept in the order of MFMA fragments: for 32
+// columns and 16 rows of the batch, lane l's eight values (column l%32, rows
+// 8*(l/32) .. +8) one after the other, so that a wave's fragment is 1 KB in a
+// row.  (As [column][batch] rows a load gathered 64 pieces of 16 bytes: with 32
+// steps ahead k_train_grads took 21.5 us at 4096 rows, and takes 14.1 so; with 16
+// ahead 24.9 and 17.2.)
+__device__ __forceinline__ size_t frag_at(int column, int row, int batch) {
+  return (((size_t)(column >> 5) * (size_t)(batch >> 4) + (size_t)(row >> 4)) * 64 +
+          (size_t)((column & 31) + 32 * ((row >> 3) & 1))) * 8 + (size_t)(row & 7);
+}
+
 // --------------------------------------------------------------------------
 // One 32x32 tile of an NT product by one wave (v_mfma_f32_32x32x16_bf16):
-// lane l supplies A[m0 + l%32][k + 8*(l/32) .. +8] and Bt[n0 + l%32][same k];
+// lane l supplies A[m0 + l%32][k + 8*(l/32) .. +8] and Bt[n0 + l%32][same k],
+// at ap and bp for k = 0 and a_step, b_step elements further per 16 k;
 // accumulator v holds C[m0 + 8*(v/4) + 4*(l/32) + v%4][n0 + l%32].  The K
 // steps run in order, k = 0, 16, ...
 //
 // A weight gradient is a chain of K / 16 = 256 such steps (4096 rows) in 64
 // waves, so what bounds it is the latency of the fragments' loads: kAhead
-// steps' fragments are in flight at any time (128 registers), 68 us down to
-// 9 for dW2 at 4096 rows against one step's loads at a time.
-// Requirements (the callers'): K % 16 == 0, rows of 16-byte alignment.
+// steps' fragments are in flight at any time.  One wave a SIMD is all there is
+// to run, so they may take 256 registers (16 steps: 17.2 us; 32: 14.1).
 // --------------------------------------------------------------------------
-constexpr int kAhead = 16;
+constexpr int kAhead = 32;
 
-__device__ __forceinline__ floatx16 tile_product(const uint16_t* __restrict__ A, size_t lda,
-                                                 const uint16_t* __restrict__ Bt, size_t ldb, int K,
-                                                 int m0, int n0, int lane) {
-  const int kofs = 8 * (lane >> 5);
-  const uint16_t* ap = A + (size_t)(m0 + (lane & 31)) * lda + kofs;
-  const uint16_t* bp = Bt + (size_t)(n0 + (lane & 31)) * ldb + kofs;
-  const int steps = K / 16;
+__device__ __forceinline__ floatx16 tile_product(const uint16_t* __restrict__ ap, size_t a_step,
+                                                 const uint16_t* __restrict__ bp, size_t b_step,
+                                                 int steps) {
   bf16x8 a[kAhead], b[kAhead];
 #pragma unroll
   for (int u = 0; u < kAhead; ++u)
     if (u < steps) {
-      a[u] = *reinterpret_cast<const bf16x8*>(ap + 16 * u);
-      b[u] = *reinterpret_cast<const bf16x8*>(bp + 16 * u);
+      a[u] = *reinterpret_cast<const bf16x8*>(ap + a_step * u);
+      b[u] = *reinterpret_cast<const bf16x8*>(bp + b_step * u);
     }
   floatx16 acc = {};
   int s0 = 0;
@@ -80,8 +87,8 @@ __device__ __forceinline__ floatx16 tile_product(const uint16_t* __restrict__ A,
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) {
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[u], b[u], acc, 0, 0, 0);
-      a[u] = *reinterpret_cast<const bf16x8*>(ap + 16 * (size_t)(s0 + u + kAhead));
-      b[u] = *reinterpret_cast<const bf16x8*>(bp + 16 * (size_t)(s0 + u + kAhead));
+      a[u] = *reinterpret_cast<const bf16x8*>(ap + a_step * (size_t)(s0 + u + kAhead));
+      b[u] = *reinterpret_cast<const bf16x8*>(bp + b_step * (size_t)(s0 + u + kAhead));
     }
   }
   for (; s0 < steps; s0 += kAhead) {
@@ -89,12 +96,21 @@ __device__ __forceinline__ floatx16 tile_product(const uint16_t* __restrict__ A,
     for (int u = 0; u < kAhead; ++u) {
       if (s0 + u < steps) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[u], b[u], acc, 0, 0, 0);
       if (s0 + u + kAhead < steps) {
-        a[u] = *reinterpret_cast<const bf16x8*>(ap + 16 * (size_t)(s0 + u + kAhead));
-        b[u] = *reinterpret_cast<const bf16x8*>(bp + 16 * (size_t)(s0 + u + kAhead));
+        a[u] = *reinterpret_cast<const bf16x8*>(ap + a_step * (size_t)(s0 + u + kAhead));
+        b[u] = *reinterpret_cast<const bf16x8*>(bp + b_step * (size_t)(s0 + u + kAhead));
       }
     }
   }
   return acc;
+}
+
+// the product over the batch of 32 columns m0 of A and 32 columns n0 of B,
+// both in fragment order
+__device__ __forceinline__ floatx16 batch_product(const uint16_t* __restrict__ A,
+                                                  const uint16_t* __restrict__ B, int m0, int n0,
+                                                  int batch, int lane) {
+  return tile_product(A + frag_at(m0, 0, batch) + 8 * lane, 512, B + frag_at(n0, 0, batch) + 8 * lane, 512,
+                      batch / 16);
 }
 
 __device__ __forceinline__ void store_tile(const floatx16& acc, float* __restrict__ C, int ldc, int m0,
@@ -105,24 +121,27 @@ __device__ __forceinline__ void store_tile(const floatx16& acc, float* __restric
     C[(size_t)(m0 + 8 * (v / 4) + 4 * (lane >> 5) + v % 4) * ldc + n] = acc[v];
 }
 
-// sum_r row[r] * (w ? w[r] : 1) by one wave: lane l adds r = l, l + 64, ...,
-// then a butterfly (sixteen loads in flight at a time)
-__device__ __forceinline__ float row_sum(const uint16_t* __restrict__ row, const float* __restrict__ w,
-                                         int rows, int lane) {
+// sum_r M[column][r] * (w ? w[r] : 1) over the batch by one wave, M in fragment
+// order: lane l adds r = l, l + 64, ..., then a butterfly (sixteen loads in
+// flight at a time; 64 rows on are four fragments on)
+__device__ __forceinline__ float column_sum(const uint16_t* __restrict__ M, int column,
+                                            const float* __restrict__ w, int batch, int lane) {
+  const uint16_t* at = M + frag_at(column, lane, batch);
   float s = 0.0f;
   int r = lane;
-  for (; r - lane + 1024 <= rows; r += 1024) {
+  for (; r - lane + 1024 <= batch; r += 1024) {
     uint16_t x[16];
     float y[16];
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
-      x[q] = row[r + 64 * q];
+      x[q] = at[2048 * (size_t)q];
       y[q] = w ? w[r + 64 * q] : 1.0f;
     }
+    at += 2048 * 16;
 #pragma unroll
     for (int q = 0; q < 16; ++q) s += w ? bf2f(x[q]) * y[q] : bf2f(x[q]);
   }
-  for (; r < rows; r += 64) s += w ? bf2f(row[r]) * w[r] : bf2f(row[r]);
+  for (; r < batch; r += 64, at += 2048) s += w ? bf2f(*at) * w[r] : bf2f(*at);
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
   return s;
 }
@@ -158,8 +177,9 @@ constexpr int kTrainPart = kMlpHidden + 4;      // padded LDS row of fp32
 // gradients read: X, H1, H2 and dH2 transposed, and dH2.
 //   loss_r = w_r [log(1 + e^-|z|) + max(z, 0) - z y],  dl_r = w_r (sigmoid(z) - y) / rows
 // with w_r = pos_weight for visible rows, 1 otherwise; dH2 = [H2 > 0] dl[r] w3[k].
-// The arithmetic and its order are the scorer's (k_mlp_score).  As six
-// launches the same work took 105 us at 4096 rows; 128 workgroups here, 10 us.
+// The arithmetic and its order are the scorer's (k_mlp_score).  At 4096 rows it
+// is 128 workgroups, half the CUs, and takes 15 us, most of it the latency of
+// its loads, barriers and stores in turn.
 __global__ __launch_bounds__(kTrainThreads) void k_train_forward(TrainArgs t) {
   __shared__ uint16_t s_h[kTrainRows * kTrainStride];  // H1, then dH2
   __shared__ float s_part[kTrainRows * kTrainPart];
@@ -170,7 +190,6 @@ __global__ __launch_bounds__(kTrainThreads) void k_train_forward(TrainArgs t) {
   const int lr = lane & 31, kh = 8 * (lane >> 5), hi = lane >> 5;
   const int n = wave * 32 + lr;  // this lane's hidden column
   const int row0 = blockIdx.x * kTrainRows;
-  const size_t B = (size_t)t.batch;
   if (threadIdx.x < kTrainRows) {
     const uint64_t i = (uint64_t)(row0 + (int)threadIdx.x);
     // (total 0: the batch's rows as they are)
@@ -198,7 +217,7 @@ __global__ __launch_bounds__(kTrainThreads) void k_train_forward(TrainArgs t) {
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         const __bf16 x = xa[s][k];
-        t.Xt[(size_t)(16 * s + kh + k) * B + row0 + lr] = __builtin_bit_cast(uint16_t, x);
+        t.Xt[frag_at(16 * s + kh + k, row0 + lr, t.batch)] = __builtin_bit_cast(uint16_t, x);
       }
   }
   // layer 1
@@ -216,7 +235,7 @@ __global__ __launch_bounds__(kTrainThreads) void k_train_forward(TrainArgs t) {
   }
 #pragma unroll
   for (int q = 0; q < 4; ++q)
-    store4(t.H1t + (size_t)n * B + row0 + 8 * q + 4 * hi, h[4 * q], h[4 * q + 1], h[4 * q + 2], h[4 * q + 3]);
+    store4(t.H1t + frag_at(n, row0 + 8 * q + 4 * hi, t.batch), h[4 * q], h[4 * q + 1], h[4 * q + 2], h[4 * q + 3]);
   __syncthreads();
   // layer 2
   acc = floatx16{};
@@ -235,7 +254,7 @@ __global__ __launch_bounds__(kTrainThreads) void k_train_forward(TrainArgs t) {
   }
 #pragma unroll
   for (int q = 0; q < 4; ++q)
-    store4(t.H2t + (size_t)n * B + row0 + 8 * q + 4 * hi, h[4 * q], h[4 * q + 1], h[4 * q + 2], h[4 * q + 3]);
+    store4(t.H2t + frag_at(n, row0 + 8 * q + 4 * hi, t.batch), h[4 * q], h[4 * q + 1], h[4 * q + 2], h[4 * q + 3]);
   __syncthreads();
   // logits, loss and its gradient: wave w takes rows w, w + 8, ...; lane l
   // adds columns l, l + 64, l + 128, l + 192, then a butterfly
@@ -266,7 +285,7 @@ __global__ __launch_bounds__(kTrainThreads) void k_train_forward(TrainArgs t) {
   }
 #pragma unroll
   for (int q = 0; q < 4; ++q)
-    store4(t.dH2t + (size_t)n * B + row0 + 8 * q + 4 * hi, h[4 * q], h[4 * q + 1], h[4 * q + 2], h[4 * q + 3]);
+    store4(t.dH2t + frag_at(n, row0 + 8 * q + 4 * hi, t.batch), h[4 * q], h[4 * q + 1], h[4 * q + 2], h[4 * q + 3]);
   __syncthreads();
   // dH2 by rows, 32 bytes a thread
   static_assert(kTrainThreads * 16 == kTrainRows * kMlpHidden, "one pass");
@@ -278,25 +297,24 @@ __global__ __launch_bounds__(kTrainThreads) void k_train_forward(TrainArgs t) {
 }
 
 // One wave per workgroup; by workgroup index: the 64 tiles of dW2 (the
-// longest chains, first), the row sums for w3 and b2, the sums for b3 and the
+// longest chains, first), the column sums for w3 and b2, the sums for b3 and the
 // loss, then the tiles of dH1.
 constexpr int kDw2Tiles = kMlpHidden / 32 * (kMlpHidden / 32);
 
 __global__ __launch_bounds__(64) void k_train_grads(TrainArgs t) {
   const int lane = threadIdx.x;
-  const size_t B = (size_t)t.batch;
   int i = (int)blockIdx.x;
   if (i < kDw2Tiles) {
     const int m0 = i / (kMlpHidden / 32) * 32, n0 = i % (kMlpHidden / 32) * 32;
-    store_tile(tile_product(t.dH2t, B, t.H1t, B, t.batch, m0, n0, lane), t.gW2, kMlpHidden, m0, n0, lane);
+    store_tile(batch_product(t.dH2t, t.H1t, m0, n0, t.batch, lane), t.gW2, kMlpHidden, m0, n0, lane);
     return;
   }
   i -= kDw2Tiles;
   if (i < 2 * kMlpHidden) {
     const bool w3 = i < kMlpHidden;
     const int j = w3 ? i : i - kMlpHidden;
-    const float s = w3 ? row_sum(t.H2t + j * B, t.dl, t.batch, lane)
-                       : row_sum(t.dH2t + j * B, nullptr, t.batch, lane);
+    const float s = w3 ? column_sum(t.H2t, j, t.dl, t.batch, lane)
+                       : column_sum(t.dH2t, j, nullptr, t.batch, lane);
     if (lane == 0) (w3 ? t.gw3 : t.gb2)[j] = s;
     return;
   }
@@ -308,32 +326,34 @@ __global__ __launch_bounds__(64) void k_train_grads(TrainArgs t) {
   }
   i -= 2;
   const int m0 = i / (kMlpHidden / 32) * 32, n0 = i % (kMlpHidden / 32) * 32;
-  const floatx16 acc = tile_product(t.dH2, kMlpHidden, t.W2t, kMlpHidden, kMlpHidden, m0, n0, lane);
-  const size_t at = (size_t)(n0 + (lane & 31)) * B + m0 + 4 * (lane >> 5);
+  const int kofs = 8 * (lane >> 5);
+  const floatx16 acc = tile_product(t.dH2 + (size_t)(m0 + (lane & 31)) * kMlpHidden + kofs, 16,
+                                    t.W2t + (size_t)(n0 + (lane & 31)) * kMlpHidden + kofs, 16,
+                                    kMlpHidden / 16);
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const uint2 mask = *reinterpret_cast<const uint2*>(t.H1t + at + 8 * q);
+    const size_t at = frag_at(n0 + (lane & 31), m0 + 8 * q + 4 * (lane >> 5), t.batch);
+    const uint2 mask = *reinterpret_cast<const uint2*>(t.H1t + at);
     uint16_t d[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const uint16_t hm = (uint16_t)((k < 2 ? mask.x : mask.y) >> (16 * (k & 1)));
       d[k] = f2bf(bf2f(hm) > 0.0f ? acc[4 * q + k] : 0.0f);
     }
-    store4(t.dH1t + at + 8 * q, d[0], d[1], d[2], d[3]);
+    store4(t.dH1t + at, d[0], d[1], d[2], d[3]);
   }
 }
 
-// the 8 tiles of dW1, then the row sums for b1
+// the 8 tiles of dW1, then the column sums for b1
 __global__ __launch_bounds__(64) void k_train_grads1(TrainArgs t) {
   const int lane = threadIdx.x;
-  const size_t B = (size_t)t.batch;
   const int i = (int)blockIdx.x;
   if (i < kMlpHidden / 32) {
-    store_tile(tile_product(t.dH1t, B, t.Xt, B, t.batch, 32 * i, 0, lane), t.gW1, kMlpIn, 32 * i, 0, lane);
+    store_tile(batch_product(t.dH1t, t.Xt, 32 * i, 0, t.batch, lane), t.gW1, kMlpIn, 32 * i, 0, lane);
     return;
   }
   const int j = i - kMlpHidden / 32;
-  const float s = row_sum(t.dH1t + j * B, nullptr, t.batch, lane);
+  const float s = column_sum(t.dH1t, j, nullptr, t.batch, lane);
   if (lane == 0) t.gb1[j] = s;
 }
 

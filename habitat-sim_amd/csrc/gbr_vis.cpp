@@ -116,8 +116,7 @@ gbr_status VisModel::reserve_batch(int batch) {
   const size_t b = (size_t)batch;
   TRY(Xb.reserve(b * kMlpIn));
   TRY(Xbt.reserve(b * kMlpIn));
-  for (DevBuf<uint16_t>* x : {&H1t, &H2t, &dH2, &dH2t, &dH1t})
-    TRY(x->reserve(b * kMlpHidden));
+  for (DevBuf<uint16_t>* x : {&H1t, &H2t, &dH2t, &dH1t, &dH2}) TRY(x->reserve(b * kMlpHidden));
   TRY(Yb.reserve(b));
   TRY(logits.reserve(b));
   TRY(dl.reserve(b));
