@@ -1,0 +1,30 @@
+// Correctly rounded single-precision quotients in a few fused operations, for
+// operands whose range is known (device code only).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+namespace gbr {
+
+// 1 / x, correctly rounded, for 2^-126 <= |x| <= 2^126: the hardware
+// reciprocal (1 ulp) and one Newton step in fused arithmetic, three
+// instructions instead of the ten of the general division.  (Compared with
+// it over every float of that range.)
+__device__ __forceinline__ float rcp_exact(float x) {
+  const float r = __builtin_amdgcn_rcpf(x);
+  return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+}
+
+// a / b, correctly rounded, from r = rcp_exact(b), where a, b and a / b stay
+// within 2^+-60 (or a is 0): the quotient's remainder corrects it (Markstein
+// 1990)
+__device__ __forceinline__ float div_exact(float a, float b, float r) {
+  const float q = a * r;
+  return __builtin_fmaf(__builtin_fmaf(-b, q, a), r, q);
+}
+
+__device__ __forceinline__ bool in_range(float x, float lo, float hi) {
+  return __builtin_amdgcn_fmed3f(fabsf(x), lo, hi) == fabsf(x);
+}
+
+}  // namespace gbr

@@ -46,6 +46,7 @@
 
 #include "gbr.h"
 #include "gbr_device.h"
+#include "gbr_exact.h"
 
 #pragma clang fp contract(off)
 
@@ -116,27 +117,6 @@ __device__ __forceinline__ int local_tid() {
   int t = (int)threadIdx.x;
   asm volatile("" : "+v"(t));
   return t;
-}
-
-// 1 / x, correctly rounded, for 2^-126 <= |x| <= 2^126: the hardware
-// reciprocal (1 ulp) and one Newton step in fused arithmetic, three
-// instructions instead of the ten of the general division.  (Compared with
-// it over every float of that range.)
-__device__ __forceinline__ float rcp_exact(float x) {
-  const float r = __builtin_amdgcn_rcpf(x);
-  return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
-}
-
-// a / b, correctly rounded, from r = rcp_exact(b), where a, b and a / b stay
-// within 2^+-60 (or a is 0): the quotient's remainder corrects it (Markstein
-// 1990)
-__device__ __forceinline__ float div_exact(float a, float b, float r) {
-  const float q = a * r;
-  return __builtin_fmaf(__builtin_fmaf(-b, q, a), r, q);
-}
-
-__device__ __forceinline__ bool in_range(float x, float lo, float hi) {
-  return __builtin_amdgcn_fmed3f(fabsf(x), lo, hi) == fabsf(x);
 }
 
 struct Snap {

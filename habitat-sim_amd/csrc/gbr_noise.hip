@@ -11,17 +11,18 @@
 // model's seed as key, turned into normals by the Box-Muller transform.  A
 // counter generator needs no per-thread state in memory (the reference keeps
 // a curand state per thread) and makes every call reproducible from (seed,
-// call index).  The kernel is HBM-bound: 4 bytes read (the gathered depth
-// mostly hits the cache lines of its neighbours) and 4 written per pixel.
+// call index).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 #include <new>
 #include <string>
 
 #include "gbr.h"
+#include "gbr_exact.h"
 #include "gbr_host.h"
 
 #pragma STDC FP_CONTRACT OFF
@@ -36,12 +37,13 @@ __device__ __forceinline__ void philox4x32(uint32_t c0, uint32_t c1, uint32_t c2
                                            uint32_t k0, uint32_t k1, uint32_t* out) {
 #pragma unroll
   for (int r = 0; r < 10; ++r) {
-    const uint32_t hi0 = __umulhi(0xD2511F53u, c0), lo0 = 0xD2511F53u * c0;
-    const uint32_t hi1 = __umulhi(0xCD9E8D57u, c2), lo1 = 0xCD9E8D57u * c2;
-    c0 = hi1 ^ c1 ^ k0;
-    c1 = lo1;
-    c2 = hi0 ^ c3 ^ k1;
-    c3 = lo0;
+    // one 64-bit product (v_mad_u64_u32) instead of its two halves, and both
+    // exclusive ors in one operation
+    const uint64_t p0 = (uint64_t)c0 * 0xD2511F53u, p1 = (uint64_t)c2 * 0xCD9E8D57u;
+    c0 = __builtin_amdgcn_bitop3_b32((uint32_t)(p1 >> 32), c1, k0, 0x96);
+    c1 = (uint32_t)p1;
+    c2 = __builtin_amdgcn_bitop3_b32((uint32_t)(p0 >> 32), c3, k1, 0x96);
+    c3 = (uint32_t)p0;
     k0 += 0x9E3779B9u;
     k1 += 0xBB67AE85u;
   }
@@ -51,9 +53,9 @@ __device__ __forceinline__ void philox4x32(uint32_t c0, uint32_t c1, uint32_t c2
   out[3] = c3;
 }
 
-// uniform in (0, 1): the top 24 bits, centred in their interval
+// uniform in (0, 1): the top 24 bits plus a half, by 2^-24
 __device__ __forceinline__ float unit_open(uint32_t x) {
-  return ((float)(x >> 8) + 0.5f) * (1.0f / 16777216.0f);
+  return __builtin_fmaf((float)(x >> 8), 0x1p-24f, 0x1p-25f);
 }
 
 // three N(0, 1) deviates of pixel `g` in call `call`
@@ -74,79 +76,126 @@ __device__ __forceinline__ void pixel_normals(uint64_t seed, uint64_t call, uint
   n[2] = rb * __builtin_amdgcn_cosf(tb);
 }
 
-__device__ __forceinline__ float undistort(int x_, int y_, float z, const float* __restrict__ model) {
-  const int i2 = (int)((z + 1.0f) / 2.0f);
-  const int i1 = i2 - 1;
-  float a = (float)i1 * 2.0f;
-  a = a + 1.0f;
-  a = z - a;
-  a = a / 2.0f;
-  const int x = x_ / 8, y = y_ / 6;
-  const float* row = model + (y * kRwCols + x) * kRwDims;
-  const int k1 = min(max(i1, 0), 4), k2 = min(i2, 4);
-  const float wa = 1.0f - a;
-  const float p = wa * row[k1];
-  const float q = a * row[k2];
-  const float f = p + q;
-  if (f < 1e-5f) return 0.0f;
-  return z / f;
+// n / d for n < 2^31 by a multiplication: d > 1 is fixed for a launch
+// (Granlund & Montgomery 1994: with 2^(shift-1) < d <= 2^shift and
+// mul = ceil(2^(31 + shift) / d) the error stays below 1 / d)
+struct Divider {
+  uint32_t mul, shift;  // n / d = (n * mul >> 32) >> shift
+};
+
+Divider make_divider(uint32_t d) {
+  uint32_t s = 1;
+  while ((1ull << s) < d) ++s;
+  return {(uint32_t)(((1ull << (31 + s)) + d - 1) / d), s - 1};
 }
 
-// images x rows x cols, consecutive; normals: 3 per pixel or null (generator)
-__global__ __launch_bounds__(kNoiseBlock) void k_redwood(const float* __restrict__ depth,
-                                                         long long total, int H, int W,
-                                                         const float* __restrict__ model, float mult,
-                                                         const float* __restrict__ normals,
-                                                         uint64_t seed, uint64_t call,
-                                                         float* __restrict__ out) {
-  const long long g = (long long)blockIdx.x * kNoiseBlock + threadIdx.x;
-  if (g >= total) return;
-  const long long npx = (long long)H * W;
-  const long long img = g / npx;
-  const int idx = (int)(g - img * npx);
-  const float* dimg = depth + img * npx;
+__device__ __forceinline__ uint32_t divide(uint32_t n, Divider d) { return __umulhi(n, d.mul) >> d.shift; }
+
+// the disparity step in the general arithmetic
+__device__ __forceinline__ float disparity(float u, float nz) {
+  double t = (double)35.130f / (double)u;
+  t = t + (double)nz;
+  t = t * 8.0;
+  const double q = round(t);
+  return q > 1e-5 ? (float)((double)(35.130f * 8.0f) / q) : 0.0f;
+}
+
+struct RedwoodArgs {
+  const float* depth;    // images x rows x cols, consecutive
+  const float* model;
+  const float* normals;  // 3 per pixel, or null (generator)
+  float* out;
+  uint32_t total;        // pixels, < 2^31
+  uint32_t npx, W;
+  Divider by_npx, by_w;
+  float xmax, ymax;      // W - 1, H - 1
+  double rx, ry;         // 1 / xmax, 1 / ymax
+  float mult, mult4;     // the noise multiplier, and a quarter of it
+  uint64_t seed, call, first;  // first: the generator's number of pixel 0
+};
+
+// One thread per pixel.  8 bytes a pixel move, but what bounds the kernel is
+// the arithmetic: ten Philox rounds, two Box-Muller transforms, five quotients
+// and four integer divisions (one of 64 bits), 340 vector operations a pixel in
+// the general forms and 165 here: 512 images of 128x128 take 35 us, and took 56
+// (the copy of their bytes takes 13).  Every quotient is the cheapest form that
+// rounds the same:
+//  * pixel -> image, row, column: multiplications (`Divider`);
+//  * x / xmax: (float)((double)x * rx).  The product errs by less than 2^-52,
+//    and a quotient of two 24-bit numbers lies at least 2^-49 from the middle
+//    between two floats;
+//  * z / f and 281.04 / q: div_exact();
+//  * 35.13 / u in double: two Newton steps from the single reciprocal (2^-45)
+//    and a correction by the exact remainder (2^-90); the quotient of two
+//    24-bit numbers lies at least 2^-78 from the middle between two doubles;
+//  * the last quotient in single precision: for two floats a double quotient
+//    rounded to float is the float quotient (53 >= 2 * 24 + 2).
+// Operands outside their ranges (depths under a millimetre, factors f over 8,
+// quotients q of 2^23 and more, infinities and NaN in the table) take the
+// general arithmetic.
+__global__ __launch_bounds__(kNoiseBlock) void k_redwood(RedwoodArgs a) {
+  const uint32_t g = blockIdx.x * kNoiseBlock + threadIdx.x;
+  if (g >= a.total) return;
+  const uint32_t img = divide(g, a.by_npx), idx = g - img * a.npx;
   float n[3];
-  if (normals) {
-    n[0] = normals[3 * g];
-    n[1] = normals[3 * g + 1];
-    n[2] = normals[3 * g + 2];
+  if (a.normals) {
+    const float* nn = a.normals + 3 * (size_t)g;
+    n[0] = nn[0];
+    n[1] = nn[1];
+    n[2] = nn[2];
   } else {
-    pixel_normals(seed, call, (uint64_t)g, n);
+    pixel_normals(a.seed, a.call, a.first + g, n);
   }
-  const float ymax = (float)(H - 1), xmax = (float)(W - 1);
-  const int j = idx / W, i = idx - j * W;
-  float fy = n[0] * 0.25f;
-  fy = fy * mult;
-  fy = (float)j + fy;
-  fy = fminf(fmaxf(fy, 0.0f), ymax);
-  const int y = (int)(fy + 0.5f);
-  float fx = n[1] * 0.25f;
-  fx = fx * mult;
-  fx = (float)i + fx;
-  fx = fminf(fmaxf(fx, 0.0f), xmax);
-  const int x = (int)(fx + 0.5f);
-  const float d = dimg[(y - y % 2) * W + x - x % 2];
+  const uint32_t j = divide(idx, a.by_w), i = idx - j * a.W;
+  const float fy = n[0] * a.mult4 + (float)(int)j;
+  const float fx = n[1] * a.mult4 + (float)(int)i;
+  // nearest row and column, clamped (the median; 0 for NaN)
+  const int y = (int)__builtin_amdgcn_fmed3f(fy + 0.5f, 0.0f, a.ymax);
+  const int x = (int)__builtin_amdgcn_fmed3f(fx + 0.5f, 0.0f, a.xmax);
+  const float d = a.depth[(size_t)(g - idx + (uint32_t)(y & ~1) * a.W + (uint32_t)(x & ~1))];
   float res = 0.0f;
-  // beyond 10 m the sensor returns 0; negative and NaN depths give 0 too
-  if (d < 10.0f && !(d < 0.0f)) {
-    float ux = (float)x / xmax;
+  // beyond 10 m the sensor returns 0; zero, negative and NaN depths give 0 too
+  if (d > 0.0f && d < 10.0f) {
+    float ux = (float)((double)(float)x * a.rx);
     ux = ux * 639.0f;
     ux = ux + 0.5f;
-    float uy = (float)y / ymax;
+    float uy = (float)((double)(float)y * a.ry);
     uy = uy * 479.0f;
     uy = uy + 0.5f;
-    const float u = undistort((int)ux, (int)uy, d, model);
-    if (u != 0.0f) {
+    // the undistortion factor of (column / 8, row / 6) at this depth (the
+    // product is row / 6 for rows up to 1000)
+    const uint32_t cell = (__umul24((uint32_t)(int)uy, 10923u) >> 16) * kRwCols + ((uint32_t)(int)ux >> 3);
+    const int i2 = (int)((d + 1.0f) * 0.5f);
+    const float w = (d - __builtin_fmaf((float)i2, 2.0f, -1.0f)) * 0.5f;
+    const uint32_t at = cell * kRwDims;
+    const float wa = 1.0f - w;
+    const float p = wa * a.model[at + (uint32_t)max(i2 - 1, 0)];
+    const float q = w * a.model[at + (uint32_t)min(i2, 4)];
+    const float f = p + q;
+    if (!(f < 1e-5f)) {
       float nz = n[2] * 0.027778f;
-      nz = nz * mult;
-      double t = (double)35.130f / (double)u;
+      nz = nz * a.mult;
+      const float u = div_exact(d, f, rcp_exact(f));
+      const double du = (double)u, r0 = (double)__builtin_amdgcn_rcpf(u);
+      const double r1 = __builtin_fma(__builtin_fma(-du, r0, 1.0), r0, r0);
+      const double q0 = (double)35.130f * r1;
+      double t = __builtin_fma(__builtin_fma(-du, q0, (double)35.130f), r1, q0);
       t = t + (double)nz;
-      t = t * 8.0;
-      const double q = round(t);
-      if (q > 1e-5) res = (float)((double)(35.130f * 8.0f) / q);
+      if (d >= 0x1p-10f && f <= 8.0f && fabs(t) < 0x1p20) {
+        // 8 t rounded half away from zero: half to even, and one more where
+        // that went down from a half (a negative one ends as 0 either way)
+        const double shifted = __builtin_fma(t, 8.0, 0x1.8p52);
+        int k = (int)(uint32_t)__builtin_bit_cast(uint64_t, shifted);
+        k += __builtin_fma(t, 8.0, 0x1.8p52 - shifted) == 0.5 ? 1 : 0;
+        const float kf = (float)k;
+        if (k > 0) res = div_exact(35.130f * 8.0f, kf, rcp_exact(kf));
+      } else {
+        const float v = d / f;
+        if (v != 0.0f) res = disparity(v, nz);
+      }
     }
   }
-  out[g] = res;
+  a.out[g] = res;
 }
 
 __global__ __launch_bounds__(kNoiseBlock) void k_philox_bits(uint64_t seed, uint64_t call,
@@ -227,13 +276,36 @@ gbr_status check_dims(int32_t images, int32_t rows, int32_t cols, const char* fn
 
 gbr_status launch(gbr_redwood* m, const float* depth, int32_t images, int32_t rows, int32_t cols,
                   const float* normals, float* out, hipStream_t s) {
-  const long long total = (long long)images * rows * cols;
+  const long long npx = (long long)rows * cols, total = images * npx;
   if (total == 0) return GBR_OK;
-  const long long blocks = (total + gbr::kNoiseBlock - 1) / gbr::kNoiseBlock;
-  if (blocks > 0x7fffffffll) return fail(GBR_ERR_SIZE, "redwood: batch too large");
-  hipLaunchKernelGGL(gbr::k_redwood, dim3((uint32_t)blocks), dim3(gbr::kNoiseBlock), 0, s, depth,
-                     total, rows, cols, m->d_model.ptr, m->mult, normals, m->seed, m->calls, out);
-  HIP_TRY(hipGetLastError());
+  if ((total + gbr::kNoiseBlock - 1) / gbr::kNoiseBlock > 0x7fffffffll)
+    return fail(GBR_ERR_SIZE, "redwood: batch too large");
+  gbr::RedwoodArgs a{};
+  a.model = m->d_model.ptr;
+  a.npx = (uint32_t)npx;
+  a.W = (uint32_t)cols;
+  a.by_npx = gbr::make_divider(a.npx);
+  a.by_w = gbr::make_divider(a.W);
+  a.xmax = (float)(cols - 1);
+  a.ymax = (float)(rows - 1);
+  a.rx = 1.0 / (double)a.xmax;
+  a.ry = 1.0 / (double)a.ymax;
+  a.mult = m->mult;
+  a.mult4 = m->mult * 0.25f;
+  a.seed = m->seed;
+  a.call = m->calls;
+  // launches of as many whole images as keep the pixel number under 2^31
+  const long long run = 0x7fffffffll / npx * npx;
+  for (long long first = 0; first < total; first += run) {
+    a.depth = depth + first;
+    a.normals = normals ? normals + 3 * first : nullptr;
+    a.out = out + first;
+    a.first = (uint64_t)first;
+    a.total = (uint32_t)std::min(run, total - first);
+    hipLaunchKernelGGL(gbr::k_redwood, dim3((a.total + gbr::kNoiseBlock - 1) / gbr::kNoiseBlock),
+                       dim3(gbr::kNoiseBlock), 0, s, a);
+    HIP_TRY(hipGetLastError());
+  }
   if (!normals) ++m->calls;
   return GBR_OK;
 }

@@ -41,6 +41,36 @@ def test_given_deviates_bit_exact(shape, mult):
     assert m.calls == 0  # caller deviates do not advance the generator
 
 
+@pytest.mark.parametrize("shape", [(1, 2, 2), (1, 2, 515), (300, 3, 2), (7, 31, 129), (1, 1023, 3), (2, 257, 641)])
+@pytest.mark.parametrize("mult", [0.0, 1.0, 4000.0])
+def test_every_operand_range_is_bit_exact(shape, mult):
+    """Depths and undistortion factors over all magnitudes, zeros of both
+    signs, denormals, infinities and NaN among them, so that both the quotients
+    made for the ordinary range and the general ones run: the outputs equal the
+    oracle's bit for bit."""
+    rng = np.random.default_rng(shape[0] * 1000 + shape[1] + shape[2])
+    depth = rng.uniform(0.0, 10.5, shape).astype(np.float32)
+    small = rng.random(shape) < 0.3
+    depth[small] = np.ldexp(rng.random(shape), rng.integers(-149, 4, shape)).astype(np.float32)[small]
+    flat = depth.reshape(-1)
+    odd = np.array([0.0, -0.0, 1e-45, -1e-45, 2.0 ** -60, 9.999999, 10.0, np.inf, -np.inf, np.nan], np.float32)
+    at = rng.random(flat.size) < 0.1
+    flat[at] = rng.choice(odd, at.sum())
+    model = rng.uniform(0.5, 1.5, 80 * 80 * 5).astype(np.float32)
+    wild = rng.random(model.size) < 0.1
+    model[wild] = np.ldexp(rng.random(model.size), rng.integers(-30, 120, model.size)).astype(np.float32)[wild]
+    wild = rng.random(model.size) < 0.03
+    model[wild] = rng.choice(np.array([0.0, 1e-5, -1.0, np.inf, np.nan], np.float32), wild.sum())
+    normals = (rng.standard_normal(shape + (3,)) * 2.0).astype(np.float32)
+    normals.reshape(-1)[::101] = np.nan
+    normals.reshape(-1)[::103] = -np.inf
+    m = RedwoodDepthNoiseModel(model, noise_multiplier=mult)
+    d, n = hip.to_device(depth), hip.to_device(normals)
+    out = hip.DeviceBuffer(depth.nbytes)
+    m.simulate_device_normals(d.value, shape[0], shape[1], shape[2], n.value, out.value)
+    np.testing.assert_array_equal(_host(out, shape), redwood_noise(depth, model, mult, normals))
+
+
 def test_generator_blocks_bit_exact():
     seed = 0x0123456789ABCDEF
     m = RedwoodDepthNoiseModel(load_model(MODEL), seed=seed)
