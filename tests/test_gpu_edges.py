@@ -1,0 +1,274 @@
+"""The rasteriser, clipper, texture sampler, frame inputs and readback at the
+sizes where their work is split, bit for bit against the oracle: triangles from
+a fraction of a pixel to beyond the guard band, workgroups' and waves' worth of
+them and one more, tiles that end inside a bin and inside an 8x8 block, more
+textures than fit in LDS, every filter and wrap mode at sizes that are no power
+of two, any subset of the planes."""
+import os
+
+import numpy as np
+import pytest
+
+import synth
+from habitat_sim_amd import RendererConfiguration, RendererStandalone
+from habitat_sim_amd import _native as N
+from habitat_sim_amd import math3d as m3
+from habitat_sim_amd.assets import (GL_CLAMP_TO_EDGE, GL_LINEAR, GL_LINEAR_MIPMAP_LINEAR,
+                                    GL_LINEAR_MIPMAP_NEAREST, GL_MIRRORED_REPEAT, GL_NEAREST,
+                                    GL_NEAREST_MIPMAP_LINEAR, GL_NEAREST_MIPMAP_NEAREST, GL_REPEAT)
+from oracle.oracle import OracleRenderer
+
+pytestmark = pytest.mark.gpu
+
+NTHREADS = min(16, os.cpu_count() or 1)
+BITS = {"color": N.PLANE_COLOR, "depth": N.PLANE_DEPTH, "linear_depth": N.PLANE_LINEAR_DEPTH,
+        "semantic": N.PLANE_SEMANTIC}
+
+
+def _soup(rng, n, size):
+    """n triangles around the camera at the origin, which looks along -z; edge
+    lengths from a hundredth of `size` to `size`, some across the near plane."""
+    c = rng.uniform((-6.0, -6.0, -12.0), (6.0, 6.0, 1.0), (n, 1, 3))
+    s = size * 10.0 ** rng.uniform(-2.0, 0.0, (n, 1, 1))
+    return (c + s * rng.uniform(-1.0, 1.0, (n, 3, 3))).reshape(-1, 3).astype(np.float32)
+
+
+def _pair(tile, grid, planes=N.PLANE_ALL, **tuning):
+    r = RendererStandalone(RendererConfiguration().set_tile_size_count(tile, grid), planes=planes)
+    if tuning:
+        r.set_tuning(**tuning)
+    return r, OracleRenderer(tile, grid)
+
+
+def _draw(r, o):
+    r.draw()
+    o.draw(NTHREADS)
+
+
+def _same(r, o, names=tuple(BITS), tag=""):
+    for name in names:
+        a, b = getattr(r, f"{name}_image")(), getattr(o, f"{name}_image")()
+        diff = a != b
+        if diff.ndim == 3:
+            diff = diff.any(-1)
+        assert not diff.any(), f"{tag} {name}: {int(diff.sum())} pixels differ from the oracle"
+
+
+def _camera(x, scene, tile, pose=None):
+    P = m3.perspective_projection(1.4, tile[0] / tile[1], 0.05, 50.0)
+    x.update_camera(scene, P, m3.inverted_rigid(m3.identity() if pose is None else pose))
+
+
+@pytest.mark.parametrize("tile,tuning", [((64, 64), {}), ((131, 77), {}), ((131, 77), dict(bin_size=8)),
+                                         ((33, 129), dict(bin_size=16)), ((8, 8), {}), ((1, 1), {}),
+                                         ((131, 77), dict(raster_mode=1)),
+                                         ((131, 77), dict(raster_mode=1, bin_size=8, cull_mode=N.CULL_HIZ)),
+                                         ((200, 9), dict(cull_mode=N.CULL_FRUSTUM)),
+                                         ((97, 97), dict(cull_mode=N.CULL_HIZ, lane_pixels=16))])
+def test_triangles_of_every_size(tile, tuning):
+    """Seven scenes of 0 to 1500 triangles each; two frames, so that a culled
+    one has a previous frame's visible set too."""
+    rng = np.random.default_rng(tile[0] * 1000 + tile[1])
+    counts = (1, 0, 63, 64, 65, 257, 1500)
+    meshes = [(_soup(rng, max(n, 1), size), np.arange(3 * max(n, 1), dtype=np.uint32), None, None, k % 2)
+              for k, (n, size) in enumerate(zip(counts, (300.0, 1.0, 3.0, 40.0, 2.0, 1.0, 1.0)))]
+    fd = synth.mesh_file(meshes, [synth.flat((0.9, 0.5, 0.2, 1)), synth.flat((0.3, 0.6, 1.0, 1))])
+    r, o = _pair(tile, (4, 2), **tuning)
+    for x in (r, o):
+        assert x.add_file_data(fd)
+        for s, n in enumerate(counts):
+            if n:
+                x.add_node_hierarchy(s, f"m{s}", None, s + 1)
+            # (outside the frustum behind the camera: every vertex beyond a plane)
+            x.add_node_hierarchy(s, "m2", m3.translation((0.0, 0.0, 60.0)), 90)
+            _camera(x, s, tile)
+    _draw(r, o)
+    _same(r, o, tag="first")
+    if min(tile) > 1:
+        assert len(np.unique(r.semantic_image())) > 4
+    for x in (r, o):
+        for s in range(len(counts)):
+            _camera(x, s, tile, m3.rotation_y(0.4))
+    _draw(r, o)
+    _same(r, o, tag="second")
+    r.close()
+
+
+@pytest.mark.parametrize("tuning", [{}, dict(cull_mode=N.CULL_HIZ), dict(bin_size=8)])
+def test_a_whole_scene_in_one_bin(tuning):
+    """9000 small triangles inside 16x16 pixels: a bin's list many times longer
+    than the mean."""
+    rng = np.random.default_rng(5)
+    p = rng.uniform((-0.1, -0.1, -3.0), (0.1, 0.1, -1.0), (9000, 1, 3)) + rng.uniform(-0.02, 0.02, (9000, 3, 3))
+    mesh = (p.reshape(-1, 3).astype(np.float32), np.arange(27000, dtype=np.uint32), None, None, 0)
+    r, o = _pair((128, 128), (2, 1), **tuning)
+    for x in (r, o):
+        assert x.add_file_data(synth.mesh_file([mesh], [synth.flat((1, 1, 1, 1))]))
+        x.add_node_hierarchy(1, "m0", None, 7)
+        for s in range(2):
+            _camera(x, s, (128, 128))
+    for _ in range(2):
+        _draw(r, o)
+        _same(r, o)
+    r.close()
+
+
+def _levels(rng, w, h):
+    out = []
+    while True:
+        out.append(rng.integers(0, 256, (h, w, 4), dtype=np.uint8))
+        if w == h == 1:
+            return out
+        w, h = max(w // 2, 1), max(h // 2, 1)
+
+
+MINS = (GL_NEAREST, GL_LINEAR, GL_NEAREST_MIPMAP_NEAREST, GL_LINEAR_MIPMAP_NEAREST,
+        GL_NEAREST_MIPMAP_LINEAR, GL_LINEAR_MIPMAP_LINEAR)
+WRAPS = (GL_REPEAT, GL_CLAMP_TO_EDGE, GL_MIRRORED_REPEAT)
+
+
+@pytest.mark.parametrize("count", [1, 7, 8, 9, 18])
+def test_textures_filters_and_wraps(count):
+    """`count` textures (8 descriptors fit in LDS), their sizes from 1x1 to
+    37x64, each filter with each wrap mode, seen under perspective with
+    coordinates well outside [0, 1]; the last texel of the last one is read."""
+    rng = np.random.default_rng(count)
+    sizes = ((4, 4), (1, 1), (37, 64), (2, 1), (5, 3), (16, 16), (1, 9), (33, 17), (64, 8))
+    textures, meshes = [], []
+    for k in range(count):
+        w, h = sizes[k % len(sizes)]
+        t = synth.texture(_levels(rng, w, h), min_filter=MINS[k % 6], mag_filter=(GL_NEAREST, GL_LINEAR)[k // 3 % 2],
+                          wrap=WRAPS[(k + k // 6) % 3])
+        t.wrap_t = WRAPS[(k // 2) % 3]
+        textures.append(t)
+        tilt = rng.uniform(-1.5, 1.5, 2)
+        pos = np.array([[x, y, -4.0 + tilt[0] * x + tilt[1] * y] for x, y in ((-1, -1), (1, -1), (1, 1), (-1, 1))])
+        pos += (rng.uniform(-1.5, 1.5), rng.uniform(-1.5, 1.5), 0.0)
+        scale = 10.0 ** rng.uniform(-1.0, 1.3)
+        uv = np.array([(0, 0), (1, 0), (1, 1), (0, 1)]) * scale + rng.uniform(-2.0, 2.0, 2)
+        meshes.append((pos.astype(np.float32), np.array([0, 1, 2, 0, 2, 3], np.uint32), uv.astype(np.float32), None, k))
+    fd = synth.mesh_file(meshes, [synth.flat((1, 1, 1, 1), texture=k) for k in range(count)], textures)
+    tile = (150, 101)
+    r, o = _pair(tile, (3, 1))
+    for x in (r, o):
+        assert x.add_file_data(fd)
+        for s in range(3):
+            for k in range(count):
+                if s == 0 or (k + s) % 2 == 0:
+                    x.add_node_hierarchy(s, f"m{k}", None, k + 1)
+            _camera(x, s, tile, m3.translation((0.0, 0.0, -1.2 * s)))
+    _draw(r, o)
+    _same(r, o)
+    r.close()
+
+
+@pytest.mark.parametrize("names", [("color",), ("depth",), ("semantic",), ("linear_depth",),
+                                   ("linear_depth", "semantic"), ("color", "depth"), ("color", "semantic")])
+def test_any_subset_of_the_planes(names):
+    rng = np.random.default_rng(11)
+    tile = (70, 41)
+    planes = sum(BITS[n] for n in names)
+    r, o = _pair(tile, (2, 2), planes=planes)
+    mesh = (_soup(rng, 200, 2.0), np.arange(600, dtype=np.uint32), rng.uniform(-1, 2, (600, 2)), None, 0)
+    fd = synth.mesh_file([mesh], [synth.flat((1, 1, 1, 1), texture=0)],
+                         [synth.texture(_levels(rng, 13, 7), min_filter=GL_LINEAR_MIPMAP_LINEAR, mag_filter=GL_LINEAR)])
+    for x in (r, o):
+        assert x.add_file_data(fd)
+        for s in range(4):
+            x.add_node_hierarchy(s, "m0", m3.rotation_y(0.5 * s), s + 1)
+            _camera(x, s, tile)
+    _draw(r, o)
+    _same(r, o, names)
+    r.close()
+
+
+@pytest.mark.parametrize("graph", [0, 1])
+@pytest.mark.parametrize("envs", [1, 5])
+def test_moved_nodes_lights_and_cameras_over_frames(envs, graph):
+    """Frames that move nothing, one node, every node, only cameras, only
+    lights, nodes and lights of some scenes: the image is always the one of the
+    present state."""
+    rng = np.random.default_rng(envs)
+    tile = (48, 48)
+    n = 150
+    nodes = 40
+    pos = _soup(rng, n, 1.0)
+    mesh = (pos, np.arange(3 * n, dtype=np.uint32), None, None, 0)
+    fd = synth.mesh_file([mesh], [synth.flat((0.8, 0.8, 0.8, 1))])
+    fd.materials[0].flat = False
+    normal = rng.standard_normal(pos.shape)
+    fd.meshes[0].normals = (normal / np.linalg.norm(normal, axis=1, keepdims=True)).astype(np.float32)
+    grid = (envs, 1)
+    r = RendererStandalone(RendererConfiguration().set_tile_size_count(tile, grid).set_max_light_count(2))
+    r.set_tuning(graph=graph)
+    o = OracleRenderer(tile, grid, max_light_count=2)
+    ids = {}
+    for x in (r, o):
+        assert x.add_file_data(fd)
+        for s in range(envs):
+            ids[s] = [x.add_node_hierarchy(s, "m0", m3.scaling((0.3, 0.3, 0.3)), k + 1) for k in range(nodes)]
+            light = x.add_empty_node(s)
+            ids[s].append(light)
+            x.add_light(s, light, N.LIGHT_POINT)
+            _camera(x, s, tile)
+    frames = [(), ("all",), (), ("one",), ("camera",), ("light",), ("one", "camera", "light"), ("some",), ("all", "light")]
+    for f, what in enumerate(frames):
+        for s in range(envs):
+            move = []
+            if "all" in what:
+                move = list(range(nodes + 1))
+            elif "one" in what and s == envs - 1:
+                move = [int(rng.integers(nodes))]
+            elif "some" in what and s % 2 == 0:
+                move = sorted(rng.choice(nodes + 1, 7, replace=False))
+            poses = [m3.mul(m3.translation(tuple(rng.uniform(-2, 2, 3) - (0, 0, 3))), m3.rotation_y(rng.uniform(0, 6)))
+                     for _ in move]
+            colour = rng.uniform(0.0, 2.0, 3).astype(np.float32)
+            yaw = rng.uniform(-0.3, 0.3)
+            for x in (r, o):
+                t = x.transformations(s)
+                for k, p in zip(move, poses):
+                    t[ids[s][k]] = p
+                if "light" in what:
+                    x.light_colors(s)[0] = colour
+                    x.light_ranges(s)[0] = np.float32(5.0 + f)
+                if "camera" in what:
+                    _camera(x, s, tile, m3.rotation_y(yaw))
+        _draw(r, o)
+        _same(r, o, tag=f"frame {f} {what}")
+    r.close()
+
+
+def test_readback_rectangles_strides_and_large_images():
+    """A framebuffer beyond 8 MB a plane, whole, in rectangles of odd offsets
+    and sizes, into padded rows and as three channels."""
+    rng = np.random.default_rng(2)
+    tile = (523, 701)
+    r, o = _pair(tile, (4, 2))
+    mesh = (_soup(rng, 60, 4.0), np.arange(180, dtype=np.uint32), None, None, 0)
+    for x in (r, o):
+        assert x.add_file_data(synth.mesh_file([mesh], [synth.flat((0.2, 0.7, 0.4, 1))]))
+        for s in range(8):
+            x.add_node_hierarchy(s, "m0", m3.rotation_y(0.3 * s), s + 1)
+            _camera(x, s, tile)
+    _draw(r, o)
+    _same(r, o)
+    w, h = 4 * tile[0], 2 * tile[1]
+    color, sem, lin = o.color_image(), o.semantic_image(), o.linear_depth_image()
+    for x0, y0, x1, y1 in ((0, 0, w, h), (1, 3, 2, 4), (5, 0, 5 + 131, h), (0, h - 1, w, h), (w - 7, 11, w, 500)):
+        pad = rng.integers(0, 256, (y1 - y0, x1 - x0 + 3, 4), dtype=np.uint8)
+        keep = pad.copy()
+        r.color_image_into((x0, y0, x1, y1), pad[:, :x1 - x0])
+        np.testing.assert_array_equal(pad[:, :x1 - x0], color[y0:y1, x0:x1])
+        np.testing.assert_array_equal(pad[:, x1 - x0:], keep[:, x1 - x0:])
+        rgb = np.zeros((y1 - y0, x1 - x0, 3), np.uint8)
+        r.color_image_into((x0, y0, x1, y1), rgb)
+        np.testing.assert_array_equal(rgb, color[y0:y1, x0:x1, :3])
+        ids = np.zeros((y1 - y0, x1 - x0 + 5), np.uint32)
+        r.semantic_image_into((x0, y0, x1, y1), ids[:, :x1 - x0])
+        np.testing.assert_array_equal(ids[:, :x1 - x0], sem[y0:y1, x0:x1])
+        assert not ids[:, x1 - x0:].any()
+        z = np.zeros((y1 - y0, x1 - x0), np.float32)
+        r.linear_depth_image_into((x0, y0, x1, y1), z)
+        np.testing.assert_array_equal(z, lin[y0:y1, x0:x1])
+    r.close()

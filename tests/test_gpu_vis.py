@@ -54,6 +54,30 @@ def test_loss_and_gradient_match_oracle(rows, pos_weight):
     r.close()
 
 
+@pytest.mark.parametrize("rows", [32, 96, 512, 992, 1024, 1056, 2112])
+def test_gradient_at_the_edges_of_the_batch_split(rows):
+    """One tile of rows; batches that are no multiple of 64, and ones below, at
+    and above the 32 steps of 16 rows whose loads run ahead and the 1024 rows
+    of a column sum's inner loop.  Tolerances as in
+    test_loss_and_gradient_match_oracle."""
+    r = _small()
+    flat = M.he_uniform(rows).astype(np.float32)
+    r.set_vis_weights(flat)
+    X, y = _rows(rows, rows)
+    loss, g = r.vis_loss_grad(X, y, 2.0)
+    ref_loss, ref_g = M.loss_grad(flat.astype(np.float64), X, y, 2.0, rounding=True)
+    assert abs(loss - ref_loss) <= 1e-4 * abs(ref_loss)
+    o = 0
+    for name, shape in M.SIZES:
+        n = int(np.prod(shape))
+        a, b = g[o:o + n].astype(np.float64), ref_g[o:o + n]
+        assert np.linalg.norm(a - b) <= 1e-2 * np.linalg.norm(b) + 1e-7, name
+        o += n
+    again, g2 = r.vis_loss_grad(X, y, 2.0)
+    assert again == loss and np.array_equal(g, g2)
+    r.close()
+
+
 @pytest.mark.parametrize("rows", [100, 20000])
 def test_logits_match_oracle(rows):
     # the renderer's fused scorer: 100 rows are a ragged last tile; 20000 rows
