@@ -1,4 +1,4 @@
-// Correctly rounded single-precision quotients in a few fused operations, for
+// Correctly rounded single-precision quotients and roots in a few fused operations, for
 // operands whose range is known (device code only).
 #pragma once
 
@@ -21,6 +21,13 @@ __device__ __forceinline__ float rcp_exact(float x) {
 __device__ __forceinline__ float div_exact(float a, float b, float r) {
   const float q = a * r;
   return __builtin_fmaf(__builtin_fmaf(-b, q, a), r, q);
+}
+
+// sqrt(x), correctly rounded, for 2^-80 <= x <= 2^80 (compared with the general
+// square root over every float of that range)
+__device__ __forceinline__ float sqrt_exact(float x) {
+  const float y = __builtin_amdgcn_rsqf(x), s = x * y;
+  return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
 }
 
 __device__ __forceinline__ bool in_range(float x, float lo, float hi) {

@@ -1586,6 +1586,27 @@ __device__ __forceinline__ uint32_t to_unorm8(float c) {
   return (uint32_t)(int)v;
 }
 
+// v / |v|, each operation rounded as by itself; returns |v|.  The short forms
+// serve lengths within 2^+-30 whose components are 0 or at least 2^-60 (a
+// component's bits, doubled, less one: 0 becomes the largest value).
+__device__ __forceinline__ float normalise(float* v) {
+  float vv = v[0] * v[0]; float v1 = v[1] * v[1]; vv = vv + v1; float v2 = v[2] * v[2];
+  vv = vv + v2;
+  uint32_t least = ~0u;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) least = min(least, 2u * __float_as_uint(v[k]) - 1u);
+  if (in_range(vv, 0x1p-60f, 0x1p60f) && least >= 2u * 0x21800000u - 1u) {
+    const float len = sqrt_exact(vv), r = rcp_exact(len);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) v[k] = div_exact(v[k], len, r);
+    return len;
+  }
+  const float len = sqrtf(vv);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) v[k] = v[k] / len;
+  return len;
+}
+
 // Phong diffuse term of the scene's lights (no specular) for a shaded
 // material, in world space: per light, intensity = max(0, N.L) * attenuation
 // with attenuation clamp(1 - (d/R)^4, 0, 1)^2 / (1 + d^2) for point lights
@@ -1594,6 +1615,11 @@ __device__ __forceinline__ uint32_t to_unorm8(float c) {
 // material diffuse * texture colour * vertex colour.  Vertex positions and
 // normals come from the mesh through the draw's absolute transform and normal
 // matrix, interpolated with the pixel's barycentrics b.
+// A pixel spends its time on the latency of what it gathers and on quotients:
+// with the vertices' loads in flight together, the lights in scalar registers
+// (uniform over a workgroup; as vector loads each light was two dependent
+// round trips) and the short roots and quotients k_resolve takes 39 us for 64
+// scenes of 128x128 with four lights, and took 59.
 __device__ void add_lights(const FrameParams& p, const DrawDesc& d, uint32_t prim, uint32_t scene,
                            const float* b, const float* texc, const float* vc, float* c) {
   const MaterialDesc& mat = p.materials[d.material];
@@ -1605,50 +1631,53 @@ __device__ void add_lights(const FrameParams& p, const DrawDesc& d, uint32_t pri
   const uint32_t* ip = p.indices + d.index_base + 3 * (prim - d.prim_base);
   const float* M = p.abs_nodes + (size_t)d.node * 16;
   const float* NM = p.normal_mats + (size_t)d.node * 12;
-  // world position and normal interpolated vertex by vertex: the sums
-  // b0*a0 + b1*a1 + b2*a2 of interp3, in its order
-  float n[3], pw[3];
-#pragma unroll 1
+  // the three vertices' loads all in flight, then world position and normal
+  // interpolated vertex by vertex: the sums b0*a0 + b1*a1 + b2*a2 of interp3,
+  // in its order
+  float n[3], pw[3], vp[3][3], vn[3][3];
+#pragma unroll
   for (int k = 0; k < 3; ++k) {
     const uint32_t v = ip[k];
-    const float bk = k == 0 ? b[0] : (k == 1 ? b[1] : b[2]);
+    vp[k][0] = p.pos_x[v];
+    vp[k][1] = p.pos_y[v];
+    vp[k][2] = p.pos_z[v];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) vn[k][r] = p.normals[3 * (size_t)v + r];
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
     float q[4];
-    mat4_vec(M, p.pos_x[v], p.pos_y[v], p.pos_z[v], 1.0f, q);
-    const float n0 = p.normals[3 * (size_t)v], n1 = p.normals[3 * (size_t)v + 1],
-                n2 = p.normals[3 * (size_t)v + 2];
+    mat4_vec(M, vp[k][0], vp[k][1], vp[k][2], 1.0f, q);
 #pragma unroll
     for (int r = 0; r < 3; ++r) {
-      float x = NM[r] * n0; float y = NM[3 + r] * n1; x = x + y;
-      float z = NM[6 + r] * n2; x = x + z;
-      const float tn = bk * x, tp = bk * q[r];
+      float x = NM[r] * vn[k][0]; float y = NM[3 + r] * vn[k][1]; x = x + y;
+      float z = NM[6 + r] * vn[k][2]; x = x + z;
+      const float tn = b[k] * x, tp = b[k] * q[r];
       n[r] = k == 0 ? tn : n[r] + tn;
       pw[r] = k == 0 ? tp : pw[r] + tp;
     }
   }
-  float nn = n[0] * n[0]; float n1 = n[1] * n[1]; nn = nn + n1; float n2 = n[2] * n[2];
-  nn = nn + n2;
-  const float nl = sqrtf(nn);
-#pragma unroll
-  for (int k = 0; k < 3; ++k) n[k] = n[k] / nl;
-  const uint32_t first = p.scene_lights[2 * scene], count = p.scene_lights[2 * scene + 1];
+  normalise(n);
+  const uint32_t first = uniform_load(p.scene_lights, 2 * scene),
+                 count = uniform_load(p.scene_lights, 2 * scene + 1);
   for (uint32_t l = first; l < first + count; ++l) {
-    const LightDesc ld = p.lights[l];
-    const float* T = p.abs_nodes + (size_t)ld.node * 16;
-    float L[3], att = 1.0f;
+    // (uniform: the light and its node's transform are scalar loads)
+    const LightDesc ld = uniform_load(p.lights, l);
+    const float4 T =
+        uniform_load(reinterpret_cast<const float4*>(p.abs_nodes) + (size_t)ld.node * 4,
+                     ld.type == GBR_LIGHT_POINT ? 3u : 2u);
+    float L[3] = {-T.x, -T.y, -T.z}, att = 1.0f;
     if (ld.type == GBR_LIGHT_POINT) {
-#pragma unroll
-      for (int k = 0; k < 3; ++k) L[k] = T[12 + k] - pw[k];
-    } else {
-#pragma unroll
-      for (int k = 0; k < 3; ++k) L[k] = -T[8 + k];
+      L[0] = T.x - pw[0];
+      L[1] = T.y - pw[1];
+      L[2] = T.z - pw[2];
     }
-    float ll = L[0] * L[0]; float l1 = L[1] * L[1]; ll = ll + l1; float l2 = L[2] * L[2];
-    ll = ll + l2;
-    const float dist = sqrtf(ll);
-#pragma unroll
-    for (int k = 0; k < 3; ++k) L[k] = L[k] / dist;
+    const float dist = normalise(L);
     if (ld.type == GBR_LIGHT_POINT) {
-      float qd = dist / ld.range;
+      const bool in = in_range(dist, 0x1p-30f, 0x1p30f);
+      float qd;
+      if (in && in_range(ld.range, 0x1p-30f, 0x1p30f)) qd = div_exact(dist, ld.range, rcp_exact(ld.range));
+      else qd = dist / ld.range;
       qd = qd * qd;
       qd = qd * qd;
       float wdw = 1.0f - qd;
@@ -1657,7 +1686,9 @@ __device__ void add_lights(const FrameParams& p, const DrawDesc& d, uint32_t pri
       att = wdw * wdw;
       float den = dist * dist;
       den = 1.0f + den;
-      att = att / den;
+      // (att is 0 or at least 2^-48)
+      if (in) att = div_exact(att, den, rcp_exact(den));
+      else att = att / den;
     }
     float ndl = n[0] * L[0]; float t1 = n[1] * L[1]; ndl = ndl + t1; float t2 = n[2] * L[2];
     ndl = ndl + t2;

@@ -239,6 +239,46 @@ def test_moved_nodes_lights_and_cameras_over_frames(envs, graph):
     r.close()
 
 
+@pytest.mark.parametrize("scale", [1.0, 1e-12, 1e-25, 1e-40, 1e12, 1e20, 0.0])
+def test_light_operands_of_every_magnitude(scale):
+    """Normals of every length with zero and nearly zero components, lights of
+    no, tiny, huge and infinite range, far away and on the surface."""
+    tile = (64, 48)
+    quads = [((-2, -2), (0, 0, 1)), ((0, -2), (0, 1, 0)), ((-2, 0), (1e-20, 0.6, 0.8)), ((0, 0), (0.3, -1e-30, 0.9))]
+    meshes, normals = [], []
+    for (x, y), n in quads:
+        pos = np.array([(x, y, -3), (x + 2, y, -3), (x + 2, y + 2, -3), (x, y + 2, -3)], np.float32)
+        meshes.append((pos, np.array([0, 1, 2, 0, 2, 3], np.uint32), None, None, 0))
+        normals.append(np.tile(np.array(n, np.float64) * scale, (4, 1)).astype(np.float32))
+    fd = synth.mesh_file(meshes, [synth.flat((0.9, 0.7, 0.8, 1))])
+    fd.materials[0].flat = False
+    for mesh, n in zip(fd.meshes, normals):
+        mesh.normals = n
+    lights = [((0.5, 0.5, -2.0), np.inf), ((-0.5, 0.5, -2.5), 3.0), ((0.0, 0.0, -3.0), 1e-35), ((1e12, 0.0, 0.0), 1e30),
+              ((1e-25, 1e-25, -3.0), 5.0), ((0.0, 1e30, 0.0), np.inf), None, ((0.3, -0.4, -1.0), 0.0)]
+    r = RendererStandalone(RendererConfiguration().set_tile_size_count(tile, (2, 1)).set_max_light_count(8))
+    o = OracleRenderer(tile, (2, 1), max_light_count=8)
+    for x in (r, o):
+        assert x.add_file_data(fd)
+        for s in range(2):
+            for k in range(4):
+                x.add_node_hierarchy(s, f"m{k}", None, k + 1)
+            for i, light in enumerate(lights):
+                node = x.add_empty_node(s)
+                if light is None:
+                    x.transformations(s)[node] = m3.look_at((0, 0, 0), (0.2, -1.0, -0.5), (0.0, 0.0, 1.0))
+                    x.add_light(s, node, N.LIGHT_DIRECTIONAL)
+                else:
+                    x.transformations(s)[node] = m3.translation(light[0])
+                    x.add_light(s, node, N.LIGHT_POINT)
+                    x.light_ranges(s)[i] = np.float32(light[1])
+                x.light_colors(s)[i] = np.array((0.2, 0.3, 0.1), np.float32)
+            _camera(x, s, tile, m3.rotation_y(0.1 * s))
+    _draw(r, o)
+    _same(r, o)
+    r.close()
+
+
 def test_readback_rectangles_strides_and_large_images():
     """A framebuffer beyond 8 MB a plane, whole, in rectangles of odd offsets
     and sizes, into padded rows and as three channels."""
