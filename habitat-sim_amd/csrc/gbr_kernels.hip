@@ -1,6 +1,7 @@
 // HIP kernels of the batch renderer for gfx950 (CDNA4, wave64).
 //
 // Pipeline per frame (all scenes in one launch per stage, on one stream):
+//   k_inputs      cameras, lights and moved nodes from a pinned host block
 //   k_nodes       per node: absolute transform = parent chain product
 //                 (Renderer.cpp:1214-1220 moved to the GPU); resets the
 //                 frame's counters

@@ -10,8 +10,9 @@
 //   k_train_grads1   dW1 = dH1^T X and the sums for b1
 //   k_adam           the weights, and their bf16 copies
 // Every product is an "NT" one, C[M][N] = sum_k A[M][K] * Bt[N][K], with the
-// eight k of an MFMA fragment's lane contiguous in both operands.  The sums are reductions with one writer per output (no atomics),
-// and every sum runs in a fixed order, whatever the launch geometry.
+// eight k of an MFMA fragment's lane contiguous in both operands.  The sums
+// are reductions with one writer per output (no atomics), and every sum runs
+// in a fixed order, whatever the launch geometry.
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>

@@ -112,7 +112,9 @@ typedef struct gbr_scene_stats_info {
 typedef struct gbr_tuning {
   int32_t bin_size;           /* screen bin edge in pixels: 8, 16 or 32 */
   int32_t chunk_triangles;    /* triangles per setup work item: 1..1024 */
-  float bin_capacity_factor;  /* per-bin entry capacity relative to tris/bins */
+  float bin_capacity_factor;  /* per-bin entry capacity relative to tris/bins; from 1
+                                 on, bins get several times that, bounded per bin
+                                 and scene (a camera sees triangles unevenly) */
   int32_t min_bin_capacity;   /* lower bound of the per-bin capacity */
   int32_t cull_mode;          /* GBR_CULL_* */
   int32_t queue_grain;        /* setup work items claimed per queue fetch: 1..64 */
@@ -123,7 +125,7 @@ typedef struct gbr_tuning {
                                  exceeds this */
   int32_t lane_pixels;        /* raster_mode 0: triangles covering more than this
                                  many pixels of a bin are rasterised by a whole
-                                 wave (the rectangle spread over its lanes), the
+                                 wave in blocks of 8x8 pixels, the
                                  rest by one lane each: 1..1024; default 64 */
   int32_t graph;              /* 1: gbr_draw() replays its kernel sequence as a
                                  captured HIP graph while nothing but cameras and
