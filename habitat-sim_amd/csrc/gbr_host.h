@@ -33,9 +33,10 @@ template <class T>
 struct DevBuf {
   T* ptr = nullptr;
   size_t cap = 0;
-  gbr_status reserve(size_t n, bool keep = false, hipStream_t s = nullptr) {
+  // (`spare`: with room to grow by half)
+  gbr_status reserve(size_t n, bool keep = false, hipStream_t s = nullptr, bool spare = true) {
     if (n <= cap && ptr) return GBR_OK;
-    size_t ncap = std::max<size_t>(n + n / 2, 64);
+    size_t ncap = std::max<size_t>(spare ? n + n / 2 : n, 64);
     T* np = nullptr;
     hipError_t e = hipMalloc(reinterpret_cast<void**>(&np), ncap * sizeof(T));
     if (e != hipSuccess)

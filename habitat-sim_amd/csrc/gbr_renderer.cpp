@@ -431,6 +431,54 @@ gbr_status upload_assets(gbr_renderer* r) {
   return GBR_OK;
 }
 
+// Gives every bin its capacity and its place in the entry list; returns the
+// list's length.
+//
+// A camera sees its triangles unevenly: a bin of a scene with few triangles,
+// or with many bins, gets several times the average, and an overflowed bin
+// costs a rescan of the whole scene (54 us of a 145 us frame of 16 rooms, 150
+// to 250 of 1000 us on 512 uneven environments).  So a bin holds all triangles
+// of its scene, up to kSkewCap, as long as the scene's entries stay within 2
+// MB or kSkew times their number (64 bytes per triangle, beside the 96 of its
+// records).  Above kSkewCap it holds kMore times the factor, and at least
+// kLeast, times the average: the rescan grows with the scene, 8 ms for a bin of
+// a million triangles (at 2 times the average, frames of 1024 uneven
+// environments at random poses took 9.1 ms, at 3 times 1.9, at 4 times 1.4).
+// A long list is allocated without room to grow (it had half as much again),
+// so this costs a third more memory than it did.  A factor below 1 asks for
+// bins smaller than the average: it gets exactly its share, as does every scene
+// where the wide list would not fit a quarter of the memory that is free beside
+// all other arrays.
+uint64_t bin_capacities(gbr_renderer* r, std::vector<RasterItem>& ritems, bool wide) {
+  constexpr double kSkew = 8.0, kSkewCap = 4096.0, kSceneEntries = 1 << 19;
+  constexpr double kMore = 2.0, kLeast = 4.0;
+  const double factor = r->tun.bin_capacity_factor;
+  uint64_t entries = 0;
+  size_t k = 0;
+  for (uint32_t si = 0; si < r->scene_count(); ++si) {
+    SceneDesc& sd = r->scene_desc[si];
+    size_t end = k;
+    while (end < ritems.size() && ritems[end].scene == si) ++end;
+    const size_t nb = end - k;
+    const double prim = (double)sd.prim_count, mean = prim / (double)nb;
+    double per_bin = mean * factor;
+    if (wide && factor >= 1.0)
+      per_bin = std::min(prim, std::max(mean * std::max(kMore * factor, kLeast),
+                                        std::min(kSkewCap, std::max(kSkew * per_bin,
+                                                                    kSceneEntries / (double)nb))));
+    uint32_t cap = (uint32_t)std::min<double>(std::max<double>(per_bin, r->tun.min_bin_capacity), 1u << 24);
+    cap = (cap + 63) & ~63u;
+    sd.bin_cap = cap;
+    sd.entry_base = entries;
+    for (; k < end; ++k) {
+      ritems[k].bin_cap = cap;
+      ritems[k].entries = entries;
+      entries += cap;
+    }
+  }
+  return entries;
+}
+
 gbr_status rebuild_structure(gbr_renderer* r) {
   hipStream_t s = r->stream;
   const uint32_t nsc = r->scene_count();
@@ -458,7 +506,7 @@ gbr_status rebuild_structure(gbr_renderer* r) {
   std::vector<RasterItem> ritems;
   r->scene_node_base.assign(nsc, 0);
   r->scene_desc.assign(nsc, SceneDesc{});
-  uint64_t bins = 0, entries = 0, tris = 0;
+  uint64_t bins = 0, tris = 0;
   for (uint32_t si = 0; si < nsc; ++si) {
     Scene& sc = r->scenes[si];
     const uint32_t nbase = (uint32_t)parents.size();
@@ -537,25 +585,7 @@ gbr_status rebuild_structure(gbr_renderer* r) {
     tris += prim;
     const uint32_t nb = (uint32_t)(bins_x * bins_y);
     sd.bin_base = (uint32_t)bins;
-    // A camera sees its triangles unevenly: a bin of a scene with few
-    // triangles, or with many bins, gets several times the average, and an
-    // overflowed bin costs a rescan of the whole scene (54 us of a 145 us
-    // frame of 16 rooms, 150 to 250 of 1000 us on 512 uneven environments).
-    // So a bin holds all triangles of its scene, up to kSkewCap, as long as
-    // the scene's entries stay within 2 MB or kSkew times their number (64
-    // bytes per triangle, beside the 96 of its records).  A factor below 1
-    // asks for bins smaller than the average: it gets exactly its share.
-    constexpr double kSkew = 8.0, kSkewCap = 4096.0, kSceneEntries = 1 << 19;
-    double per_bin = (double)prim / nb * r->tun.bin_capacity_factor;
-    if (r->tun.bin_capacity_factor >= 1.0f)
-      per_bin = std::max(per_bin, std::min({(double)prim, kSkewCap,
-                                            std::max(kSkew * per_bin, kSceneEntries / nb)}));
-    uint32_t cap = (uint32_t)std::min<double>(std::max<double>(per_bin, r->tun.min_bin_capacity), 1u << 24);
-    cap = (cap + 63) & ~63u;
-    sd.bin_cap = cap;
-    sd.entry_base = entries;
     bins += nb;
-    entries += (uint64_t)nb * cap;
     for (uint32_t b = 0; b < nb; ++b) {
       RasterItem ri{};
       ri.scene = si;
@@ -565,17 +595,39 @@ gbr_status rebuild_structure(gbr_renderer* r) {
       ri.y0 = (int16_t)(by * B);
       ri.x1 = (int16_t)(std::min(bx * B + B, vw) - 1);
       ri.y1 = (int16_t)(std::min(by * B + B, vh) - 1);
-      ri.bin_cap = cap;
       ri.plane_offset = sd.plane_offset;
       ri.width = vw;
       ri.height = vh;
-      ri.entries = sd.entry_base + (uint64_t)b * cap;
       ri.rec_base = sd.rec_base;
       ri.stride = W;
       ri.planes = sd.planes;
       ritems.push_back(ri);
     }
   }
+  // the arrays that grow with the triangles, then the bins' entries in what
+  // is left
+  TRY(r->d_rrecs.reserve(std::max<uint64_t>(tris, 1)));
+  TRY(r->d_srecs.reserve(std::max<uint64_t>(tris, 1)));
+  // every primitive is listed at most once; the sub-triangle pool gives list
+  // slot i the fan slots [7 i, 7 i + 7) and is bounded (bins of a fan past
+  // it fall back to the exact rescan)
+  r->clipped_cap = (uint32_t)std::max<uint64_t>(tris, 1);
+  r->sub_cap = (uint32_t)std::min<uint64_t>(7 * std::max<uint64_t>(tris, 1024), 7u << 20);
+  // the clip pass's fast entries cover the first slots of the list (beyond
+  // them it reads a primitive through its draw)
+  r->clip_fast_cap = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(tris, 1), 1u << 20);
+  TRY(r->d_clipped.reserve(r->clipped_cap));
+  TRY(r->d_clip_fast.reserve(r->clip_fast_cap));
+  TRY(r->d_sub_recs.reserve(r->sub_cap));
+  TRY(r->d_sub_prims.reserve(r->sub_cap));
+  constexpr uint64_t kLongList = 64ull << 20;  // entries
+  uint64_t entries = bin_capacities(r, ritems, true);
+  if (entries > kLongList && entries > r->d_bin_entries.cap) {
+    size_t free_bytes = 0, total_bytes = 0;
+    HIP_TRY(hipMemGetInfo(&free_bytes, &total_bytes));
+    if (entries * sizeof(uint32_t) > free_bytes / 4) entries = bin_capacities(r, ritems, false);
+  }
+  TRY(r->d_bin_entries.reserve(std::max<uint64_t>(entries, 1), false, nullptr, entries <= kLongList));
   r->n_nodes = (uint32_t)parents.size();
   r->n_items = (uint32_t)items.size();
   r->n_ritems = (uint32_t)ritems.size();
@@ -620,22 +672,7 @@ gbr_status rebuild_structure(gbr_renderer* r) {
   TRY(r->d_active.reserve(std::max<size_t>(ritems.size(), 1)));
   TRY(r->d_overflow.reserve(std::max<size_t>(ritems.size(), 1)));
   HIP_TRY(hipMemsetAsync(r->d_bin_heavy.ptr, 0, r->d_bin_heavy.cap * sizeof(uint32_t), s));
-  TRY(r->d_bin_entries.reserve(std::max<uint64_t>(entries, 1)));
   r->entries_cap = entries;
-  TRY(r->d_rrecs.reserve(std::max<uint64_t>(tris, 1)));
-  TRY(r->d_srecs.reserve(std::max<uint64_t>(tris, 1)));
-  // every primitive is listed at most once; the sub-triangle pool gives list
-  // slot i the fan slots [7 i, 7 i + 7) and is bounded (bins of a fan past
-  // it fall back to the exact rescan)
-  r->clipped_cap = (uint32_t)std::max<uint64_t>(tris, 1);
-  r->sub_cap = (uint32_t)std::min<uint64_t>(7 * std::max<uint64_t>(tris, 1024), 7u << 20);
-  // the clip pass's fast entries cover the first slots of the list (beyond
-  // them it reads a primitive through its draw)
-  r->clip_fast_cap = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(tris, 1), 1u << 20);
-  TRY(r->d_clipped.reserve(r->clipped_cap));
-  TRY(r->d_clip_fast.reserve(r->clip_fast_cap));
-  TRY(r->d_sub_recs.reserve(r->sub_cap));
-  TRY(r->d_sub_prims.reserve(r->sub_cap));
   HIP_TRY(hipStreamSynchronize(s));
   r->structure_dirty = false;
   r->nodes_dirty = true;  // new node arrays: every absolute transform is stale
