@@ -2736,11 +2736,7 @@ __device__ __forceinline__ void abs_bound(const float* M, const float* PV, float
 // (Single-address atomics from every wave serialise at the memory side and
 // cost more than the work they count.)  Every thread of the block calls it
 // once, with its flags; slot[l] is valid where flag[l] is set.
-// 512: with 1024, 168k items were 165 workgroups on 256 CUs, and 256 doubles
-// the atomics (k_cull 36 / 29 / 33 us for 337k items with 1024 / 512 / 256,
-// 11.2 / 8.2 / 7.3 for 21k, 19.5 / 20.7 / 21.3 for 168k; k_cull_hiz 9.8 / 8.7 /
-// 9.7, 7.5 / 6.4 / 6.1 and 9.1 / 7.7 / 7.5; frames 0.6 to 1.4% faster).
-constexpr int kListBlock = 512;
+constexpr int kListBlock = 1024;
 
 template <int L>
 __device__ __forceinline__ void block_slots(uint32_t* const (&counter)[L], const bool (&flag)[L],
