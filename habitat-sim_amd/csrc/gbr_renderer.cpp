@@ -504,6 +504,7 @@ gbr_status rebuild_structure(gbr_renderer* r) {
   std::vector<WorkItem> items;
   std::vector<ItemBounds> bounds;
   std::vector<RasterItem> ritems;
+  r->moved.clear();  // (of a frame that failed: every transform is uploaded below)
   r->scene_node_base.assign(nsc, 0);
   r->scene_desc.assign(nsc, SceneDesc{});
   uint64_t bins = 0, tris = 0;

@@ -1,0 +1,56 @@
+"""libgbr.so over tests/cpp/hip_host.cpp: the library's host code with HIP calls
+served from host memory.  Import it before habitat_sim_amd loads the library, in
+a process of its own (tests/test_host_runtime.py starts one per case)."""
+import ctypes
+import os
+import sys
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+for p in (ROOT, os.path.join(ROOT, "habitat-sim_amd"), os.path.join(ROOT, "tests")):
+    if p not in sys.path:
+        sys.path.insert(0, p)
+
+LIB = os.path.join(ROOT, "tests", "cpp", "_build", "libhip_host.so")
+_lib = ctypes.CDLL(LIB, mode=ctypes.RTLD_GLOBAL)
+_lib.hip_host_calls.restype = ctypes.c_int64
+_lib.hip_host_used.restype = ctypes.c_int64
+_HOOK = ctypes.CFUNCTYPE(None, ctypes.c_char_p, ctypes.POINTER(ctypes.c_uint32), ctypes.POINTER(ctypes.c_void_p))
+_hook = None
+
+
+class InputArgs(ctypes.Structure):
+    """gbr_device.h InputArgs, the argument of k_inputs."""
+    _fields_ = [("src", ctypes.c_void_p), ("dst", ctypes.c_void_p * 6), ("end", ctypes.c_uint32 * 6),
+                ("nodes", ctypes.POINTER(ctypes.c_uint32)), ("transforms", ctypes.POINTER(ctypes.c_float)),
+                ("local", ctypes.c_void_p), ("n_nodes", ctypes.c_uint32)]
+
+
+def on_launch(kernel: str, argument, function) -> None:
+    """Calls function(arguments[0] as an `argument` structure, grid, arguments)
+    at each launch of a kernel whose (mangled) name holds `kernel`."""
+    global _hook
+
+    def hook(name, grid, args):
+        if kernel in name.decode():
+            function(argument.from_address(args[0]) if argument else None, tuple(grid[:3]), args)
+
+    _hook = _HOOK(hook)
+    _lib.hip_host_hook(_hook)
+
+
+def fail(call: str, after: int = 0) -> None:
+    """The HIP call of this name fails once, after `after` more that succeed."""
+    _lib.hip_host_fail(call.encode(), ctypes.c_int64(after))
+
+
+def calls(call: str) -> int:
+    return _lib.hip_host_calls(call.encode())
+
+
+def device_memory(limit: int, free: int) -> None:
+    """hipMalloc fails beyond `limit` bytes in all; hipMemGetInfo reports `free`."""
+    _lib.hip_host_memory(ctypes.c_int64(limit), ctypes.c_int64(free))
+
+
+def device_memory_used() -> int:
+    return _lib.hip_host_used()

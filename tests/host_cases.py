@@ -1,0 +1,61 @@
+"""Cases of tests/test_host_runtime.py, each run in a process of its own as
+``python host_cases.py CASE``: the library's host code without a GPU."""
+import sys
+
+import hip_host
+import numpy as np
+import synth
+from habitat_sim_amd import RendererConfiguration, RendererStandalone
+from habitat_sim_amd import _native as N
+from habitat_sim_amd import math3d as m3
+
+
+def _triangle():
+    pos = np.array([(-1, -1, -3), (1, -1, -3), (0, 1, -3)], np.float32)
+    return synth.mesh_file([(pos, np.arange(3, dtype=np.uint32), None, None, 0)], [synth.flat((1, 1, 1, 1))])
+
+
+def _scenes(tile, grid, nodes):
+    r = RendererStandalone(RendererConfiguration().set_tile_size_count(tile, grid))
+    assert r.add_file_data(_triangle())
+    for s in range(grid[0] * grid[1]):
+        for k in range(nodes):
+            r.add_node_hierarchy(s, "m0", None, k + 1)
+    return r
+
+
+def moved_nodes_of_a_failed_frame():
+    """A frame that ends at an allocation leaves nothing of its moved nodes to
+    the next one, whose scenes may have lost them: that one sends everything."""
+    moved = []
+    hip_host.on_launch("k_inputs", hip_host.InputArgs, lambda a, grid, args: moved.append(
+        {a.nodes[i]: list(a.transforms[16 * i:16 * i + 16]) for i in range(a.n_nodes)}))
+    r = _scenes((32, 32), (3, 1), 3000)
+    r.draw()
+    assert moved.pop() == {}
+    # more moved nodes than the pinned block has room for: it is allocated again
+    for s in range(3):
+        r.transformations(s)._a[:] = m3.translation((0.0, 0.0, -1.0 - s))
+    hip_host.fail("hipHostMalloc")
+    try:
+        r.draw()
+        raise AssertionError("the frame did not fail")
+    except N.GbrError as e:
+        assert e.status == N.ERR_OOM, e
+    assert not moved
+    r.clear(1)
+    r.clear(2)
+    r.draw()
+    assert moved.pop() == {}, "nodes of the failed frame were sent again"
+    # and later frames send what moves in them
+    t = m3.translation((1.0, 2.0, 3.0))
+    r.transformations(0)[5] = t
+    r.draw()
+    sent = moved.pop()
+    assert list(sent) == [5] and np.array_equal(np.float32(sent[5]), np.asarray(t, np.float32).reshape(-1)), sent
+    r.close()
+
+
+if __name__ == "__main__":
+    globals()[sys.argv[1]]()
+    print("case passed:", sys.argv[1])
