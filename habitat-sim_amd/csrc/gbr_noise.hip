@@ -89,6 +89,14 @@ Divider make_divider(uint32_t d) {
   return {(uint32_t)(((1ull << (31 + s)) + d - 1) / d), s - 1};
 }
 
+// the largest float that is a row or column number of a side of n pixels:
+// n - 1 itself up to 2^24, beyond which (float)(n - 1) may round up to n and
+// a pixel clamped to it lies outside the image
+float last_index(int n) {
+  const float f = (float)(n - 1);
+  return (double)f > (double)(n - 1) ? std::nextafter(f, 0.0f) : f;
+}
+
 __device__ __forceinline__ uint32_t divide(uint32_t n, Divider d) { return __umulhi(n, d.mul) >> d.shift; }
 
 // the disparity step in the general arithmetic
@@ -108,8 +116,8 @@ struct RedwoodArgs {
   uint32_t total;        // pixels, < 2^31
   uint32_t npx, W;
   Divider by_npx, by_w;
-  float xmax, ymax;      // W - 1, H - 1
-  double rx, ry;         // 1 / xmax, 1 / ymax
+  float xmax, ymax;      // last_index() of W and H
+  double rx, ry;         // 1 / (W - 1), 1 / (H - 1), the sides rounded to floats
   float mult, mult4;     // the noise multiplier, and a quarter of it
   uint64_t seed, call, first;  // first: the generator's number of pixel 0
 };
@@ -286,10 +294,10 @@ gbr_status launch(gbr_redwood* m, const float* depth, int32_t images, int32_t ro
   a.W = (uint32_t)cols;
   a.by_npx = gbr::make_divider(a.npx);
   a.by_w = gbr::make_divider(a.W);
-  a.xmax = (float)(cols - 1);
-  a.ymax = (float)(rows - 1);
-  a.rx = 1.0 / (double)a.xmax;
-  a.ry = 1.0 / (double)a.ymax;
+  a.xmax = gbr::last_index(cols);
+  a.ymax = gbr::last_index(rows);
+  a.rx = 1.0 / (double)(float)(cols - 1);
+  a.ry = 1.0 / (double)(float)(rows - 1);
   a.mult = m->mult;
   a.mult4 = m->mult * 0.25f;
   a.seed = m->seed;

@@ -25,6 +25,14 @@ class InputArgs(ctypes.Structure):
                 ("local", ctypes.c_void_p), ("n_nodes", ctypes.c_uint32)]
 
 
+class RedwoodArgs(ctypes.Structure):
+    """The head of gbr_noise.hip RedwoodArgs, the argument of k_redwood."""
+    _fields_ = [("depth", ctypes.c_void_p), ("model", ctypes.c_void_p), ("normals", ctypes.c_void_p),
+                ("out", ctypes.c_void_p), ("total", ctypes.c_uint32), ("npx", ctypes.c_uint32),
+                ("W", ctypes.c_uint32), ("by_npx", ctypes.c_uint32 * 2), ("by_w", ctypes.c_uint32 * 2),
+                ("xmax", ctypes.c_float), ("ymax", ctypes.c_float)]
+
+
 def on_launch(kernel: str, argument, function) -> None:
     """Calls function(arguments[0] as an `argument` structure, grid, arguments)
     at each launch of a kernel whose (mangled) name holds `kernel`."""

@@ -1,5 +1,6 @@
 """Cases of tests/test_host_runtime.py, each run in a process of its own as
 ``python host_cases.py CASE``: the library's host code without a GPU."""
+import ctypes
 import sys
 
 import hip_host
@@ -54,6 +55,30 @@ def moved_nodes_of_a_failed_frame():
     sent = moved.pop()
     assert list(sent) == [5] and np.array_equal(np.float32(sent[5]), np.asarray(t, np.float32).reshape(-1)), sent
     r.close()
+
+
+def redwood_stays_inside_wide_images():
+    """The last row and column that k_redwood clamps to lie inside the image at
+    every size: as floats, sides beyond 2^24 pixels may round up."""
+    seen = []
+    hip_host.on_launch("k_redwood", hip_host.RedwoodArgs,
+                       lambda a, grid, args: seen.append((a.npx, a.W, int(a.xmax), int(a.ymax))))
+    h = ctypes.c_void_p()
+    table = np.ones(N.REDWOOD_MODEL_FLOATS, np.float32)
+    N.call("gbr_redwood_create", table.ctypes.data, 0, 1.0, 1, ctypes.byref(h))
+    image = ctypes.c_void_p(1 << 20)  # never read: kernels do not run
+    sides = [2, 3, 640, (1 << 23) - 1, 1 << 23, (1 << 23) + 2, (1 << 24) - 1, 1 << 24, (1 << 24) + 1, (1 << 24) + 2,
+             16777220, 33554437, (1 << 29) - 3]
+    for side in sides:
+        for rows, cols in ((3, side), (side, 3)):
+            N.call("gbr_redwood_simulate", h, image, 1, rows, cols, image, None)
+            npx, w, xmax, ymax = seen.pop()
+            assert (npx, w) == (rows * cols, cols)
+            for last, n in ((xmax, cols), (ymax, rows)):
+                f = np.float32(n - 1)
+                assert last <= n - 1, f"{rows} x {cols}: clamped to {last}"
+                assert last == int(f if int(f) <= n - 1 else np.nextafter(f, np.float32(0))), (last, n)
+    N.call("gbr_redwood_destroy", h)
 
 
 if __name__ == "__main__":
