@@ -1812,15 +1812,18 @@ __device__ __forceinline__ uint32_t shade_pixel(const FrameParams& p, const Reso
 // --------------------------------------------------------------------------
 
 
-// forces the exact rescan for every bin the rectangle touches
+// forces the exact rescan for every bin the rectangle touches.  The count is
+// raised to cap + 1, never added to: a bin may be forced more than a million
+// times a frame (every fan past the record slots), and cap + 1 each time
+// would take its count around 2^32, back below the capacity and listed again.
 __device__ __forceinline__ void overflow_rect(const FrameParams& p, const SceneDesc& sc,
                                               const PixRect& r, int phase) {
   const int sh = p.bin_shift;
   for (int by = r.y0 >> sh; by <= (r.y1 >> sh); ++by)
     for (int bx = r.x0 >> sh; bx <= (r.x1 >> sh); ++bx) {
       const uint32_t gbin = sc.bin_base + (uint32_t)(by * sc.bins_x + bx);
-      const uint32_t old = atomicAdd(&p.bin_count[gbin], sc.bin_cap + 1u);
-      note_heavy(p, gbin, old, sc.bin_cap + 1u, phase, sc.bin_cap);
+      const uint32_t old = atomicMax(&p.bin_count[gbin], sc.bin_cap + 1u);
+      if (old <= sc.bin_cap) note_heavy(p, gbin, old, sc.bin_cap + 1u - old, phase, sc.bin_cap);
     }
 }
 

@@ -312,3 +312,36 @@ def test_readback_rectangles_strides_and_large_images():
         r.linear_depth_image_into((x0, y0, x1, y1), z)
         np.testing.assert_array_equal(z, lin[y0:y1, x0:x1])
     r.close()
+
+
+def test_a_bin_forced_to_the_rescan_more_often_than_a_word_holds():
+    """More clipped primitives than record slots (2^20; every triangle here is
+    a work item too wide for the vertex cache, which the clip pass takes), all
+    in the tile's one bin: each one past the slots forces the bin's exact
+    rescan.  Their number is the first for which adding the capacity and one
+    each time would take the 32-bit count past 2^32 to below the capacity."""
+    slots = 1 << 20
+    extra = next(k for k in range(4000, 5000)
+                 if (slots + k * (((slots + k + 63) & ~63) + 1)) % (1 << 32) <= ((slots + k + 63) & ~63))
+    n = slots + extra
+    rng = np.random.default_rng(17)
+    tile = (32, 32)
+    # right triangles of three pixels a side (each holds a pixel centre), facing the camera
+    corner = rng.uniform(0.0, 29.0, (n, 1, 2)) + np.array([(0, 0), (3, 0), (0, 3)])
+    pos = np.concatenate([corner / 16.0 - 1.0, rng.uniform(-0.9, 0.9, (n, 3, 1))], -1).reshape(-1, 3)
+    where = rng.permutation(3 * n).astype(np.uint32)  # vertex k of the list lies at where[k]
+    verts = np.empty((3 * n, 3), np.float32)
+    verts[where] = pos
+    mesh = (verts, where, None, rng.uniform(0, 1, (3 * n, 4)), 0)
+    fd = synth.mesh_file([mesh], [synth.flat((1, 1, 1, 1))])
+    r, o = _pair(tile, (1, 1), planes=N.PLANE_COLOR | N.PLANE_DEPTH | N.PLANE_SEMANTIC)
+    for x in (r, o):
+        assert x.add_file_data(fd)
+        x.add_node_hierarchy(0, "m0", None, 3)
+        x.update_camera(0, m3.identity(), m3.identity())
+    for _ in range(2):
+        _draw(r, o)
+        _same(r, o, ("color", "depth", "semantic"))
+        st = r.frame_stats()
+        assert st["triangles_clipped"] > slots and st["overflowed_bins"] == 1, st
+    r.close()
