@@ -328,7 +328,7 @@ void set_sampler(TextureDesc& td, uint32_t min_filter, uint32_t mag_filter, uint
                  uint32_t wrap_t) {
   constexpr uint32_t kLinear = 9729, kNearest = 9728, kNearestMipNearest = 9984,
                      kLinearMipNearest = 9985, kNearestMipLinear = 9986, kLinearMipLinear = 9987;
-  constexpr uint32_t kClamp = 33071, kMirror = 33648;
+  constexpr uint32_t kClamp = 33071, kMirror = 33648, kRepeat = 10497;
   td.filter = 0;
   if (mag_filter == kLinear) td.filter |= kTexMagLinear;
   if (min_filter == kLinear || min_filter == kLinearMipNearest || min_filter == kLinearMipLinear)
@@ -342,10 +342,11 @@ void set_sampler(TextureDesc& td, uint32_t min_filter, uint32_t mag_filter, uint
   auto axis = [&](uint32_t mode, int32_t size, int32_t& wrap_or) {
     wrap_or = mode == kClamp ? -1 : 0;
     if (mode != kClamp && (mode == kMirror || (size & (size - 1)) != 0)) td.filter |= kTexWrapSlow;
+    // (a mode of neither kind repeats, whatever the file's number is)
+    return mode == kClamp || mode == kMirror ? mode : kRepeat;
   };
-  axis(wrap_s, td.width, td.wrap_or_s);
-  axis(wrap_t, td.height, td.wrap_or_t);
-  td.wraps = (wrap_s & 0xffffu) | (wrap_t << 16);
+  td.wraps = axis(wrap_s, td.width, td.wrap_or_s);
+  td.wraps |= axis(wrap_t, td.height, td.wrap_or_t) << 16;
 }
 
 void set_level(TextureDesc& td, int level, size_t offset) {

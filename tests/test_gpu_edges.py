@@ -345,3 +345,26 @@ def test_a_bin_forced_to_the_rescan_more_often_than_a_word_holds():
         st = r.frame_stats()
         assert st["triangles_clipped"] > slots and st["overflowed_bins"] == 1, st
     r.close()
+
+
+@pytest.mark.parametrize("wrap", [GL_CLAMP_TO_EDGE, GL_MIRRORED_REPEAT, GL_REPEAT])
+@pytest.mark.parametrize("size", [(5, 3), (8, 4)])
+def test_wrap_modes_that_are_none(wrap, size):
+    """A file may carry any number as a wrap mode; one that is none of GL's
+    repeats, also where its low 16 bits are another mode's."""
+    rng = np.random.default_rng(3)
+    t = synth.texture(_levels(rng, *size), min_filter=GL_LINEAR, mag_filter=GL_LINEAR, wrap=wrap + (1 << 16))
+    t.wrap_t = wrap + (5 << 16)
+    pos = np.array([(-1, -1, -2), (1, -1, -2), (1, 1, -2), (-1, 1, -2)], np.float32)
+    uv = np.array([(-1.6, -1.3), (2.7, -1.3), (2.7, 2.2), (-1.6, 2.2)], np.float32)
+    fd = synth.mesh_file([(pos, np.array([0, 1, 2, 0, 2, 3], np.uint32), uv, None, 0)],
+                         [synth.flat((1, 1, 1, 1), texture=0)], [t])
+    tile = (61, 47)
+    r, o = _pair(tile, (1, 1))
+    for x in (r, o):
+        assert x.add_file_data(fd)
+        x.add_node_hierarchy(0, "m0", None, 1)
+        _camera(x, 0, tile)
+    _draw(r, o)
+    _same(r, o)
+    r.close()
