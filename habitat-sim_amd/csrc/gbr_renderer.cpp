@@ -432,8 +432,7 @@ gbr_status upload_assets(gbr_renderer* r) {
   return GBR_OK;
 }
 
-// Gives every bin its capacity and its place in the entry list; returns the
-// list's length.
+// Entries per bin of a scene of `prims` triangles in `nb` bins.
 //
 // A camera sees its triangles unevenly: a bin of a scene with few triangles,
 // or with many bins, gets several times the average, and an overflowed bin
@@ -445,36 +444,60 @@ gbr_status upload_assets(gbr_renderer* r) {
 // kLeast, times the average: the rescan grows with the scene, 8 ms for a bin of
 // a million triangles (at 2 times the average, frames of 1024 uneven
 // environments at random poses took 9.1 ms, at 3 times 1.9, at 4 times 1.4).
-// A long list is allocated without room to grow (it had half as much again),
-// so this costs a third more memory than it did.  A factor below 1 asks for
-// bins smaller than the average: it gets exactly its share, as does every scene
-// where the wide list would not fit a quarter of the memory that is free beside
-// all other arrays.
-uint64_t bin_capacities(gbr_renderer* r, std::vector<RasterItem>& ritems, bool wide) {
+// A long list is allocated without room to grow, so at the default this takes
+// a third more memory than twice the average with half as much again.  A
+// factor below kWideFactor, the default, bounds the list's memory: bins get
+// exactly its share, as they do in every scene where the wide list would not
+// fit a quarter of the memory that is free beside all other arrays.
+constexpr float kWideFactor = 2.0f;
+
+uint32_t bin_capacity(const gbr_tuning& t, uint32_t prims, uint32_t nb, bool wide) {
   constexpr double kSkew = 8.0, kSkewCap = 4096.0, kSceneEntries = 1 << 19;
   constexpr double kMore = 2.0, kLeast = 4.0;
-  const double factor = r->tun.bin_capacity_factor;
+  const double factor = t.bin_capacity_factor;
+  const double prim = (double)prims, mean = prim / (double)nb;
+  double per_bin = mean * factor;
+  if (wide && t.bin_capacity_factor >= kWideFactor)
+    per_bin = std::min(prim, std::max(mean * std::max(kMore * factor, kLeast),
+                                      std::min(kSkewCap, std::max(kSkew * per_bin, kSceneEntries / (double)nb))));
+  const uint32_t cap = (uint32_t)std::min<double>(std::max<double>(per_bin, t.min_bin_capacity), 1u << 24);
+  return (cap + 63) & ~63u;
+}
+
+uint32_t bins_across(int pixels, int B) { return (uint32_t)((pixels + B - 1) / B); }
+
+// bins of scene si at a bin size of B pixels
+uint32_t scene_bins(const gbr_renderer* r, uint32_t si, int B) {
+  const Scene& sc = r->scenes[si];
+  const int vw = sc.vp_w ? sc.vp_w : r->cfg.tile_size[0], vh = sc.vp_h ? sc.vp_h : r->cfg.tile_size[1];
+  return bins_across(vw, B) * bins_across(vh, B);
+}
+
+// whether two tunings give every bin of the frame last laid out the same
+// capacity (they have the same bins)
+bool same_capacities(const gbr_renderer* r, const gbr_tuning& a, const gbr_tuning& b) {
+  for (uint32_t si = 0; si < (uint32_t)r->scene_desc.size(); ++si) {
+    const uint32_t prims = r->scene_desc[si].prim_count, nb = scene_bins(r, si, a.bin_size);
+    if (bin_capacity(a, prims, nb, true) != bin_capacity(b, prims, nb, true)) return false;
+  }
+  return true;
+}
+
+// Gives every bin its capacity and its place in the entry list; returns the
+// list's length.
+uint64_t bin_capacities(gbr_renderer* r, std::vector<RasterItem>& ritems, bool wide) {
   uint64_t entries = 0;
   size_t k = 0;
   for (uint32_t si = 0; si < r->scene_count(); ++si) {
     SceneDesc& sd = r->scene_desc[si];
     size_t end = k;
     while (end < ritems.size() && ritems[end].scene == si) ++end;
-    const size_t nb = end - k;
-    const double prim = (double)sd.prim_count, mean = prim / (double)nb;
-    double per_bin = mean * factor;
-    if (wide && factor >= 1.0)
-      per_bin = std::min(prim, std::max(mean * std::max(kMore * factor, kLeast),
-                                        std::min(kSkewCap, std::max(kSkew * per_bin,
-                                                                    kSceneEntries / (double)nb))));
-    uint32_t cap = (uint32_t)std::min<double>(std::max<double>(per_bin, r->tun.min_bin_capacity), 1u << 24);
-    cap = (cap + 63) & ~63u;
-    sd.bin_cap = cap;
+    sd.bin_cap = bin_capacity(r->tun, sd.prim_count, (uint32_t)(end - k), wide);
     sd.entry_base = entries;
     for (; k < end; ++k) {
-      ritems[k].bin_cap = cap;
+      ritems[k].bin_cap = sd.bin_cap;
       ritems[k].entries = entries;
-      entries += cap;
+      entries += sd.bin_cap;
     }
   }
   return entries;
@@ -491,9 +514,7 @@ gbr_status rebuild_structure(gbr_renderer* r) {
   // appends them straight to the global bins otherwise
   r->lds_bins = 0;
   for (uint32_t si = 0; si < nsc; ++si) {
-    const Scene& sc = r->scenes[si];
-    const int vw = sc.vp_w ? sc.vp_w : W, vh = sc.vp_h ? sc.vp_h : H;
-    const uint32_t nb = (uint32_t)(((vw + B - 1) / B) * ((vh + B - 1) / B));
+    const uint32_t nb = scene_bins(r, si, B);
     if (nb <= (uint32_t)kMaxSceneBins) r->lds_bins = std::max(r->lds_bins, nb);
   }
   r->setup_bpc = setup_blocks_per_cu(r->lds_bins);
@@ -527,7 +548,7 @@ gbr_status rebuild_structure(gbr_renderer* r) {
         if (sc.draws[i].batch == b) order.push_back(i);
     SceneDesc& sd = r->scene_desc[si];
     const int vw = sc.vp_w ? sc.vp_w : W, vh = sc.vp_h ? sc.vp_h : H;
-    const int bins_x = (vw + B - 1) / B, bins_y = (vh + B - 1) / B;
+    const int bins_x = (int)bins_across(vw, B), bins_y = (int)bins_across(vh, B);
     sd.width = vw;
     sd.height = vh;
     sd.guard_x = kGuardPx / ((float)vw * 0.5f);
@@ -1244,7 +1265,7 @@ gbr_status gbr_tuning_init(gbr_tuning* t) {
   std::memset(t, 0, sizeof *t);
   t->bin_size = 32;
   t->chunk_triangles = kChunkTris;
-  t->bin_capacity_factor = 2.0f;
+  t->bin_capacity_factor = kWideFactor;
   t->min_bin_capacity = 256;
   t->cull_mode = GBR_CULL_NONE;
   t->queue_grain = 4;
@@ -2063,7 +2084,10 @@ gbr_status gbr_autotune(gbr_renderer* r, const gbr_autotune_params* params,
   report->candidates = 1;
   // candidate values per parameter
   const int bins[] = {8, 16, 32};
-  const float caps[] = {1.0f, 1.5f, 2.0f, 3.0f};
+  // (a smaller list than the default's is never faster than one that holds the
+  // frame, and slower at the first camera that overflows it: a factor below it
+  // is the caller's choice)
+  const float caps[] = {kWideFactor, 1.5f * kWideFactor};
   const int lanes[] = {32, 64, 96, 128, 192};
   const int grains[] = {1, 2, 4, 8, 16};
   const int modes[] = {0, 1};
@@ -2073,7 +2097,7 @@ gbr_status gbr_autotune(gbr_renderer* r, const gbr_autotune_params* params,
   const int nparams = best.cull_mode == GBR_CULL_LEARNED ? 7 : 6;
   for (int pass = 0; pass < params->passes; ++pass) {
     for (int param = 0; param < nparams; ++param) {
-      const int n = param == 0 ? 3 : param == 1 ? 4 : param == 2 ? 5 : param == 3 ? 5 : param == 4 ? 2
+      const int n = param == 0 ? 3 : param == 1 ? 2 : param == 2 ? 5 : param == 3 ? 5 : param == 4 ? 2
                     : param == 5 ? 5 : 4;
       for (int k = 0; k < n; ++k) {
         gbr_tuning t = best;
@@ -2086,7 +2110,7 @@ gbr_status gbr_autotune(gbr_renderer* r, const gbr_autotune_params* params,
           case 5: t.heavy_entries = heavies[k]; break;
           default: t.proposal_threshold = thresholds[k]; break;
         }
-        if (std::memcmp(&t, &best, sizeof t) == 0) continue;
+        if (std::memcmp(&t, &best, sizeof t) == 0 || (param == 1 && same_capacities(r, t, best))) continue;
         float ms = 0.0f;
         TRY(time_tuning(r, t, *params, &ms));
         ++report->candidates;

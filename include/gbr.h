@@ -112,9 +112,10 @@ typedef struct gbr_scene_stats_info {
 typedef struct gbr_tuning {
   int32_t bin_size;           /* screen bin edge in pixels: 8, 16 or 32 */
   int32_t chunk_triangles;    /* triangles per setup work item: 1..1024 */
-  float bin_capacity_factor;  /* per-bin entry capacity relative to tris/bins; from 1
-                                 on, bins get several times that, bounded per bin
-                                 and scene (a camera sees triangles unevenly) */
+  float bin_capacity_factor;  /* per-bin entry capacity relative to tris/bins: exactly
+                                 that share below 2 (bounds memory); from 2 (default)
+                                 on several times it, bounded per bin and scene (a
+                                 camera sees triangles unevenly) */
   int32_t min_bin_capacity;   /* lower bound of the per-bin capacity */
   int32_t cull_mode;          /* GBR_CULL_* */
   int32_t queue_grain;        /* setup work items claimed per queue fetch: 1..64 */

@@ -25,6 +25,14 @@ class InputArgs(ctypes.Structure):
                 ("local", ctypes.c_void_p), ("n_nodes", ctypes.c_uint32)]
 
 
+class RasterItem(ctypes.Structure):
+    """gbr_device.h RasterItem: a bin, in the second argument of k_raster_lane."""
+    _fields_ = [("scene", ctypes.c_uint32), ("gbin", ctypes.c_uint32), ("rect", ctypes.c_int16 * 4),
+                ("bin_cap", ctypes.c_uint32), ("plane_offset", ctypes.c_uint32), ("size", ctypes.c_int32 * 2),
+                ("entries", ctypes.c_uint64), ("rec_base", ctypes.c_uint64), ("stride", ctypes.c_int32),
+                ("planes", ctypes.c_uint32), ("pad", ctypes.c_uint32 * 2)]
+
+
 class RedwoodArgs(ctypes.Structure):
     """The head of gbr_noise.hip RedwoodArgs, the argument of k_redwood."""
     _fields_ = [("depth", ctypes.c_void_p), ("model", ctypes.c_void_p), ("normals", ctypes.c_void_p),

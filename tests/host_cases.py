@@ -25,6 +25,20 @@ def _scenes(tile, grid, nodes):
     return r
 
 
+def _bins(function):
+    """Calls function(list of RasterItem) at each launch of the lane rasteriser."""
+    def launched(_, grid, args):
+        items = ctypes.cast(args[1], ctypes.POINTER(ctypes.POINTER(hip_host.RasterItem))).contents
+        function(items[:ctypes.cast(args[2], ctypes.POINTER(ctypes.c_uint32)).contents.value])
+    hip_host.on_launch("k_raster_lane", None, launched)
+
+
+def _soup(n):
+    """n triangles, three vertices each."""
+    pos = np.random.default_rng(n).uniform(-1.0, 1.0, (3 * n, 3)).astype(np.float32)
+    return synth.mesh_file([(pos, np.arange(3 * n, dtype=np.uint32), None, None, 0)], [synth.flat((1, 1, 1, 1))])
+
+
 def moved_nodes_of_a_failed_frame():
     """A frame that ends at an allocation leaves nothing of its moved nodes to
     the next one, whose scenes may have lost them: that one sends everything."""
@@ -79,6 +93,30 @@ def redwood_stays_inside_wide_images():
                 assert last <= n - 1, f"{rows} x {cols}: clamped to {last}"
                 assert last == int(f if int(f) <= n - 1 else np.nextafter(f, np.float32(0))), (last, n)
     N.call("gbr_redwood_destroy", h)
+
+
+def bin_capacity_follows_the_factor():
+    """Below 2 a bin holds the factor's share of its scene's triangles and no
+    more; from 2 (the default) on it holds more, and more with each factor."""
+    bins = []
+    _bins(bins.append)
+    n = 40000  # 16 bins of 2500 triangles on average
+    r = RendererStandalone(RendererConfiguration().set_tile_size_count((128, 128), (1, 1)))
+    assert r.add_file_data(_soup(n))
+    r.add_node_hierarchy(0, "m0", None, 1)
+    assert r.tuning().bin_capacity_factor == 2.0
+    caps = {}
+    for factor in (0.25, 0.5, 1.0, 1.25, 1.5, 1.9, 2.0, 2.5, 3.0, 6.0):
+        r.set_tuning(bin_capacity_factor=factor, graph=0)
+        r.draw()
+        (cap,) = {b.bin_cap for b in bins[-1]}
+        assert len(bins[-1]) == 16 and all(b.entries == i * cap for i, b in enumerate(bins[-1]))
+        caps[factor] = cap
+        if factor < 2.0:
+            share = int(n / 16 * np.float32(factor))
+            assert share <= cap < share + 64, (factor, cap)
+    assert sorted(set(caps.values())) == list(caps.values()), caps
+    r.close()
 
 
 if __name__ == "__main__":
