@@ -33,6 +33,10 @@ template <class T>
 struct DevBuf {
   T* ptr = nullptr;
   size_t cap = 0;
+  DevBuf() = default;
+  DevBuf(const DevBuf&) = delete;
+  DevBuf& operator=(const DevBuf&) = delete;
+  ~DevBuf() { release(); }  // (on the current device: its owner's)
   // (`spare`: with room to grow by half)
   gbr_status reserve(size_t n, bool keep = false, hipStream_t s = nullptr, bool spare = true) {
     if (n <= cap && ptr) return GBR_OK;

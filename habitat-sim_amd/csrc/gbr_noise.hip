@@ -347,7 +347,6 @@ gbr_status gbr_redwood_create(const float* model, int32_t device, float noise_mu
     if (e != hipSuccess) st = fail(GBR_ERR_DEVICE, std::string("redwood_create: ") + hipGetErrorString(e));
   }
   if (st != GBR_OK) {
-    m->d_model.release();
     delete m;
     return st;
   }
@@ -358,9 +357,6 @@ gbr_status gbr_redwood_create(const float* model, int32_t device, float noise_mu
 gbr_status gbr_redwood_destroy(gbr_redwood* m) {
   if (!m) return GBR_OK;
   (void)hipSetDevice(m->device);
-  m->d_model.release();
-  m->d_in.release();
-  m->d_out.release();
   delete m;
   return GBR_OK;
 }

@@ -1364,45 +1364,6 @@ gbr_status gbr_destroy(gbr_renderer* r) {
   (void)hipSetDevice(r->device);
   if (r->stream) (void)hipStreamSynchronize(r->stream);
   release_graph(r);
-  r->d_frame.release();
-  r->d_nodes_dirty.release();
-  DevBuf<float>* fb[] = {&r->d_pos_x, &r->d_pos_y, &r->d_pos_z, &r->d_lut, &r->d_local, &r->d_abs,
-                         &r->d_cameras, &r->d_unproj, &r->d_depth, &r->d_lin};
-  for (auto* b : fb) b->release();
-  DevBuf<uint32_t>* ub[] = {&r->d_uv16, &r->d_col8, &r->d_indices, &r->d_bin_count,
-                            &r->d_bin_entries, &r->d_color, &r->d_sem, &r->d_heavy,
-                            &r->d_bin_heavy, &r->d_active, &r->d_overflow};
-  for (auto* b : ub) b->release();
-  r->d_uv32.release();
-  r->d_col32.release();
-  r->d_texels.release();
-  r->d_textures.release();
-  r->d_materials.release();
-  r->d_draws.release();
-  r->d_rrecs.release();
-  r->d_srecs.release();
-  r->d_sub_prims.release();
-  r->d_sub_recs.release();
-  r->d_clipped.release();
-  r->d_clip_fast.release();
-  r->d_counters.release();
-  r->d_vis.release();
-  r->d_scenes.release();
-  r->d_items.release();
-  r->d_item_draws.release();
-  r->d_ritems.release();
-  r->d_parents.release();
-  r->d_stats.release();
-  r->d_caminfo.release();
-  r->vis.release();
-  r->d_fb_color.release();
-  r->d_fb_depth.release();
-  r->d_stage.release();
-  r->d_hiz.release();
-  r->d_nrm.release();
-  r->d_nmat.release();
-  r->d_lights.release();
-  r->d_scene_lights.release();
   if (r->h_inputs) (void)hipHostFree(r->h_inputs);
   for (auto& blk : r->inputs)
     if (blk.read) (void)hipEventDestroy(blk.read);

@@ -24,20 +24,6 @@ uint16_t host_f2bf(float f) {
 
 }  // namespace
 
-void VisModel::release() {
-  for (DevBuf<float>* b : {&w, &g, &m, &v, &logits, &dl, &lossr, &losses, &logits_i}) b->release();
-  for (DevBuf<uint16_t>* b : {&W1b, &W2b, &W2tb, &w3b, &Xd, &Xb, &Xbt, &H1t, &H2t, &dH2, &dH2t,
-                              &dH1t, &Xi})
-    b->release();
-  Yd.release();
-  Yb.release();
-  positives.release();
-  prop.release();
-  ready = false;
-  rows = cap = 0;
-  bcap = 0;
-}
-
 gbr_status VisModel::refresh_bf16(hipStream_t s) {
   TRY(W1b.reserve((size_t)kMlpHidden * kMlpIn));
   TRY(W2b.reserve((size_t)kMlpHidden * kMlpHidden));

@@ -62,7 +62,6 @@ struct VisModel {
   gbr_status loss_grad(const float* X, const uint8_t* labels, int rows, float pos_weight,
                        float* loss, float* grad, hipStream_t s);
   gbr_status predict(const float* X, int rows, float* out, hipStream_t s);
-  void release();
 
  private:
   gbr_status reserve_batch(int batch);

@@ -86,6 +86,7 @@ void hip_host_memory(int64_t device_limit, int64_t free_bytes) {
   g_free = free_bytes;
 }
 int64_t hip_host_used() { return g_device_used; }
+int64_t hip_host_blocks() { return (int64_t)g_blocks.size(); }
 
 // ---- modules -----------------------------------------------------------------
 void** __hipRegisterFatBinary(const void*) {

@@ -14,6 +14,7 @@ LIB = os.path.join(ROOT, "tests", "cpp", "_build", "libhip_host.so")
 _lib = ctypes.CDLL(LIB, mode=ctypes.RTLD_GLOBAL)
 _lib.hip_host_calls.restype = ctypes.c_int64
 _lib.hip_host_used.restype = ctypes.c_int64
+_lib.hip_host_blocks.restype = ctypes.c_int64
 _HOOK = ctypes.CFUNCTYPE(None, ctypes.c_char_p, ctypes.POINTER(ctypes.c_uint32), ctypes.POINTER(ctypes.c_void_p))
 _hook = None
 
@@ -70,3 +71,8 @@ def device_memory(limit: int, free: int) -> None:
 
 def device_memory_used() -> int:
     return _lib.hip_host_used()
+
+
+def memory_blocks() -> int:
+    """Device and pinned allocations not yet freed."""
+    return _lib.hip_host_blocks()

@@ -119,6 +119,41 @@ def bin_capacity_follows_the_factor():
     r.close()
 
 
+def closed_objects_free_their_memory():
+    """Device and pinned memory is all given back by close()."""
+    def renderer(tuning, lights):
+        cfg = RendererConfiguration().set_tile_size_count((64, 48), (2, 1)).set_max_light_count(lights)
+        r = RendererStandalone(cfg)
+        assert r.add_file_data(_triangle())
+        for s in range(2):
+            r.add_node_hierarchy(s, "m0", None, 1)
+        if lights:
+            r.add_light(0, 0, N.LIGHT_POINT)
+        r.vis_init(1)
+        r.set_tuning(**tuning)
+        for _ in range(2):
+            r.draw()
+        r.vis_collect()
+        r.color_image()
+        r.depth_image()
+        r.color_image_into((0, 0, 8, 8), np.zeros((8, 8, 3), np.uint8))
+        r.vis_loss_grad(np.zeros((32, N.VIS_FEATURES), np.float32), np.zeros(32, np.uint8))
+        r.close()
+
+    for tuning in (dict(), dict(cull_mode=N.CULL_HIZ), dict(cull_mode=N.CULL_LEARNED, raster_mode=1),
+                   dict(timing=1, graph=0)):
+        for lights in (0, 2):
+            renderer(tuning, lights)
+            assert hip_host.memory_blocks() == 0, (tuning, lights, hip_host.memory_blocks())
+    h = ctypes.c_void_p()
+    table = np.ones(N.REDWOOD_MODEL_FLOATS, np.float32)
+    N.call("gbr_redwood_create", table.ctypes.data, 0, 1.0, 1, ctypes.byref(h))
+    depth = np.ones((4, 6), np.float32)
+    N.call("gbr_redwood_simulate_host", h, depth.ctypes.data, 4, 6, depth.ctypes.data)
+    N.call("gbr_redwood_destroy", h)
+    assert hip_host.memory_blocks() == 0
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]]()
     print("case passed:", sys.argv[1])

@@ -9,7 +9,8 @@ import sys
 import pytest
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-CASES = ["moved_nodes_of_a_failed_frame", "redwood_stays_inside_wide_images", "bin_capacity_follows_the_factor"]
+CASES = ["moved_nodes_of_a_failed_frame", "redwood_stays_inside_wide_images", "bin_capacity_follows_the_factor",
+         "closed_objects_free_their_memory"]
 
 
 @pytest.fixture(scope="module", autouse=True)
