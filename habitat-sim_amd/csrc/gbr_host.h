@@ -15,12 +15,16 @@ namespace gbr {
 // records msg for gbr_last_error() and returns s
 gbr_status fail(gbr_status s, const std::string& msg);
 
+// (a call that fails leaves its error for the next launch's hipGetLastError()
+// to report again: it is taken here)
 #define HIP_TRY(expr)                                                                  \
   do {                                                                                 \
     hipError_t e_ = (expr);                                                            \
-    if (e_ != hipSuccess)                                                              \
+    if (e_ != hipSuccess) {                                                            \
+      (void)hipGetLastError();                                                         \
       return ::gbr::fail(e_ == hipErrorOutOfMemory ? GBR_ERR_OOM : GBR_ERR_DEVICE,     \
                          std::string(#expr) + ": " + hipGetErrorString(e_));           \
+    }                                                                                  \
   } while (0)
 
 #define TRY(expr)                    \
@@ -43,8 +47,10 @@ struct DevBuf {
     size_t ncap = std::max<size_t>(spare ? n + n / 2 : n, 64);
     T* np = nullptr;
     hipError_t e = hipMalloc(reinterpret_cast<void**>(&np), ncap * sizeof(T));
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
       return ::gbr::fail(GBR_ERR_OOM, std::string("hipMalloc: ") + hipGetErrorString(e));
+    }
     if (keep && ptr && cap) {
       (void)hipMemcpyAsync(np, ptr, cap * sizeof(T), hipMemcpyDeviceToDevice, s);
       (void)hipStreamSynchronize(s);

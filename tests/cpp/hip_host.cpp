@@ -24,6 +24,7 @@ std::map<const void*, std::string> g_kernels;
 std::map<std::string, int64_t> g_calls;
 std::map<std::string, int64_t> g_fail;  // calls left until the named one fails (0: the next)
 int64_t g_device_limit = -1, g_device_used = 0, g_free = 64ll << 30;
+int g_last_error = kSuccess;
 void (*g_hook)(const char* kernel, const uint32_t* grid, void** args) = nullptr;
 
 struct Dim3 {
@@ -44,11 +45,11 @@ bool fails(const char* name) {
   return true;
 }
 
-int allocate(void** p, size_t n, int type) {
+int allocate(const char* call, void** p, size_t n, int type) {
   *p = nullptr;
-  if (type == kDevice && g_device_limit >= 0 && g_device_used + (int64_t)n > g_device_limit) return kOutOfMemory;
-  void* m = calloc(1, n ? n : 1);
-  if (!m) return kOutOfMemory;
+  const bool full = type == kDevice && g_device_limit >= 0 && g_device_used + (int64_t)n > g_device_limit;
+  void* m = fails(call) || full ? nullptr : calloc(1, n ? n : 1);
+  if (!m) return g_last_error = kOutOfMemory;
   g_blocks[(uintptr_t)m] = {n, type};
   if (type == kDevice) g_device_used += (int64_t)n;
   *p = m;
@@ -146,7 +147,11 @@ int hipDeviceGetAttribute(int* v, int, int) {
   *v = 256;
   return kSuccess;
 }
-int hipGetLastError() { return kSuccess; }
+int hipGetLastError() {
+  const int e = g_last_error;
+  g_last_error = kSuccess;
+  return e;
+}
 const char* hipGetErrorString(int e) { return e == kOutOfMemory ? "out of memory" : e ? "error" : "no error"; }
 int hipMemGetInfo(size_t* free_bytes, size_t* total) {
   *free_bytes = *total = (size_t)g_free;
@@ -191,11 +196,9 @@ int hipEventElapsedTime(float* ms, void*, void*) {
 }
 
 // ---- memory --------------------------------------------------------------------
-int hipMalloc(void** p, size_t n) { return fails("hipMalloc") ? (*p = nullptr, kOutOfMemory) : allocate(p, n, kDevice); }
+int hipMalloc(void** p, size_t n) { return allocate("hipMalloc", p, n, kDevice); }
 int hipFree(void* p) { return release(p); }
-int hipHostMalloc(void** p, size_t n, unsigned) {
-  return fails("hipHostMalloc") ? (*p = nullptr, kOutOfMemory) : allocate(p, n, kHost);
-}
+int hipHostMalloc(void** p, size_t n, unsigned) { return allocate("hipHostMalloc", p, n, kHost); }
 int hipHostFree(void* p) { return release(p); }
 int hipMemcpy(void* d, const void* s, size_t n, int) {
   memcpy(d, s, n);
