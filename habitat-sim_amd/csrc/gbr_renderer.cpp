@@ -645,7 +645,7 @@ gbr_status rebuild_structure(gbr_renderer* r) {
   TRY(r->d_sub_prims.reserve(r->sub_cap));
   constexpr uint64_t kLongList = 64ull << 20;  // entries
   uint64_t entries = bin_capacities(r, ritems, true);
-  if (entries > kLongList && entries > r->d_bin_entries.cap) {
+  if (entries > r->d_bin_entries.cap) {
     size_t free_bytes = 0, total_bytes = 0;
     HIP_TRY(hipMemGetInfo(&free_bytes, &total_bytes));
     if (entries * sizeof(uint32_t) > free_bytes / 4) entries = bin_capacities(r, ritems, false);

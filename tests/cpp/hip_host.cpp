@@ -23,7 +23,7 @@ std::map<uintptr_t, Block> g_blocks;
 std::map<const void*, std::string> g_kernels;
 std::map<std::string, int64_t> g_calls;
 std::map<std::string, int64_t> g_fail;  // calls left until the named one fails (0: the next)
-int64_t g_device_limit = -1, g_device_used = 0, g_free = 64ll << 30;
+int64_t g_device_limit = -1, g_device_used = 0;
 int g_last_error = kSuccess;
 void (*g_hook)(const char* kernel, const uint32_t* grid, void** args) = nullptr;
 
@@ -82,10 +82,7 @@ extern "C" {
 void hip_host_hook(void (*hook)(const char*, const uint32_t*, void**)) { g_hook = hook; }
 void hip_host_fail(const char* call, int64_t after) { g_fail[call] = after; }
 int64_t hip_host_calls(const char* call) { return g_calls[call]; }
-void hip_host_memory(int64_t device_limit, int64_t free_bytes) {
-  g_device_limit = device_limit;
-  g_free = free_bytes;
-}
+void hip_host_memory(int64_t device_limit) { g_device_limit = device_limit; }
 int64_t hip_host_used() { return g_device_used; }
 int64_t hip_host_blocks() { return (int64_t)g_blocks.size(); }
 
@@ -154,7 +151,8 @@ int hipGetLastError() {
 }
 const char* hipGetErrorString(int e) { return e == kOutOfMemory ? "out of memory" : e ? "error" : "no error"; }
 int hipMemGetInfo(size_t* free_bytes, size_t* total) {
-  *free_bytes = *total = (size_t)g_free;
+  *total = (size_t)(g_device_limit < 0 ? 64ll << 30 : g_device_limit);
+  *free_bytes = *total - (size_t)g_device_used;
   return kSuccess;
 }
 static char g_handle;

@@ -64,9 +64,9 @@ def calls(call: str) -> int:
     return _lib.hip_host_calls(call.encode())
 
 
-def device_memory(limit: int, free: int) -> None:
-    """hipMalloc fails beyond `limit` bytes in all; hipMemGetInfo reports `free`."""
-    _lib.hip_host_memory(ctypes.c_int64(limit), ctypes.c_int64(free))
+def device_memory(limit: int) -> None:
+    """hipMalloc fails beyond `limit` bytes in all."""
+    _lib.hip_host_memory(ctypes.c_int64(limit))
 
 
 def device_memory_used() -> int:

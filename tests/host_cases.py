@@ -154,6 +154,33 @@ def closed_objects_free_their_memory():
     assert hip_host.memory_blocks() == 0
 
 
+def wide_bins_give_way_to_memory():
+    """Where the wide entry list does not fit a quarter of the free memory, bins
+    get the factor's share: a scene that fits with that is drawn."""
+    bins = []
+    _bins(bins.append)
+
+    def draw():
+        r = RendererStandalone(RendererConfiguration().set_tile_size_count((128, 128), (4, 2)))
+        assert r.add_file_data(_soup(40000))
+        for s in range(8):
+            r.add_node_hierarchy(s, "m0", None, 1)
+        r.draw()
+        used = hip_host.device_memory_used()
+        (cap,) = {b.bin_cap for b in bins[-1]}
+        assert all(b.entries == i * cap for i, b in enumerate(bins[-1]))
+        r.draw()
+        r.close()
+        return cap, used
+
+    wide, used = draw()
+    assert wide == 10048
+    # 128 bins of 10048 or 5056 entries of 4 bytes, with half as much room again
+    hip_host.device_memory(used - (2 << 20))
+    cap, less = draw()
+    assert cap == 5056 and less == used - 6 * 128 * (10048 - 5056), (cap, used - less)
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]]()
     print("case passed:", sys.argv[1])
