@@ -76,3 +76,8 @@ def device_memory_used() -> int:
 def memory_blocks() -> int:
     """Device and pinned allocations not yet freed."""
     return _lib.hip_host_blocks()
+
+
+def runtime():
+    """The runtime itself, for calls a user's program makes."""
+    return _lib

@@ -181,6 +181,33 @@ def wide_bins_give_way_to_memory():
     assert cap == 5056 and less == used - 6 * 128 * (10048 - 5056), (cap, used - less)
 
 
+def _pinned(shape):
+    p = ctypes.c_void_p()
+    hip_host.runtime().hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(int(np.prod(shape))), ctypes.c_uint(0))
+    return np.frombuffer((ctypes.c_uint8 * int(np.prod(shape))).from_address(p.value), np.uint8).reshape(shape)
+
+
+def readback_by_destination():
+    """An image read into memory that HIP knows (pinned, managed) is one 2D copy
+    by the device, without a second copy by the host, unless it is small;
+    pageable memory gets its rows from the renderer's pinned staging."""
+    r = _scenes((512, 512), (2, 1), 1)
+    r.draw()
+    page, pin = np.zeros((512, 1024, 4), np.uint8), _pinned((512, 1024, 4))
+    rgb, pin_rgb = np.zeros((512, 1024, 3), np.uint8), _pinned((512, 1024, 3))
+    for image, w, h, copies in ((page, 1024, 512, 0), (rgb, 1024, 512, 0), (pin, 1024, 512, 1), (pin, 700, 511, 1),
+                                (pin_rgb, 1024, 512, 1), (pin, 128, 128, 0), (pin_rgb, 64, 64, 0), (pin_rgb, 128, 128, 1)):
+        before = hip_host.calls("hipMemcpy2DAsync")
+        r.color_image_into((0, 0, w, h), image[:h, :w])
+        assert hip_host.calls("hipMemcpy2DAsync") - before == copies, (image.shape, w, h)
+    # (kernels do not run: the copied rows are those of fresh, zeroed device memory)
+    pin[:] = 7
+    r.color_image_into((0, 0, 700, 511), pin[:511, 300:1000])
+    assert not pin[:511, 300:1000].any() and (pin[:511, :300] == 7).all() and (pin[511:] == 7).all()
+    assert (pin[:, 1000:] == 7).all()
+    r.close()
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]]()
     print("case passed:", sys.argv[1])

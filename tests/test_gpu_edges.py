@@ -4,6 +4,7 @@ a fraction of a pixel to beyond the guard band, workgroups' and waves' worth of
 them and one more, tiles that end inside a bin and inside an 8x8 block, more
 textures than fit in LDS, every filter and wrap mode at sizes that are no power
 of two, any subset of the planes."""
+import ctypes
 import os
 
 import numpy as np
@@ -12,6 +13,7 @@ import pytest
 import synth
 from habitat_sim_amd import RendererConfiguration, RendererStandalone
 from habitat_sim_amd import _native as N
+from habitat_sim_amd import hip
 from habitat_sim_amd import math3d as m3
 from habitat_sim_amd.assets import (GL_CLAMP_TO_EDGE, GL_LINEAR, GL_LINEAR_MIPMAP_LINEAR,
                                     GL_LINEAR_MIPMAP_NEAREST, GL_MIRRORED_REPEAT, GL_NEAREST,
@@ -368,3 +370,42 @@ def test_wrap_modes_that_are_none(wrap, size):
     _draw(r, o)
     _same(r, o)
     r.close()
+
+
+def test_readback_into_pinned_memory():
+    """Images on both sides of the line above which the device copies into
+    pinned memory itself, whole and in padded rows, four bytes and packed RGB8."""
+    tile = (401, 263)
+    runtime, pin = hip.hip(), ctypes.c_void_p()
+    assert runtime.hipHostMalloc(ctypes.byref(pin), ctypes.c_size_t(1 << 20), ctypes.c_uint(0)) == 0
+    pinned = np.frombuffer((ctypes.c_uint8 * (1 << 20)).from_address(pin.value), np.uint8)
+
+    def nines(dtype, *shape):
+        image = pinned[:int(np.prod(shape)) * np.dtype(dtype).itemsize].view(dtype).reshape(shape)
+        image[...] = 9
+        return image
+
+    r, o = _pair(tile, (2, 1))
+    mesh = (_soup(np.random.default_rng(4), 60, 4.0), np.arange(180, dtype=np.uint32), None, None, 0)
+    for x in (r, o):
+        assert x.add_file_data(synth.mesh_file([mesh], [synth.flat((0.2, 0.7, 0.4, 1))]))
+        for s in range(2):
+            x.add_node_hierarchy(s, "m0", m3.rotation_y(0.3 * s), s + 1)
+            _camera(x, s, tile)
+    _draw(r, o)
+    color, lin = o.color_image(), o.linear_depth_image()
+    for x0, y0, x1, y1 in ((0, 0, 802, 263), (1, 3, 2, 4), (10, 0, 138, 256), (10, 0, 139, 256), (300, 7, 428, 92),
+                           (300, 7, 428, 93), (3, 1, 802, 40)):
+        w, h = x1 - x0, y1 - y0
+        for pad in (0, 5):
+            for c in (4, 3):
+                image = nines(np.uint8, h, w + pad, c)
+                r.color_image_into((x0, y0, x1, y1), image[:, :w])
+                np.testing.assert_array_equal(image[:, :w], color[y0:y1, x0:x1, :c])
+                assert (image[:, w:] == 9).all()
+            depth = nines(np.float32, h, w + pad)
+            r.linear_depth_image_into((x0, y0, x1, y1), depth[:, :w])
+            np.testing.assert_array_equal(depth[:, :w], lin[y0:y1, x0:x1])
+            assert (depth[:, w:] == 9).all()
+    r.close()
+    assert runtime.hipHostFree(pin) == 0
