@@ -747,8 +747,9 @@ gbr_status upload_inputs(gbr_renderer* r) {
 
   if (r->input_cap < need) {
     // all blocks at once, with room for moved nodes, so that frames after
-    // the first do not allocate
-    const size_t room = std::max<size_t>({nm, std::min<size_t>(r->n_nodes, 4096), r->n_nodes / 16});
+    // the first rarely allocate: half as many again as now, up to all nodes
+    const size_t all = r->n_nodes;
+    const size_t room = std::max({std::min(nm + nm / 2, all), std::min<size_t>(all, 4096), all / 16});
     const size_t cap = padded(fixed + room * (sizeof(Mat4) + sizeof(uint32_t)));
     for (auto& b : r->inputs) {
       if (b.pending) HIP_TRY(hipEventSynchronize(b.read));

@@ -208,6 +208,31 @@ def readback_by_destination():
     r.close()
 
 
+def more_moved_nodes_every_frame():
+    """A program that moves a few more nodes each frame makes the pinned blocks
+    grow now and then, not every frame; every moved node is sent."""
+    moved = []
+    hip_host.on_launch("k_inputs", hip_host.InputArgs, lambda a, grid, args: moved.append(
+        [(a.nodes[i], a.transforms[16 * i + 12]) for i in range(a.n_nodes)]))
+    r = _scenes((32, 32), (3, 1), 3000)  # 6000 nodes each
+    r.draw()
+    blocks = []
+    for frame, n in enumerate(list(range(4000, 4400)) + list(range(17700, 18000, 50)) + [18000]):
+        left = n
+        for s in range(3):
+            m = min(left, 6000)
+            r.transformations(s)._a[:m, 3, 0] = frame + 1.0
+            left -= m
+        before = hip_host.calls("hipHostMalloc")
+        r.draw()
+        if hip_host.calls("hipHostMalloc") != before:
+            blocks.append(n)
+        sent = moved.pop()
+        assert sent == [(k, frame + 1.0) for k in range(n)], (frame, n)
+    assert len(blocks) <= 5, blocks
+    r.close()
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]]()
     print("case passed:", sys.argv[1])
