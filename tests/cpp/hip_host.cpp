@@ -178,14 +178,23 @@ int hipGraphLaunch(void*, void*) { return kSuccess; }
 int hipGraphDestroy(void*) { return kSuccess; }
 int hipGraphExecDestroy(void*) { return kSuccess; }
 int hipEventCreate(void** e) {
-  *e = &g_handle;
+  *e = new char;
   return kSuccess;
 }
 int hipEventCreateWithFlags(void** e, unsigned) { return hipEventCreate(e); }
-int hipEventDestroy(void*) { return kSuccess; }
-int hipEventRecord(void*, void*) { return kSuccess; }
-int hipEventSynchronize(void*) {
-  ++g_calls["hipEventSynchronize"];
+int hipEventDestroy(void* e) {
+  delete static_cast<char*>(e);
+  return kSuccess;
+}
+// (the hook sees events too: the call's name, and the event as its argument)
+int hipEventRecord(void* e, void*) {
+  const uint32_t none[3] = {};
+  if (g_hook) g_hook("hipEventRecord", none, &e);
+  return kSuccess;
+}
+int hipEventSynchronize(void* e) {
+  const uint32_t none[3] = {};
+  if (g_hook) g_hook("hipEventSynchronize", none, &e);
   return kSuccess;
 }
 int hipEventElapsedTime(float* ms, void*, void*) {

@@ -42,17 +42,19 @@ class RedwoodArgs(ctypes.Structure):
                 ("xmax", ctypes.c_float), ("ymax", ctypes.c_float)]
 
 
+def on_call(function) -> None:
+    """Calls function(name, grid, arguments) at each launch (the kernel's
+    mangled name), event record and event wait (the call's name, the event)."""
+    global _hook
+    _hook = _HOOK(lambda name, grid, args: function(name.decode(), tuple(grid[:3]), args))
+    _lib.hip_host_hook(_hook)
+
+
 def on_launch(kernel: str, argument, function) -> None:
     """Calls function(arguments[0] as an `argument` structure, grid, arguments)
     at each launch of a kernel whose (mangled) name holds `kernel`."""
-    global _hook
-
-    def hook(name, grid, args):
-        if kernel in name.decode():
-            function(argument.from_address(args[0]) if argument else None, tuple(grid[:3]), args)
-
-    _hook = _HOOK(hook)
-    _lib.hip_host_hook(_hook)
+    on_call(lambda name, grid, args: kernel in name and function(
+        argument.from_address(args[0]) if argument else None, grid, args))
 
 
 def fail(call: str, after: int = 0) -> None:

@@ -233,6 +233,37 @@ def more_moved_nodes_every_frame():
     r.close()
 
 
+def input_blocks_are_waited_for():
+    """Draws alternate between three pinned input blocks, and one is written
+    again only after the event behind the kernel that last read it."""
+    pending = {}  # block -> its event, recorded and not yet waited for
+    used = []     # the block of each launch
+    early = []    # launches whose block was still in use
+
+    def call(name, grid, args):
+        if "k_inputs" in name:
+            src = hip_host.InputArgs.from_address(args[0]).src
+            if src in pending:  # (an exception would end here, in the runtime's call)
+                early.append(len(used))
+            used.append(src)
+            pending[src] = None
+        elif name == "hipEventRecord" and used and pending.get(used[-1], 0) is None:
+            pending[used[-1]] = args[0]
+        elif name == "hipEventSynchronize":
+            for src in [s for s, e in pending.items() if e == args[0]]:
+                del pending[src]
+
+    r = _scenes((32, 32), (2, 1), 40)
+    hip_host.on_call(call)
+    for frame in range(10):
+        r.transformations(frame % 2)._a[frame, 3, 0] = frame + 1.0
+        r.draw()
+    assert not early, f"frames {early} wrote blocks that were not waited for"
+    assert len(used) == 10 and len(set(used)) == 3 and all(a == b for a, b in zip(used, used[3:]))
+    assert len(pending) == 3 and None not in pending.values()
+    r.close()
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]]()
     print("case passed:", sys.argv[1])

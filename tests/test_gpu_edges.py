@@ -13,7 +13,7 @@ import pytest
 import synth
 from habitat_sim_amd import RendererConfiguration, RendererStandalone
 from habitat_sim_amd import _native as N
-from habitat_sim_amd import hip
+from habitat_sim_amd import hip, scenes
 from habitat_sim_amd import math3d as m3
 from habitat_sim_amd.assets import (GL_CLAMP_TO_EDGE, GL_LINEAR, GL_LINEAR_MIPMAP_LINEAR,
                                     GL_LINEAR_MIPMAP_NEAREST, GL_MIRRORED_REPEAT, GL_NEAREST,
@@ -409,3 +409,56 @@ def test_readback_into_pinned_memory():
             assert (depth[:, w:] == 9).all()
     r.close()
     assert runtime.hipHostFree(pin) == 0
+
+
+def test_frames_submitted_ahead_of_the_gpu():
+    """Ten frames with their own cameras and moved nodes, submitted without a
+    wait between them (a frame takes longer on the GPU than its submission on
+    the host), their planes copied in stream order: each is the frame that the
+    same inputs give when every draw is waited for."""
+    spec = scenes.apartments(256, tile=64)
+    cfg = RendererConfiguration().set_tile_size_count(spec.tile, spec.grid)
+    rng = np.random.default_rng(8)
+    names = ("color", "linear_depth", "semantic")
+    r = RendererStandalone(cfg, planes=sum(BITS[n] for n in names))
+    scenes.populate(r, spec)
+    n = len(spec.envs)
+    proj = np.stack([e.projection for e in spec.envs]).astype(np.float32)
+    views = np.stack([[m3.inverted_rigid(scenes.random_pose_in_box(rng, (2.0, 2.0), (10.0, 10.0))) for _ in range(n)]
+                      for _ in range(10)]).astype(np.float32)
+    tops = len(r.transformations(0)) // 2
+    moves = [[(int(rng.integers(n)), 2 * int(rng.integers(1, tops)), m3.translation(tuple(rng.uniform(-1, 1, 3))))
+              for _ in range(40)] for _ in range(10)]
+    start = [np.array(r.transformations(s)._a) for s in range(n)]
+    runtime, size = hip.hip(), 4 * n * spec.tile[0] * spec.tile[1]
+
+    def frames(wait):
+        for s in range(n):
+            r.transformations(s)._a[:] = start[s]
+        r.draw()
+        r.synchronize()
+        kept = [[hip.DeviceBuffer(size) for _ in names] for _ in range(10)]
+        for k in range(10):
+            r.update_cameras(0, proj, views[k])
+            for s, node, t in moves[k]:
+                r.transformations(s)[node] = t
+            r.draw()
+            for name, buf in zip(names, kept[k]):
+                assert runtime.hipMemcpyAsync(buf.ptr, ctypes.c_void_p(r.plane_device_pointer(BITS[name])),
+                                              ctypes.c_size_t(size), hip.D2D, ctypes.c_void_p(r.stream())) == 0
+            if wait:
+                r.synchronize()
+        r.synchronize()
+        out = np.zeros((10, len(names), size // 4), np.uint32)
+        for k in range(10):
+            for i in range(len(names)):
+                kept[k][i].to_host(out[k, i])
+                kept[k][i].close()
+        return out
+
+    ref = frames(True)
+    got = frames(False)
+    for k in range(10):
+        np.testing.assert_array_equal(got[k], ref[k], err_msg=f"frame {k}")
+        assert k == 0 or (ref[k] != ref[k - 1]).any()
+    r.close()

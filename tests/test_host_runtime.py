@@ -11,7 +11,7 @@ import pytest
 HERE = os.path.dirname(os.path.abspath(__file__))
 CASES = ["moved_nodes_of_a_failed_frame", "redwood_stays_inside_wide_images", "bin_capacity_follows_the_factor",
          "closed_objects_free_their_memory", "wide_bins_give_way_to_memory", "readback_by_destination",
-         "more_moved_nodes_every_frame"]
+         "more_moved_nodes_every_frame", "input_blocks_are_waited_for"]
 
 
 @pytest.fixture(scope="module", autouse=True)
