@@ -53,12 +53,6 @@
 
 namespace gbr {
 
-#define GL_NEAREST 9728
-#define GL_LINEAR 9729
-#define GL_NEAREST_MIPMAP_NEAREST 9984
-#define GL_LINEAR_MIPMAP_NEAREST 9985
-#define GL_NEAREST_MIPMAP_LINEAR 9986
-#define GL_LINEAR_MIPMAP_LINEAR 9987
 #define GL_CLAMP_TO_EDGE 33071
 #define GL_MIRRORED_REPEAT 33648
 
@@ -299,7 +293,10 @@ __device__ __forceinline__ unsigned long long block_sum(unsigned long long v,
 // fields loaded before their loops stay in scalar registers, which overflow
 // into vector lanes (a v_readlane for each use: 245 of the 2155 vector
 // instructions of k_setup_bin).  Through a pointer the compiler cannot see
-// through, each loop iteration loads what it uses by scalar loads.
+// through, each loop iteration loads what it uses by scalar loads.  (What an
+// item itself needs still overflows, above all its two matrices: 29 registers
+// in k_setup_bin<false> and 30 in <true>, 11 and 6 in the rasteriser storing
+// its keys and resolving.)
 __device__ __forceinline__ const FrameParams& params_again() {
   typedef const __attribute__((address_space(4))) FrameParams* Segment;
   Segment k = (Segment)__builtin_amdgcn_kernarg_segment_ptr();
@@ -1350,7 +1347,11 @@ __device__ __forceinline__ float floor_clamped(float u) {
 // descriptors of the first kLdsTextures textures.  The resolve is bound by
 // the L1's accesses beside its VALU work (610 accesses per 64 pixels on the
 // 512-env frame), and a descriptor costs every pixel two dependent loads,
-// of the header and of the level.
+// of the header and of the level.  Eight (288 bytes each, the first is the
+// white pixel's) leave room for the scenes in use, whose textures are layers of
+// one or a few arrays; the LDS would hold more at the same occupancy, but a
+// texture beyond them costs little (256 scenes of 128x128, each of 64 trilinear
+// quads: 206 us a frame with 7 textures, 210 with 8, 212 to 214 with 16 to 64).
 constexpr uint32_t kLdsTextures = 8;
 
 struct ResolveLds {
@@ -2261,7 +2262,7 @@ __device__ __forceinline__ void bin_hiz(const FrameParams& p, const BinInfo& b, 
 // the longest bins start first and the frame's tail is short.  Per bin, one
 // binned triangle per lane walking its clipped rectangle; rectangles above
 // the lane limit (gbr_tuning.lane_pixels) go to an LDS queue whose
-// triangles the waves take one at a time, each spread over a wave's lanes.
+// triangles the waves share, each in 8x8 blocks of a wave's lanes.
 // Phase 1 starts every bin from the clear key; phase 2 merges into the
 // phase-1 keys and leaves bins without new entries untouched (or, when it
 // resolves in place, resolves them from their phase-1 keys).
@@ -2340,9 +2341,9 @@ __device__ __forceinline__ void raster_bin(const FrameParams& p, const RasterIte
   if (tid == 0) L.nbig[0] = L.nbig[1] = 0;
   __syncthreads();
   // per batch of kBlock entries: lanes append large rectangles to the queue
-  // (fill and claim counters of this batch's parity; the other ones, read
-  // before the previous batch's second barrier, are cleared for the next
-  // batch), then the waves take the queued triangles one at a time
+  // (fill counter of this batch's parity; the other one, read before the
+  // previous batch's second barrier, is cleared for the next batch), then each
+  // wave takes every fourth queued triangle
   int parity = 0;
   for (uint32_t base = 0; base < n; base += kBlock, parity ^= 1) {
     const uint32_t k = base + tid;
@@ -2375,10 +2376,10 @@ __device__ __forceinline__ void raster_bin(const FrameParams& p, const RasterIte
 
 // kWaves: the waves per SIMD the register allocation must allow.  A bin is a
 // chain of dependent loads and barriers, so resident workgroups are what the
-// kernel needs most: without the resolve 8 (64 VGPRs, 20 KB of LDS), measured
-// on the learned 512-env frame 148 / 139 / 133 us at 6 / 7 / 8; with the
-// resolve 5 (96 VGPRs, 4 spilled; 183 -> 173 us after the depth pyramid
-// against 4 without spills).
+// kernel needs most: without the resolve 8 (62 VGPRs and 2 spilled, 18.5 KB of
+// LDS), measured on the learned 512-env frame 148 / 139 / 133 us at 6 / 7 / 8;
+// with the resolve 5 (94 VGPRs, none spilled; 173 us after the depth pyramid
+// against 183 at 4).
 template <bool kResolve, int kWaves>
 __global__ __launch_bounds__(kBlock, kWaves) void k_raster_lane(FrameParams params,
                                                         const RasterItem* __restrict__ items,

@@ -129,11 +129,11 @@ struct RedwoodArgs {
 // (the copy of their bytes takes 13).  Every quotient is the cheapest form that
 // rounds the same:
 //  * pixel -> image, row, column: multiplications (`Divider`);
-//  * x / xmax: (float)((double)x * rx).  The product errs by less than 2^-52,
+//  * x / (W - 1): (float)((double)x * rx).  The product errs by less than 2^-52,
 //    and a quotient of two 24-bit numbers lies at least 2^-49 from the middle
 //    between two floats;
 //  * z / f and 281.04 / q: div_exact();
-//  * 35.13 / u in double: two Newton steps from the single reciprocal (2^-45)
+//  * 35.13 / u in double: one Newton step from the single reciprocal (2^-45)
 //    and a correction by the exact remainder (2^-90); the quotient of two
 //    24-bit numbers lies at least 2^-78 from the middle between two doubles;
 //  * the last quotient in single precision: for two floats a double quotient
