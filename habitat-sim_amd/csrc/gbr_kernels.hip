@@ -965,7 +965,8 @@ __global__ __launch_bounds__(kBlock, 5) void k_setup_bin(FrameParams params,
       }
     }
     __syncthreads();
-    const uint32_t np = min(s_npairs, (uint32_t)kPairCap);
+    // (a scene without LDS counters staged nothing: its s_npairs only says full)
+    const uint32_t np = nlb ? min(s_npairs, (uint32_t)kPairCap) : 0u;
     for (uint32_t i = threadIdx.x; i < np; i += kBlock) {
       const uint32_t e = s_pair[i];
       const uint32_t b = e >> 21;

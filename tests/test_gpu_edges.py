@@ -462,3 +462,31 @@ def test_frames_submitted_ahead_of_the_gpu():
         np.testing.assert_array_equal(got[k], ref[k], err_msg=f"frame {k}")
         assert k == 0 or (ref[k] != ref[k - 1]).any()
     r.close()
+
+
+@pytest.mark.parametrize("tile,tuning", [((1100, 1000), {}), ((1100, 1000), dict(cull_mode=N.CULL_HIZ)),
+                                         ((270, 262), dict(bin_size=8)),
+                                         ((270, 262), dict(bin_size=8, cull_mode=N.CULL_HIZ)),
+                                         ((270, 262), dict(bin_size=8, raster_mode=1, cull_mode=N.CULL_HIZ)),
+                                         ((530, 517), dict(bin_size=16, chunk_triangles=64))])
+def test_more_bins_than_the_lds_counts(tile, tuning):
+    """Scenes of more than 1024 bins, whose (bin, triangle) pairs go straight to
+    the bins, beside one with a small viewport, whose pairs are counted in LDS."""
+    rng = np.random.default_rng(29)
+    r, o = _pair(tile, (3, 1), **tuning)
+    meshes = [(_soup(rng, n, size), np.arange(3 * n, dtype=np.uint32), None, rng.uniform(0, 1, (3 * n, 4)), 0)
+              for n, size in ((4000, 1.0), (2500, 3.0))]
+    fd = synth.mesh_file(meshes, [synth.flat((1, 1, 1, 1))])
+    for x in (r, o):
+        assert x.add_file_data(fd)
+        x.set_scene_viewport(1, (70, 50))
+        for s in range(3):
+            x.add_node_hierarchy(s, "m0", None, 1 + s)
+            x.add_node_hierarchy(s, "m1", m3.rotation_y(0.5), 7)
+    for f in range(3):
+        for x in (r, o):
+            for s in range(3):
+                _camera(x, s, tile, m3.rotation_y(0.3 * f + s))
+        _draw(r, o)
+        _same(r, o, tag=f"frame {f}")
+    r.close()
